@@ -80,12 +80,22 @@ __device__ __forceinline__ half8_t u8x8_to_h8(uint2 w) {
 
 // One output: (acc * alpha) * rs + bi, activation, then store or add into the residual `old`
 // (gated by gt) in the reference's order (app/gpu/gemm.js:159-164).
-// Activation chosen at compile time (the launch dispatches on the argument).
+// Activation: compile-time for the launches the model makes, else by the argument.
+constexpr int kActAny = -1;  // chosen by the argument at run time
+
 template <int ACT>
-__device__ __forceinline__ float act_t(float x) {
+__device__ __forceinline__ float act_t(float x, int act) {
+  if (ACT == kActAny) return apply_act(x, act);
   if (ACT == NS2_ACT_SILU) return silu(x);
-  if (ACT == NS2_ACT_GELU_TANH) return gelu_tanh(x);
   return x;
+}
+
+// The GLU epilogue's gate activation: SiLU with the hardware reciprocal (1 ulp) in place of the IEEE
+// division, whose correction steps were a third of the epilogue's vector instructions.
+template <int ACT>
+__device__ __forceinline__ float glu_act(float x, int act) {
+  if (ACT == NS2_ACT_SILU) return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x));
+  return act_t<ACT>(x, act);
 }
 
 // XCD-aware tile order: consecutive block ids go to different XCDs (round-robin dispatch);
@@ -117,69 +127,93 @@ __device__ __forceinline__ void block_tile(const TGemmArgs& p, int& tm, int& tn)
   tn = rem / rows_in_g;
 }
 
-// Old outputs of a residual launch, loaded before the k loop (their latency hides behind it):
-// cold[i][j][r] = C[mb + 32i + 8(r/4) + r%4][nb + 32j + lq].
-template <int TM, int TN>
-__device__ __forceinline__ void load_old(const TGemmArgs& p, float (&cold)[TM][TN][16], int mb, int nb, int lq) {
+// The epilogues below work on a wave's sums acc[i][j][r] = C[mw + 32i + 8(r/4) + 4hi + r%4][nw + 32j + lq]
+// (mw, nw the wave's first row and column, both uniform; lq = lane % 32, hi = lane / 32). Rows are
+// addressed as a uniform pointer plus a 32-bit lane offset. Every value loaded for an epilogue is
+// waited for once, before the first store (pin): the stores then issue back to back. With the
+// wait inside a per-row branch the compiler drained every earlier store before each one, and the
+// stores of a wave ran one memory round trip after another.
+__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
+
+// Old outputs of tile (i, j).
+__device__ __forceinline__ void load_old(const TGemmArgs& p, float (&old)[16], int mw, int nw, int lq, int hi) {
+  const float* base = p.C + p.cOff + (long long)mw * p.ldc + nw;
+  const int rows = p.M - mw;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = nb + 32 * j + lq;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = mb + 32 * i + 8 * (r >> 2) + (r & 3);
-        cold[i][j][r] = (m < p.M && n < p.N) ? p.C[p.cOff + (long long)m * p.ldc + n] : 0.0f;
-      }
+  for (int r = 0; r < 16; ++r) {
+    // rows past M read the last one (their results are dropped)
+    int dm = 8 * (r >> 2) + 4 * hi + (r & 3);
+    dm = dm < rows ? dm : (rows > 0 ? rows - 1 : 0);
+    old[r] = base[(unsigned)(dm * p.ldc + lq)];
   }
 }
 
-// Plain epilogue of one wave (EPI 0): acc[i][j][r] = C[mb + 32i + 8(r/4) + r%4][nb + 32j + lq],
-// mb = the wave's first row + 4hi. Per column: scale, bias, gate and the row-mb pointer; per
-// element one multiply-add of its row offset and the arithmetic, with the row check only in
-// tiles that cross M. RM 0 stores, RM 1 adds, RM 2 adds gate times the result
-// (gemm.js:159-164); old outputs come from cold when PRE_C, else they are loaded here in a batch.
+// Plain epilogue of one wave (EPI 0). Per column: scale, bias and gate; per element the
+// arithmetic of gemm.js:159-164, with the row check only in tiles that cross M. RM 0 stores, RM 1
+// adds (gate times) the result (no gate: times 1, the same sum); old outputs come from cold when
+// PRE_C, else they are loaded here one tile ahead of the tile being stored.
 // LORA: the low-rank term of each tile (lora_tile) is added after the bias.
 template <int TM, int TN, int ACT, int RM, bool PRE_C, bool LORA, int CI, int CJ>
 __device__ __forceinline__ void store_plain(const TGemmArgs& p, const float16_t (&acc)[TM][TN],
-                                            const float (&cold)[CI][CJ][16], int mb, int nb, bool full, int lq) {
+                                            const float (&cold)[CI][CJ][16], int mw, int nw, bool full, int lq, int hi) {
+  if (mw >= p.M) return;
+  float rs[TN], bi[TN], gt[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int n = nb + 32 * j + lq;
-    if (n >= p.N) continue;
-    const float rs = p.scale ? p.scale[n] : 1.0f;  // no per-row scale on fp16 weights
-    const float bi = p.bias ? p.bias[n] : 0.0f;
-    const float gt = RM == 2 ? p.gate[p.gOff + n] : 1.0f;
-    float* cj = p.C + p.cOff + (long long)mb * p.ldc + n;
+    const bool in = nw + 32 * j < p.N;  // N is a multiple of 64: uniform per column tile
+    const int n = in ? nw + 32 * j + lq : 0;
+    rs[j] = p.scale ? p.scale[n] : 1.0f;  // no per-row scale on fp16 weights
+    bi[j] = p.bias ? p.bias[n] : 0.0f;
+    gt[j] = RM && p.gate ? p.gate[p.gOff + n] : 1.0f;
+  }
+  constexpr bool LOAD_OLD = RM && !PRE_C;
+  float old[2][LOAD_OLD ? 16 : 1];
+  if constexpr (LOAD_OLD) load_old(p, old[0], mw, nw < p.N ? nw : 0, lq, hi);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      float16_t d;
-      if constexpr (LORA) {
-        const int hi = (mb & 4) ? 1 : 0;  // mb = the wave's first row + 4 hi (rows are 32-aligned)
-        const int m = mb - 4 * hi + 32 * i + lq;
-        d = lora_tile(p.lt, p.lb, p.lr, m < p.M ? m : p.M - 1, n, hi);
-      }
-      float old[16];
-      if (RM != 0) {
+  for (int j = 0; j < TN; ++j) {
+    pin(rs[j]);
+    pin(bi[j]);
+    if (RM) pin(gt[j]);
+  }
+  float* base = p.C + p.cOff + (long long)mw * p.ldc + nw;
+  const unsigned lane_off = (unsigned)(4 * hi * p.ldc + lq);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int dm = 32 * i + 8 * (r >> 2) + (r & 3);
-          old[r] = PRE_C ? cold[PRE_C ? i : 0][PRE_C ? j : 0][r]
-                         : ((full || mb + dm < p.M) ? cj[(long long)dm * p.ldc] : 0.0f);
-        }
+  for (int t = 0; t < TM * TN; ++t) {
+    const int j = t / TM, i = t % TM;
+    if constexpr (LOAD_OLD) {
+      if (t + 1 < TM * TN) {
+        const int j1 = (t + 1) / TM, i1 = (t + 1) % TM;
+        const int mi = mw + 32 * i1 < p.M ? mw + 32 * i1 : mw, nj = nw + 32 * j1 < p.N ? nw + 32 * j1 : 0;
+        load_old(p, old[(t + 1) & 1], mi, nj, lq, hi);
       }
+    }
+    if (nw + 32 * j >= p.N) continue;
+    float16_t d;
+    if constexpr (LORA) {
+      const int m = mw + 32 * i + lq;
+      d = lora_tile(p.lt, p.lb, p.lr, m < p.M ? m : p.M - 1, nw + 32 * j + lq, hi);
+    }
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float x = acc[i][j][r] * p.alpha;
+      x *= rs[j];
+      x += bi[j];
+      if constexpr (LORA) x += d[r];
+      x = act_t<ACT>(x, p.act);
+      if (RM) x = (PRE_C ? cold[PRE_C ? i : 0][PRE_C ? j : 0][r] : old[t & 1][LOAD_OLD ? r : 0]) + gt[j] * x;
+      v[r] = x;
+      if (LORA || RM) pin(v[r]);
+    }
+    if (full) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        (base + (long long)(32 * i + 8 * (r >> 2) + (r & 3)) * p.ldc + 32 * j)[lane_off] = v[r];
+    } else {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int dm = 32 * i + 8 * (r >> 2) + (r & 3);
-        if (!full && mb + dm >= p.M) continue;
-        float v = acc[i][j][r] * p.alpha;
-        v *= rs;
-        v += bi;
-        if constexpr (LORA) v += d[r];
-        v = act_t<ACT>(v);
-        if (RM == 1) v = old[r] + v;
-        if (RM == 2) v = old[r] + gt * v;
-        cj[(long long)dm * p.ldc] = v;
+        if (mw + dm + 4 * hi < p.M) (base + (long long)dm * p.ldc + 32 * j)[lane_off] = v[r];
       }
     }
   }
@@ -191,95 +225,149 @@ __device__ __forceinline__ void store_plain(const TGemmArgs& p, const float16_t 
 // which the layout stores as one 16-byte chunk each (chunk 2g + hi of the group's 32 keys in
 // a 64-key tile holds keys 16g + 4hi + {0..3} then 16g + 8 + 4hi + {0..3}).
 template <int TM, int TN, int ACT, bool LORA>
-__device__ __forceinline__ void store_vpack(const TGemmArgs& p, const float16_t (&acc)[TM][TN], int mb, int nb, int lq) {
-  const int hi = (mb & 4) ? 1 : 0;  // mb = the wave's first row + 4 hi (rows are 32-aligned)
-  const int m0 = mb - 4 * hi;
+__device__ __forceinline__ void store_vpack(const TGemmArgs& p, const float16_t (&acc)[TM][TN], int mw, int nw, int lq,
+                                            int hi) {
+  float rs[TN], bi[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int n = nb + 32 * j + lq;
-    const float rs = p.scale ? p.scale[n] : 1.0f;
-    const float bi = p.bias ? p.bias[n] : 0.0f;
+    const int n = nw + 32 * j + lq;
+    rs[j] = p.scale ? p.scale[n] : 1.0f;
+    bi[j] = p.bias ? p.bias[n] : 0.0f;
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    pin(rs[j]);
+    pin(bi[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = nw + 32 * j + lq;
     const int c = n - p.vcol0, h = c / p.vD, dd = c % p.vD;
+    half_t* const dst0 = p.vpk + ((long long)h * p.vtiles * 64 * p.vD + (long long)dd * 8);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       float16_t d;
       if constexpr (LORA) {
-        const int m = m0 + 32 * i + lq;
+        const int m = mw + 32 * i + lq;
         d = lora_tile(p.lt, p.lb, p.lr, m < p.M ? m : p.M - 1, n, hi);
       }
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        const int key16 = m0 + 32 * i + 16 * g;
-        if (key16 >= p.M) continue;
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           float x = acc[i][j][8 * g + e] * p.alpha;
-          x *= rs;
-          x += bi;
+          x *= rs[j];
+          x += bi[j];
           if constexpr (LORA) x += d[8 * g + e];
-          v[e] = act_t<ACT>(x);
+          v[e] = act_t<ACT>(x, p.act);
           // the fp32 value first, as the plain store writes it: the conversion must not fuse
           // with the multiply-add into one rounding to fp16 (v_fma_mix)
-          asm volatile("" : "+v"(v[e]));
+          pin(v[e]);
         }
+        const int key16 = mw + 32 * i + 16 * g;
+        if (key16 >= p.M) continue;
         const int kt = key16 >> 6, kc = 2 * ((key16 & 63) >> 4) + hi;
-        half_t* dst = p.vpk + ((long long)h * p.vtiles + kt) * 64 * p.vD + ((long long)kc * p.vD + dd) * 8;
         uint4 q;
         q.x = pack_half2(v[0], v[1]);
         q.y = pack_half2(v[2], v[3]);
         q.z = pack_half2(v[4], v[5]);
         q.w = pack_half2(v[6], v[7]);
-        *reinterpret_cast<uint4*>(dst) = q;
+        *reinterpret_cast<uint4*>(dst0 + (kt * 8 + kc) * p.vD * 8) = q;
       }
     }
   }
 }
 
-// Block tile BM x BN (multiples of 64), BK = 64; WAVES_M x WAVES_N waves, each computing
-// (BM/WAVES_M) x (BN/WAVES_N) with v_mfma_f32_32x32x16_f16 tiles. STAGES LDS stages, one
-// barrier per k-tile: tile kt+STAGES-1 is copied in while tile kt is multiplied (with three
-// stages the wait before the barrier leaves tile kt+1's copies in flight).
-// EPI 0: C = act(A W^T * alpha * scale + bias) (RM 0), C += that (RM 1) or C += gate * that
-// (RM 2), the order of gemm.js:159-164. EPI 1 (GLU): W's rows are interleaved in 32-row blocks
-// (ns2_tile_i8_weight_glu), so the 64 columns of a wave hold 32 columns of each GLU half; the
+// What a wave does with its sums (plain epilogues): the raw partial products of a split, the
+// packed values of the attention, or store_plain.
+template <int TM, int TN, int ACT, int RM, bool PRE_C, bool LORA, int CI, int CJ>
+__device__ __forceinline__ void finish(const TGemmArgs& p, const float16_t (&acc)[TM][TN], const float (&cold)[CI][CJ][16],
+                                       int mw, int nw, bool full, int lq, int hi) {
+  if (p.part) {
+    // split-K: the raw partial products of split blockIdx.y
+    float* base = p.part + ((long long)blockIdx.y * p.M + mw) * p.N + nw;
+    const unsigned lane_off = (unsigned)(4 * hi * p.N + lq);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if (nw + 32 * j >= p.N) continue;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int dm = 32 * i + 8 * (r >> 2) + (r & 3);
+          if (full || mw + dm + 4 * hi < p.M) (base + (long long)dm * p.N + 32 * j)[lane_off] = acc[i][j][r];
+        }
+    }
+    return;
+  }
+  // a wave whose columns straddle vcol0 goes column tile by column tile
+  if (RM == 0 && p.vpk && nw + 32 * TN > p.vcol0) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      float16_t col[TM][1];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) col[i][0] = acc[i][j];
+      const int n = nw + 32 * j;
+      if (n >= p.N) continue;
+      if (n >= p.vcol0) store_vpack<TM, 1, ACT, LORA>(p, col, mw, n, lq, hi);
+      else store_plain<TM, 1, ACT, RM, false, LORA>(p, col, cold, mw, n, full, lq, hi);
+    }
+    return;
+  }
+  store_plain<TM, TN, ACT, RM, PRE_C, LORA>(p, acc, cold, mw, nw, full, lq, hi);
+}
+
+// Block tile BM x BN (multiples of 64), k-tiles of 64 KT. WAVES_M x WAVES_N waves per k group, each
+// computing (BM/WAVES_M) x (BN/WAVES_N) with v_mfma_f32_32x32x16_f16 tiles; KG k groups of waves
+// share a block's tile and take alternate k16 steps (their sums are added through LDS at the end),
+// which puts two waves on every SIMD where the grid leaves one tile per CU. STAGES LDS stages.
+//
+// What bounds it: the matrix cores, at the clock the chip's power allows (1.5-1.75 GHz with all CUs
+// multiplying). The k loop of the 192x384 tile keeps them 78 % busy (2940 clocks per k-tile of 2304),
+// that of the 64x128 tile 68 %; the rest of a launch is its prologue (2 us) and its stores. Three
+// things hold the loop there:
+//  * fragments are read one k16 step ahead, across the k-tile's barrier too: the barrier comes
+//    before the last step of a tile (whose fragments are in registers by then), so no wave waits
+//    for LDS behind it;
+//  * the weight fragment of the next column is decoded behind the current column's products;
+//  * the copies of a k-tile go out in SPREAD steps between products, since a wave that issues them
+//    all at once issues no products meanwhile (64 bytes per clock and CU).
+// Three stages or a raised wave priority around the products measured no faster.
+// EPI 0: C = act(A W^T * alpha * scale + bias) (RM 0) or C += (gate *) that (RM 1), the order of
+// gemm.js:159-164. EPI 1 (GLU): W's rows are interleaved in 32-row blocks
+// (ns2_tile_i8_weight_glu), so 64 columns of a wave hold 32 columns of each GLU half; the
 // block's 512 columns give 256 consecutive outputs act(h1) * h2, one rotation group, which is
 // rotated and written to Y as the tiled fp16 operand of the next int8 linear.
 // WF16: fp16 weight tiles (the plain bf16 linears, re-tiled as fp16; no per-row scale unless
 // given): 8 KB per 64x64 weight tile, read straight into the MFMA B operand.
-// Waves per SIMD that a launch with the LoRA term keeps: the occupancy of the plain kernel of
-// the same shape (left free, the compiler spends a few more registers on the LoRA variants and
-// they lose a resident block: 128 -> 140 for the GLU launch).
-template <int BM, int BN, int RM, bool LORA>
-constexpr int lora_waves_per_eu() {
-  if (!LORA) return 1;
-  if (BM == 64 && BN == 512) return 4;
-  if (BM == 64 && BN == 128) return RM ? 4 : 5;
-  return 1;
-}
-
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, int ACT, int RM, bool LORA, bool WF16 = false>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(lora_waves_per_eu<BM, BN, RM, LORA>())))
+// WPE: waves per SIMD the registers must leave room for.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int KG, int KT, int STAGES, int SPREAD, int EPI, int ACT, int RM, bool LORA, bool WF16, int WPE>
+__global__ __launch_bounds__(WAVES_M * WAVES_N * KG * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void gemm_tiled_kernel(TGemmArgs p) {
-  constexpr int NW = WAVES_M * WAVES_N;
+  constexpr int NW = WAVES_M * WAVES_N * KG;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int TM = WTM / 32, TN = WTN / 32;
+  constexpr int NS = 4 * KT / KG;    // k16 steps of a k-tile (64 KT wide) per wave
   constexpr int WCH = WF16 ? 8 : 4;  // 1 KB blocks per 64 weight rows of a k-tile
   constexpr int WB = WF16 ? 2 : 1;   // bytes per weight element
-  constexpr int A_BLOCKS = BM / 64 * 8, W_BLOCKS = BN / 64 * WCH;  // 1 KB blocks per stage
+  constexpr int A_BLOCKS = BM / 64 * 8 * KT, W_BLOCKS = BN / 64 * WCH * KT;  // 1 KB blocks per stage
   constexpr int BLOCKS = A_BLOCKS + W_BLOCKS;
-  constexpr int PER_WAVE = BLOCKS / NW;
+  constexpr int PER_WAVE = (BLOCKS + NW - 1) / NW;  // copies per wave and k-tile, at most
+  constexpr int FULL_WAVES = BLOCKS % NW ? BLOCKS % NW : NW;  // waves that issue that many; the others one less
+  constexpr int A_BYTES = BM * 64 * KT * 2, W_BYTES = BN * 64 * KT * WB;
   static_assert(BM % 64 == 0 && BN % 64 == 0 && WTM % 32 == 0 && WTN % 32 == 0, "tile shape");
-  static_assert(BLOCKS % NW == 0, "copies must split evenly over the waves");
-
+  static_assert(NS % 2 == 0, "an even number of steps per k-tile");
   static_assert(STAGES == 2 || STAGES == 3, "two or three LDS stages");
   static_assert(!WF16 || EPI == 0, "fp16 weights take the plain epilogue");
-  __shared__ __attribute__((aligned(16))) half_t as[STAGES][BM * 64];
-  __shared__ __attribute__((aligned(16))) uint8_t ws[STAGES][BN * 64 * WB];
+  __shared__ __attribute__((aligned(16))) char smem[STAGES * (A_BYTES + W_BYTES)];
+  char* const as = smem;
+  char* const ws = smem + STAGES * A_BYTES;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int kg = KG > 1 ? wave / (WAVES_M * WAVES_N) : 0, wi = KG > 1 ? wave % (WAVES_M * WAVES_N) : wave;
+  const int wm = wi / WAVES_N, wn = wi % WAVES_N;
   const int lq = lane & 31, hi = lane >> 5;
 
   int tm, tn;
@@ -288,7 +376,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
 
   // k-tiles of this block: all of K, or split z = blockIdx.y's range
   const int kt0 = p.part ? (int)blockIdx.y * p.ksplit : 0;
-  const int kblocks = p.part ? (p.K / 64 - kt0 < p.ksplit ? p.K / 64 - kt0 : p.ksplit) : p.K / 64;
+  const int kblocks = (p.part ? (p.K / 64 - kt0 < p.ksplit ? p.K / 64 - kt0 : p.ksplit) : p.K / 64) / KT;
   const int kall = p.K / 64;
   // Stage image: A blocks (8 k-chunks of 1 KB per 64-row block), then W blocks (WCH per 64-row
   // block). Block ids past the last real 64-row block re-read the last one (their rows are
@@ -302,29 +390,34 @@ void gemm_tiled_kernel(TGemmArgs p) {
     for (int i = 0; i < PER_WAVE; ++i) {
       const int j = wave + i * NW;
       if (j < A_BLOCKS) {
-        const int mbi = j / 8, c = j % 8;
+        const int mbi = j / (8 * KT), c = j % (8 * KT);
         int mb = m0 / 64 + mbi;
         mb = mb < p.mblocks ? mb : p.mblocks - 1;
         g_src[i] = reinterpret_cast<const char*>(p.At) + ((long long)mb * kall * 8 + (long long)kt0 * 8 + c) * 1024;
         l_dst[i] = as_base + j * 1024;
-        g_step[i] = 8 * 1024;
-        l_step[i] = BM * 64 * 2;
+        g_step[i] = 8 * KT * 1024;
+        l_step[i] = A_BYTES;
       } else {
         const int jw = j - A_BLOCKS;
-        const int nbi = jw / WCH, c = jw % WCH;
+        const int nbi = jw / (WCH * KT), c = jw % (WCH * KT);
         int nb = n0 / 64 + nbi;
         nb = nb < p.nblocks ? nb : p.nblocks - 1;
         g_src[i] = reinterpret_cast<const char*>(p.Wt) + ((long long)nb * kall * WCH + (long long)kt0 * WCH + c) * 1024;
         l_dst[i] = ws_base + jw * 1024;
-        g_step[i] = WCH * 1024;
-        l_step[i] = BN * 64 * WB;
+        g_step[i] = WCH * KT * 1024;
+        l_step[i] = W_BYTES;
       }
     }
   }
-  auto dma = [&](int kt, int st) {
-#pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i)
+  auto dma_one = [&](int i, int kt, int st) {
+    if (i + 1 < PER_WAVE || FULL_WAVES == NW || wave < FULL_WAVES)
       dma16(g_src[i] + (long long)kt * g_step[i] + lane * 16, __builtin_amdgcn_readfirstlane(l_dst[i] + st * l_step[i]));
+  };
+  // wait until at most this wave's copies of the n most recent tiles are in flight
+  auto wait_newer = [&](auto n_c) {
+    constexpr int N = decltype(n_c)::value;
+    if (FULL_WAVES == NW || wave < FULL_WAVES) vm_wait<N * PER_WAVE>();
+    else vm_wait<N * (PER_WAVE - 1)>();
   };
 
   float16_t acc[TM][TN];
@@ -337,186 +430,258 @@ void gemm_tiled_kernel(TGemmArgs p) {
 
   // Residual launches of small wave tiles load their old outputs before the k loop, where the
   // latency hides behind it, instead of in the epilogue.
-  constexpr bool PRE_C = EPI == 0 && RM != 0 && TM * TN * 16 <= 32;
+  constexpr bool PRE_C = EPI == 0 && RM != 0 && KG == 1 && TM * TN * 16 <= 32;
   float cold[PRE_C ? TM : 1][PRE_C ? TN : 1][16];
   if constexpr (PRE_C) {
-    if (!p.part) load_old<TM, TN>(p, cold, m0 + wm * WTM + 4 * hi, n0 + wn * WTN, lq);
+    if (!p.part) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int mi = m0 + wm * WTM + 32 * i, nj = n0 + wn * WTN + 32 * j;
+          load_old(p, cold[i][j], mi < p.M ? mi : 0, nj < p.N ? nj : 0, lq, hi);
+        }
+    }
   }
-
-  dma(0, 0);
-  if (STAGES == 3 && kblocks > 1) dma(1, 1);
 
   // fragments of k-step s (16 k) of a stage: A rows wm*WTM + 32i + lq, k 16s + 8hi .. +7 (chunk
   // 2s + hi); W columns wn*WTN + 32j + lq, the same k (8-byte chunk 2s + hi, or 16-byte chunk for
   // fp16 weights, read as the B operand itself)
-  auto read_a = [&](int st, int s, int i) {
-    const int row = wm * WTM + 32 * i;
-    const int mbi = row / 64, r0 = row % 64;
-    return *reinterpret_cast<const half8_t*>(&as[st][((mbi * 8 + 2 * s + hi) * 64 + r0 + lq) * 8]);
-  };
   using WRaw = std::conditional_t<WF16, half8_t, uint2>;
-  auto read_w = [&](int st, int s, int j) {
-    const int col = wn * WTN + 32 * j;
-    const int nbi = col / 64, c0 = col % 64;
-    return *reinterpret_cast<const WRaw*>(&ws[st][((nbi * 8 + 2 * s + hi) * 64 + c0 + lq) * 8 * WB]);
+  auto read_frags = [&](int st, int s, half8_t (&a)[TM], WRaw (&w)[TN]) {
+    const int kc = 2 * (s * KG + kg) + hi;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = wn * WTN + 32 * j;
+      w[j] = *reinterpret_cast<const WRaw*>(ws + st * W_BYTES + ((col / 64 * 8 * KT + kc) * 64 + col % 64 + lq) * 8 * WB);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int row = wm * WTM + 32 * i;
+      a[i] = *reinterpret_cast<const half8_t*>(as + st * A_BYTES + ((row / 64 * 8 * KT + kc) * 64 + row % 64 + lq) * 16);
+    }
   };
   auto decode = [&](const WRaw& w) {
     if constexpr (WF16) return w;
     else return u8x8_to_h8(w);
   };
 
-  for (int kt = 0; kt < kblocks; ++kt) {
-    const int st = kt % STAGES;
-    // this wave's copies of tile kt have landed once at most tile kt+1's remain in flight
-    // (three stages); the barrier then covers every wave's copies, and every wave's reads of
-    // tile kt-1, whose stage the next copies overwrite
-    if (STAGES == 3 && kt + 1 < kblocks) vm_wait<PER_WAVE>();
-    else vm_wait<0>();
-    __syncthreads();
-    if (kt + STAGES - 1 < kblocks) dma(kt + STAGES - 1, (kt + STAGES - 1) % STAGES);
-    __builtin_amdgcn_s_setprio(1);
-    // k-steps of 16, software-pipelined: fragments read two steps ahead, the weights decoded
-    // one step ahead, behind the MFMAs; scheduling barriers pin the order (the default
-    // scheduler would put every read right before its use to save registers)
-    half8_t a[3][TM], b[2][TN];
-    WRaw w[3][TN];
+  // The copies of a k-tile are issued in SPREAD steps, between the products: the first part in the
+  // last step of tile kt, once every wave has read its last fragment of it (tile kt + STAGES takes
+  // its stage), the rest in the first steps of tile kt + 1. copy_part issues those of slot `slot`.
+  constexpr int SLOTS = SPREAD * TN;
+  auto copy_part = [&](int slot, int kt, int st) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int i = 0; i < PER_WAVE; ++i)
+      if (i * SLOTS / PER_WAVE == slot) dma_one(i, kt, st);
+  };
 #pragma unroll
-      for (int i = 0; i < TM; ++i) a[s][i] = read_a(st, s, i);
+  for (int t = 0; t < STAGES; ++t)
+    if (t < kblocks) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) w[s][j] = read_w(st, s, j);
+      for (int i = 0; i < PER_WAVE; ++i)
+        if (t + 1 < STAGES || i * SLOTS / PER_WAVE < TN) dma_one(i, t, t);
     }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b[0][j] = decode(w[0][j]);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (s + 2 < 4) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[(s + 2) % 3][i] = read_a(st, s + 2, i);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) w[(s + 2) % 3][j] = read_w(st, s + 2, j);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s % 3][i], b[s & 1][j], acc[i][j], 0, 0, 0);
-      if (s + 1 < 4) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) b[(s + 1) & 1][j] = decode(w[(s + 1) % 3][j]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_s_setprio(0);
+  // tile 0 has landed; the copies of later tiles may be in flight
+  constexpr int FIRST = [] { int n = 0; for (int i = 0; i < PER_WAVE; ++i) n += i * SLOTS / PER_WAVE < TN; return n; }();
+  if (kblocks >= STAGES) {
+    // the short waves' last copy is never in the first part unless SPREAD is 1
+    if (FULL_WAVES == NW || wave < FULL_WAVES) vm_wait<(STAGES - 2) * PER_WAVE + FIRST>();
+    else vm_wait<(STAGES - 2) * (PER_WAVE - 1) + (FIRST < PER_WAVE ? FIRST : PER_WAVE - 1)>();
+  } else {
+    vm_wait<0>();
   }
+  __syncthreads();
+  half8_t a[2][TM];
+  WRaw w[2][TN];
+  read_frags(0, 0, a[0], w[0]);
+  half8_t b = decode(w[0][0]);
+  int st = 0;
+  auto ktile = [&](int kt, auto last_c) {
+    constexpr bool LAST = decltype(last_c)::value;
+    const int nst = st + 1 == STAGES ? 0 : st + 1;
+    const int pst = st == 0 ? STAGES - 1 : st - 1;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s + 1 < NS) {
+        read_frags(st, s + 1, a[(s + 1) & 1], w[(s + 1) & 1]);
+      } else if (!LAST) {
+        // this wave's copies of tile kt+1 have landed once at most the later tiles' remain in
+        // flight; the barrier then covers every wave's copies, and every wave's reads of tile
+        // kt (waited for here), whose stage the next copies overwrite
+        if (STAGES == 3 && kt + 2 < kblocks) wait_newer(std::integral_constant<int, 1>{});
+        else vm_wait<0>();
+        __syncthreads();
+        read_frags(nst, 0, a[0], w[0]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s & 1][i], b, acc[i][j], 0, 0, 0);
+        if (j + 1 < TN) b = decode(w[s & 1][j + 1]);
+        else if (s + 1 < NS || !LAST) b = decode(w[(s + 1) & 1][0]);
+        if (!LAST) {
+          if (s == NS - 1) {
+            if (kt + STAGES < kblocks) copy_part(j, kt + STAGES, st);
+          } else if (s + 1 < SPREAD) {
+            if (kt + STAGES - 1 < kblocks) copy_part((s + 1) * TN + j, kt + STAGES - 1, pst);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    st = nst;
+  };
+  for (int kt = 0; kt + 1 < kblocks; ++kt) ktile(kt, std::integral_constant<bool, false>{});
+  ktile(kblocks - 1, std::integral_constant<bool, true>{});
 
   if constexpr (EPI == 1) {
-    // ---- GLU + rotation epilogue (BM = 64, BN = 512, one wave row, 64 columns per wave)
-    static_assert(BM == 64 && BN == 512 && WAVES_M == 1 && TM == 2 && TN == 2, "GLU epilogue tile");
+    // ---- GLU + rotation epilogue (BN = 512: 256 outputs, one rotation group; a wave's columns are
+    // pairs of 32 gate and 32 value columns), 64 rows at a time
+    static_assert(KG == 1 && BN == 512 && TN % 2 == 0, "GLU epilogue tile");
+    static_assert(sizeof(smem) >= 64 * 256 * 4, "one 64 x 256 fp32 chunk in the stages");
+    constexpr int JP = TN / 2;
     const int I = p.N / 2;
-    const int gb = n0 / 2;            // first output (GLU) column of the block
-    const int gc = 32 * wn + lq;      // this lane's output column within the block
-    const int G = gb + gc;
-    const float s1 = p.scale[G], s2 = p.scale[I + G];
-    const float b1 = p.bias ? p.bias[G] : 0.0f, b2 = p.bias ? p.bias[I + G] : 0.0f;
-    __syncthreads();  // every wave is done with the LDS stages
-    float* T = reinterpret_cast<float*>(&ws[0][0]);  // [64 rows][256 columns] fp32 = the W stages
+    const int gb = n0 / 2;  // first output (GLU) column of the block
+    float* T = reinterpret_cast<float*>(smem);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      if constexpr (LORA) {
-        // the low-rank terms of the two halves' tiles (weight rows G and I + G), one tile at a
-        // time: act(h1) goes through T, then h2 multiplies it in place
-        int m = m0 + 32 * i + lq;
-        m = m < p.M ? m : p.M - 1;
-        const float16_t d1 = lora_tile(p.lt, p.lb, p.lr, m, G, hi);
+    for (int ch = 0; ch < BM / 64; ++ch) {
+      __syncthreads();  // every wave is done with the LDS stages (or the previous chunk)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = 32 * i + 8 * (r >> 2) + 4 * hi + (r & 3);
-          float h1 = acc[i][0][r] * p.alpha;
-          h1 *= s1;
-          h1 += b1;
-          T[row * 256 + gc] = act_t<ACT>(h1 + d1[r]);
-        }
-        const float16_t d2 = lora_tile(p.lt, p.lb, p.lr, m, I + G, hi);
+      for (int jj = 0; jj < JP; ++jj) {
+        const int gc = 32 * (wn * JP + jj) + lq;  // this lane's output column within the block
+        const int G = gb + gc;
+        const float s1 = p.scale[G], s2 = p.scale[I + G];
+        const float b1 = p.bias ? p.bias[G] : 0.0f, b2 = p.bias ? p.bias[I + G] : 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = 32 * i + 8 * (r >> 2) + 4 * hi + (r & 3);
-          float h2 = acc[i][1][r] * p.alpha;
-          h2 *= s2;
-          h2 += b2;
-          T[row * 256 + gc] *= h2 + d2[r];
-        }
-      } else {
+        for (int i = 0; i < TM; ++i) {
+          if ((wm * WTM + 32 * i) / 64 != ch) continue;
+          const int rb = (wm * WTM + 32 * i) % 64 + 4 * hi;
+          if constexpr (LORA) {
+            // the low-rank terms of the two halves' tiles (weight rows G and I + G), one tile at a
+            // time: act(h1) goes through T, then h2 multiplies it in place
+            int m = m0 + wm * WTM + 32 * i + lq;
+            m = m < p.M ? m : p.M - 1;
+            const float16_t d1 = lora_tile(p.lt, p.lb, p.lr, m, G, hi);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = 32 * i + 8 * (r >> 2) + 4 * hi + (r & 3);
-          // the linear's epilogue order (no activation there), then the GLU
-          float h1 = acc[i][0][r] * p.alpha;
-          h1 *= s1;
-          h1 += b1;
-          float h2 = acc[i][1][r] * p.alpha;
-          h2 *= s2;
-          h2 += b2;
-          T[row * 256 + gc] = act_t<ACT>(h1) * h2;
+            for (int r = 0; r < 16; ++r) {
+              const int row = rb + 8 * (r >> 2) + (r & 3);
+              float h1 = acc[i][2 * jj][r] * p.alpha;
+              h1 *= s1;
+              h1 += b1;
+              T[row * 256 + gc] = glu_act<ACT>(h1 + d1[r], p.act);
+            }
+            const float16_t d2 = lora_tile(p.lt, p.lb, p.lr, m, I + G, hi);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const int row = rb + 8 * (r >> 2) + (r & 3);
+              float h2 = acc[i][2 * jj + 1][r] * p.alpha;
+              h2 *= s2;
+              h2 += b2;
+              T[row * 256 + gc] *= h2 + d2[r];
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const int row = rb + 8 * (r >> 2) + (r & 3);
+              // the linear's epilogue order (no activation there), then the GLU
+              float h1 = acc[i][2 * jj][r] * p.alpha;
+              h1 *= s1;
+              h1 += b1;
+              float h2 = acc[i][2 * jj + 1][r] * p.alpha;
+              h2 *= s2;
+              h2 += b2;
+              T[row * 256 + gc] = glu_act<ACT>(h1, p.act) * h2;
+            }
+          }
         }
       }
-    }
-    __syncthreads();
-    // rotation: wave w rotates rows 8w .. 8w+7 on the matrix cores, the fp16 result in place in
-    // the first 512 bytes of the row, its 16-byte chunk c stored at chunk c ^ (row & 7): the
-    // copy-out below reads one chunk of 64 rows 1 KB apart per wave, and the swizzle puts 8
-    // consecutive rows in 8 different bank groups (unswizzled, all 64 lanes hit the same four
-    // banks)
+      __syncthreads();
+      // rotation: wave w rotates its 64 / NW rows on the matrix cores, the fp16 result in place in
+      // the first 512 bytes of the row, its 16-byte chunk c stored at chunk c ^ (row & 7): the
+      // copy-out below reads one chunk of 64 rows 1 KB apart per wave, and the swizzle puts 8
+      // consecutive rows in 8 different bank groups (unswizzled, all 64 lanes hit the same four
+      // banks)
 #pragma unroll
-    for (int rr = 0; rr < 64 / NW; ++rr) {
-      // the matrix-core FWHT: lane l holds columns lo .. lo+3, lo = 16(l%16) + 4(l/16)
-      const half4v_t hf = fwht_h16_fragment();
-      const int lo = fwht_mfma_offset();
-      const int row = (64 / NW) * wave + rr;
-      const float4 in = *reinterpret_cast<const float4*>(T + row * 256 + lo);
-      float v[4] = {in.x, in.y, in.z, in.w};
-      fwht256_mfma(v, hf);
-      uint2 o;
-      o.x = pack_half2(v[0], v[1]);
-      o.y = pack_half2(v[2], v[3]);
-      char* rb = reinterpret_cast<char*>(T + row * 256);
-      *reinterpret_cast<uint2*>(rb + ((lo >> 3) ^ (row & 7)) * 16 + ((lo >> 2) & 1) * 8) = o;
-    }
-    __syncthreads();
-    // 32 chunks of 8 columns x 64 rows: 1 KB contiguous each in the tiled layout
-    for (int q = tid; q < 32 * 64; q += NW * 64) {
-      const int row = q % 64, c = q / 64;
-      const char* rb = reinterpret_cast<const char*>(T + row * 256);
-      const uint4 v = *reinterpret_cast<const uint4*>(rb + (c ^ (row & 7)) * 16);
-      *reinterpret_cast<uint4*>(p.Y + tiled_off(m0 + row, gb + c * 8, I)) = v;
+      for (int rr = 0; rr < 64 / NW; ++rr) {
+        // the matrix-core FWHT: lane l holds columns lo .. lo+3, lo = 16(l%16) + 4(l/16)
+        const half4v_t hf = fwht_h16_fragment();
+        const int lo = fwht_mfma_offset();
+        const int row = (64 / NW) * wave + rr;
+        const float4 in = *reinterpret_cast<const float4*>(T + row * 256 + lo);
+        float v[4] = {in.x, in.y, in.z, in.w};
+        fwht256_mfma(v, hf);
+        uint2 o;
+        o.x = pack_half2(v[0], v[1]);
+        o.y = pack_half2(v[2], v[3]);
+        char* rb = reinterpret_cast<char*>(T + row * 256);
+        *reinterpret_cast<uint2*>(rb + ((lo >> 3) ^ (row & 7)) * 16 + ((lo >> 2) & 1) * 8) = o;
+      }
+      __syncthreads();
+      // 32 chunks of 8 columns x 64 rows: 1 KB contiguous each in the tiled layout; the row blocks
+      // past the last one of Y (BM > 64) are dropped
+      if (BM > 64 && m0 + 64 * ch >= p.mblocks * 64) break;
+      for (int q = tid; q < 32 * 64; q += NW * 64) {
+        const int row = q % 64, c = q / 64;
+        const char* rb = reinterpret_cast<const char*>(T + row * 256);
+        const uint4 v = *reinterpret_cast<const uint4*>(rb + (c ^ (row & 7)) * 16);
+        *reinterpret_cast<uint4*>(p.Y + tiled_off(m0 + 64 * ch + row, gb + c * 8, I)) = v;
+      }
     }
     return;
   }
-  if (p.part) {
-    // split-K: the raw partial products of split blockIdx.y
-    float* part = p.part + (long long)blockIdx.y * p.M * p.N;
-    const int mb = m0 + wm * WTM + 4 * hi, nb = n0 + wn * WTN;
+  if constexpr (KG == 1) {
+    finish<TM, TN, ACT, RM, PRE_C, LORA>(p, acc, cold, m0 + wm * WTM, n0 + wn * WTN, m0 + BM <= p.M, lq, hi);
+  } else {
+    // the two k groups' sums: group g keeps row tiles [g TM/2, (g+1) TM/2) and hands the others
+    // over through LDS, one column tile at a time (16 values per lane as four float4 planes)
+    static_assert(KG == 2 && TM % 2 == 0, "row tiles split between two k groups");
+    constexpr int H = TM / 2;
+    static_assert(sizeof(smem) >= (size_t)NW * H * 4096, "exchange buffer");
+    constexpr bool PRE = RM && H * TN * 16 <= 48;
+    float kold[PRE ? H : 1][PRE ? TN : 1][16];
+    if constexpr (PRE) {
+      // the kept tiles' old outputs, in flight behind the exchange
+      if (!p.part) {
+#pragma unroll
+        for (int i = 0; i < H; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const int mi = m0 + wm * WTM + (kg * H + i) * 32, nj = n0 + wn * WTN + 32 * j;
+            load_old(p, kold[i][j], mi < p.M ? mi : 0, nj < p.N ? nj : 0, lq, hi);
+          }
+      }
+    }
+    float16_t keep[H][TN];
+    float4* X = reinterpret_cast<float4*>(smem);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int n = nb + 32 * j + lq;
-      if (n >= p.N) continue;
+      __syncthreads();
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < H; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = mb + 32 * i + 8 * (r >> 2) + (r & 3);
-          if (m < p.M) part[(long long)m * p.N + n] = acc[i][j][r];
+        for (int q = 0; q < 4; ++q) {
+          const float16_t& g = kg ? acc[i][j] : acc[H + i][j];
+          X[((wave * H + i) * 4 + q) * 64 + lane] = make_float4(g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]);
+        }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < H; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4 o = X[(((wave ^ (NW / 2)) * H + i) * 4 + q) * 64 + lane];
+          const float16_t& k = kg ? acc[H + i][j] : acc[i][j];
+          keep[i][j][4 * q + 0] = k[4 * q + 0] + o.x;
+          keep[i][j][4 * q + 1] = k[4 * q + 1] + o.y;
+          keep[i][j][4 * q + 2] = k[4 * q + 2] + o.z;
+          keep[i][j][4 * q + 3] = k[4 * q + 3] + o.w;
         }
     }
-    return;
+    finish<H, TN, ACT, RM, PRE, LORA>(p, keep, kold, m0 + wm * WTM + kg * H * 32, n0 + wn * WTN,
+                                        m0 + BM <= p.M, lq, hi);
   }
-  if (RM == 0 && p.vpk && n0 + wn * WTN >= p.vcol0 && n0 + wn * WTN < p.N) {
-    store_vpack<TM, TN, ACT, LORA>(p, acc, m0 + wm * WTM + 4 * hi, n0 + wn * WTN, lq);
-    return;
-  }
-  store_plain<TM, TN, ACT, RM, PRE_C, LORA>(p, acc, cold, m0 + wm * WTM + 4 * hi, n0 + wn * WTN, m0 + BM <= p.M, lq);
 }
 
 // The splits of a split-K launch summed in z order (deterministic), then the plain epilogue of
@@ -630,7 +795,8 @@ __global__ __launch_bounds__(256) void tile_w16_kernel(const uint16_t* __restric
 // Weight bytes per column band of the tile order: half of an XCD's 4 MB L2.
 constexpr long long kBandBytes = 2ll << 20;
 
-template <int BM, int BN, int WM, int WN, int STAGES = 2, int EPI = 0, bool WF16 = false>
+template <int BM, int BN, int WM, int WN, int KG, int KT, int STAGES, int SPREAD, int WPE, int EPI = 0, bool WF16 = false, bool RESID = true,
+          bool LORA = true, bool ANY_ACT = false>
 int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -653,37 +819,31 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
       }
     }
   }
-  const dim3 grid(p.tiles_m * p.tiles_n, splits), block(WM * WN * 64);
+  const dim3 grid(p.tiles_m * p.tiles_n, splits), block(WM * WN * KG * 64);
   hipStream_t s = ns2::stream();
-  const int rm = !p.resid ? 0 : (p.gate ? 2 : 1);
-#define NS2_TILED(A, R)                                                                               \
-  do {                                                                                                \
-    if constexpr (BM * BN < 256 * 256) {                                                              \
-      if (p.lr) {                                                                                     \
-        gemm_tiled_kernel<BM, BN, WM, WN, STAGES, EPI, A, R, true, WF16><<<grid, block, 0, s>>>(p);   \
-        break;                                                                                        \
-      }                                                                                               \
-    }                                                                                                 \
-    gemm_tiled_kernel<BM, BN, WM, WN, STAGES, EPI, A, R, false, WF16><<<grid, block, 0, s>>>(p);      \
-  } while (0)
-  if constexpr (EPI == 1) {
-    if (p.act == NS2_ACT_SILU) NS2_TILED(NS2_ACT_SILU, 0);
-    else if (p.act == NS2_ACT_GELU_TANH) NS2_TILED(NS2_ACT_GELU_TANH, 0);
-    else NS2_TILED(NS2_ACT_NONE, 0);
-  } else {
-    switch (p.act * 3 + rm) {
-      case 0: NS2_TILED(NS2_ACT_NONE, 0); break;
-      case 1: NS2_TILED(NS2_ACT_NONE, 1); break;
-      case 2: NS2_TILED(NS2_ACT_NONE, 2); break;
-      case 3: NS2_TILED(NS2_ACT_SILU, 0); break;
-      case 4: NS2_TILED(NS2_ACT_SILU, 1); break;
-      case 5: NS2_TILED(NS2_ACT_SILU, 2); break;
-      case 6: NS2_TILED(NS2_ACT_GELU_TANH, 0); break;
-      case 7: NS2_TILED(NS2_ACT_GELU_TANH, 1); break;
-      default: NS2_TILED(NS2_ACT_GELU_TANH, 2); break;
+  auto run = [&](auto act_c, auto rm_c) {
+    constexpr int A = decltype(act_c)::value, R = decltype(rm_c)::value;
+    if constexpr (LORA) {
+      if (p.lr) {
+        gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, true, WF16, WPE><<<grid, block, 0, s>>>(p);
+        return;
+      }
     }
+    gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, false, WF16, WPE><<<grid, block, 0, s>>>(p);
+  };
+  using std::integral_constant;
+  if constexpr (EPI == 1) {
+    if (p.act == NS2_ACT_SILU) run(integral_constant<int, NS2_ACT_SILU>{}, integral_constant<int, 0>{});
+    else run(integral_constant<int, kActAny>{}, integral_constant<int, 0>{});
+  } else if (p.act == NS2_ACT_NONE) {
+    if constexpr (RESID) {
+      if (p.resid) run(integral_constant<int, NS2_ACT_NONE>{}, integral_constant<int, 1>{});
+    }
+    if (!p.resid) run(integral_constant<int, NS2_ACT_NONE>{}, integral_constant<int, 0>{});
+  } else if constexpr (ANY_ACT) {
+    if (p.resid) run(integral_constant<int, kActAny>{}, integral_constant<int, 1>{});
+    else run(integral_constant<int, kActAny>{}, integral_constant<int, 0>{});
   }
-#undef NS2_TILED
   NS2_LAUNCHED("gemm_tiled");
   if (p.part && reduce) {
     const long long mn = (long long)p.M * p.N;
@@ -698,36 +858,69 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   return NS2_OK;
 }
 
-// Block-tile configurations: BM x BN, the waves' layout, and two
-// throughput figures fitted to measurements at the DiT shapes (3952 x {4608, 1536, 8192} x
-// {1536, 4096}, 256 x 3072 x 1536), in tile-area units per microsecond at K = 1536: `rate`
-// with the CUs full, `alone` for a CU that runs a single tile of this shape.
+// Block tiles and their time model: a launch gives every CU `per` = ceil(tiles / 256) tiles, run as
+// rounds of up to `occ` co-resident blocks; a round of n blocks per CU takes e[n-1] + c[n-1] us per
+// 64-wide k-tile, and a launch L us more. The constants are least-squares fits to 139 measured
+// launches per tile (23 row counts from 64 to 3952, N x K of 4608/6144/8192/27648 x 1536 and 1536 x
+// 1536/4096/6144, weights cycled through 8 copies); choosing by the model costs 1.1 % on average
+// against the best tile of each of those launches.
+//   64x64, 4 waves (2 k groups)   few tiles: each block's k chain halved, three 128-wide stages
+//   64x128, 8 waves (2 k groups)  at most two tiles per CU (1024 x 1536 x 1536 +=: 14.4 -> 11.5 us)
+//   64x128, 4 waves               3 or 4 tiles per CU
+//   128x128, 4 waves              3 tiles per CU (1792 x 4608 x 1536: 35.4 -> 30.1 us)
+//   128x192, 4 waves              2 tiles per CU (2432 x 4608 x 1536: 47.2 -> 39.1 us)
+//   128x192, 8 waves (2 k groups) one tile per CU, long K (3952 x 1536 x 4096 +=: 62.2 -> 54.7 us)
+//   192x384, 8 waves              one tile per CU (3952 x 4608 x 1536: 70.3 -> 57.5 us)
+//   256x256, 8 waves              one tile per CU (3328 x 4608 x 1536: 51.9 -> 49.6 us)
+enum Tile { T64x64, T64x128K2, T64x128, T128x128, T128x192, T128x192K2, T192x384, T256x256, kTiles };
 struct TileCfg {
-  int bm, bn;
-  float rate, alone;
+  int bm, bn, occ;
+  float L, e[4], c[4];
 };
-constexpr TileCfg kCfgs[] = {
-    {256, 256, 1154.f, 1587.f},  // 16 waves (4 x 4) of 64x64, 96 KB LDS
-    {64, 128, 950.f, 532.f},     // 4 waves (1 x 4) of 64x32, 32 KB: each weight fragment decoded once
-    {64, 64, 350.f, 347.f},      // 4 waves (2 x 2) of 32x32, 36 KB (three stages): few rows (text tokens)
+constexpr TileCfg kCfgs[kTiles] = {
+    {64, 64, 2, 1.8f, {1.86f, 2.65f}, {0.210f, 0.322f}},
+    {64, 128, 2, 1.5f, {2.40f, 4.34f}, {0.294f, 0.474f}},
+    {64, 128, 4, 3.8f, {0.f, 1.49f, 3.17f, 0.f}, {0.413f, 0.510f, 0.731f, 1.147f}},
+    {128, 128, 3, 2.9f, {2.49f, 5.20f, 0.f}, {0.513f, 0.790f, 1.550f}},
+    {128, 192, 2, 0.9f, {5.77f, 0.f}, {0.696f, 1.497f}},
+    {128, 192, 1, 0.f, {8.83f}, {0.520f}},
+    {192, 384, 1, 0.f, {13.86f}, {1.199f}},
+    {256, 256, 1, 0.f, {12.80f}, {1.130f}},
 };
 constexpr int kCUs = 256;
+constexpr float kReduceUs = 4.0f;  // the reduce launch of a split-K linear (2.4 us of it the launch)
 
-// Estimated time: the tiles the busiest CU runs times the tile area over the full-CU rate, but
-// never less than one tile running alone. The configuration with the least estimate is used.
-int pick_config(int M, int N) {
-  int best = -1;
-  double best_t = 0;
-  for (int i = 0; i < (int)(sizeof(kCfgs) / sizeof(kCfgs[0])); ++i) {
-    const TileCfg& c = kCfgs[i];
-    const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    const long long per_cu = (tiles + kCUs - 1) / kCUs;
-    const double area = (double)c.bm * c.bn;
-    double t = per_cu * area / c.rate;
-    if (t < area / c.alone) t = area / c.alone;
-    if (best < 0 || t < best_t) {
-      best = i;
-      best_t = t;
+// Modelled time of `tiles` block tiles of configuration t over kt k-tiles each.
+float tile_time(const TileCfg& t, long long tiles, int kt) {
+  const long long per = (tiles + kCUs - 1) / kCUs, full = per / t.occ;
+  const int rem = (int)(per % t.occ);
+  float us = t.L + full * (t.e[t.occ - 1] + kt * t.c[t.occ - 1]);
+  if (rem) us += t.e[rem - 1] + kt * t.c[rem - 1];
+  return us;
+}
+
+long long tile_count(const TileCfg& t, int M, int N) {
+  return (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+}
+
+// The tile of the least modelled time, and for 64x64 tiles how many ways K is split (over
+// blockIdx.y, reduced in a second launch; at least 8 k-tiles per split). `allowed`: bit t for tile t.
+Tile pick_tile(int M, int N, int K, unsigned allowed, bool can_split, int* splits) {
+  const int kt = K / 64;
+  Tile best = T64x64;
+  float best_us = 0;
+  *splits = 0;
+  for (int i = 0; i < kTiles; ++i) {
+    if (!(allowed >> i & 1)) continue;
+    const long long tiles = tile_count(kCfgs[i], M, N);
+    const int most = i == T64x64 && can_split && tiles < kCUs ? (kt / 8 < 8 ? kt / 8 : 8) : 1;
+    for (int s = 1; s <= (most > 1 ? most : 1); ++s) {
+      const float us = tile_time(kCfgs[i], tiles * s, (kt + s - 1) / s) + (s > 1 ? kReduceUs : 0.f);
+      if (!*splits || us < best_us) {
+        best = (Tile)i;
+        best_us = us;
+        *splits = s;
+      }
     }
   }
   return best;
@@ -767,54 +960,42 @@ int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, 
     p.lr = lora_r;
   }
   ns2::ProfScope prof_(wf16 ? "gemm_f16_tiled" : "gemm_i8_tiled");
-  // the 256x256 tiles (16 waves, 128 registers each) have no room for the LoRA term's registers
-  int cfg = pick_config(M, N);
-  if (lora_r && cfg == 0) cfg = 1;
-  // Few rows (the 256 text tokens): when the 64x128 tiles do not cover the CUs more than once,
-  // 64x64 tiles, and when even those leave CUs idle, K split over blockIdx.y (reduced in a second
-  // launch) into about 320 blocks, at least 8 k-tiles per split and at most 8 splits. The
-  // weights of these launches come from HBM (each is read once per pass), so the splits hide
-  // its latency; measured at 256 rows with weights cycled through 320 MB (us, before -> after):
-  // 4608 x 1536 21.9 -> 17.8 (no split), 8192 x 1536 21.1 -> 18.8, 1536 x 1536 with += 13.0 ->
-  // 12.3 (3 splits), 1536 x 4096 with += 17.2 -> 16.8 (6 splits; 8 now).
-  int splits = 1;
-  if (cfg == 1 && (long long)((M + 63) / 64) * ((N + 127) / 128) <= kCUs) cfg = 2;
-  if (cfg != 0) {
-    const int bm = 64, bn = cfg == 1 ? 128 : 64;
-    const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  // The tiles a launch may take: activations (none of the models' tiled linears has one) are built
+  // for the two small tiles; fp16 weights for three tiles of one 64-wide k-tile per stage; the two
+  // largest tiles have no registers left for old outputs or the LoRA term, 128x128 (three blocks
+  // per CU) none for old outputs.
+  unsigned allowed = (1u << kTiles) - 1;
+  if (act != NS2_ACT_NONE) allowed = 1u << T64x64 | 1u << T64x128;
+  else if (wf16) allowed = 1u << T64x64 | 1u << T64x128 | 1u << T128x192K2;
+  else if (resid || lora_r) allowed &= ~(1u << T192x384 | 1u << T256x256 | (resid ? 1u << T128x128 : 0u));
+  int splits;
+  const Tile tile = pick_tile(M, N, K, allowed, !vpk, &splits);
+  if (splits > 1) {
     const int kt = K / 64;
-    if (tiles < kCUs && kt >= 16 && !vpk) {
-      splits = (int)((320 + tiles / 2) / tiles);
-      if (splits > kt / 8) splits = kt / 8;
-      if (splits > 8) splits = 8;
-      if (splits < 1) splits = 1;
-    }
-    if (splits > 1) {
-      p.ksplit = (kt + splits - 1) / splits;
-      splits = (kt + p.ksplit - 1) / p.ksplit;
-      p.part = static_cast<float*>(ns2::workspace(5, (size_t)splits * M * N * sizeof(float)));
-      if (!p.part) return ns2::set_error(NS2_ERR_OOM, "%s: split-K workspace allocation failed", fn);
-    }
+    p.ksplit = (kt + splits - 1) / splits;
+    if (!wf16) p.ksplit += p.ksplit & 1;  // whole 128-wide stages
+    splits = (kt + p.ksplit - 1) / p.ksplit;
+  }
+  if (splits > 1) {
+    p.part = static_cast<float*>(ns2::workspace(5, (size_t)splits * M * N * sizeof(float)));
+    if (!p.part) return ns2::set_error(NS2_ERR_OOM, "%s: split-K workspace allocation failed", fn);
   }
   if (wf16) {
-    switch (cfg) {
-      case 0: return launch_tiled<256, 256, 4, 4, 2, 0, true>(p);
-      case 1: return launch_tiled<64, 128, 1, 4, 2, 0, true>(p, splits);
-      default: return launch_tiled<64, 64, 2, 2, 2, 0, true>(p, splits);
+    switch (tile) {
+      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 1, 3, 1, 2, 0, true, true, true, true>(p, splits);
+      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 3, 0, true, true, true, true>(p);
+      default: return launch_tiled<128, 192, 2, 2, 2, 1, 2, 1, 2, 0, true>(p);
     }
   }
-  switch (cfg) {
-    case 0: return launch_tiled<256, 256, 4, 4>(p);
-    case 1:
-      // at most two blocks per CU (2432 x 1536 launches: 456 tiles) the copies' latency shows, and
-      // a third stage (48 KB, three blocks still fit) hides it: 2432 x 1536 x 6144 72.3 -> 69.6 us;
-      // at three blocks per CU (the DiT's 744-tile proj and w3) it costs more than it hides
-      if ((long long)((M + 63) / 64) * ((N + 127) / 128) <= 2 * kCUs) return launch_tiled<64, 128, 1, 4, 3>(p, splits);
-      return launch_tiled<64, 128, 1, 4>(p, splits);
-    // three stages: at a few rows each block runs alone on its CU and its weights come from HBM,
-    // so a deeper copy queue pays (text q/k/v 22.0 -> 17.0 us, text proj 15.4 -> 14.3 us in the
-    // pass); LDS is no limit at one block per CU
-    default: return launch_tiled<64, 64, 2, 2, 3>(p, splits);
+  switch (tile) {
+    case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, 0, false, true, true, true>(p, splits);
+    case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4>(p);
+    case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, 0, false, true, true, true>(p);
+    case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, 0, false, false>(p);
+    case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2>(p);
+    case T128x192K2: return launch_tiled<128, 192, 2, 2, 2, 2, 2, 2, 2>(p);
+    case T192x384: return launch_tiled<192, 384, 2, 4, 1, 1, 2, 2, 2, 0, false, false, false>(p);
+    default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, 0, false, false, false>(p);
   }
 }
 
@@ -841,7 +1022,7 @@ int ns2::linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_
   *part = p.part;
   *splits = s;
   ns2::ProfScope prof_("gemm_f16_tiled");
-  return launch_tiled<64, 64, 2, 2, 3, 0, true>(p, s, false);
+  return launch_tiled<64, 64, 2, 2, 1, 1, 3, 1, 2, 0, true, false, false>(p, s, false);
 }
 
 extern "C" {
@@ -894,7 +1075,7 @@ int ns2_linear_i8_glu_rot_tiled_lora(const uint16_t* At, const int8_t* Wt, const
     p.lr = lora_r;
   }
   ns2::ProfScope prof_("gemm_i8_glu_rot");
-  return launch_tiled<64, 512, 1, 8, 2, 1>(p);
+  return launch_tiled<64, 512, 1, 8, 1, 1, 2, 1, 4, 1>(p);
 }
 
 int ns2_linear_i8_tiled(const uint16_t* At, const int8_t* Wt, const float* scale, const float* bias,

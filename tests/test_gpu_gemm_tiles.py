@@ -1,0 +1,149 @@
+"""The block tiles of the tiled int8 / fp16 linears at their edges: ragged last rows and columns, the
+shortest K, split K, old outputs, the LoRA term and the packed values, each at a size whose launch
+takes the named tile (the time model of ns2_gemm_tiled.hip).
+
+The operands are given (fp16 activations, int8 weights), so the reference is the same product in
+float64 and the only error is that of fp32 sums: the K products of an output are added in fp32, a
+random walk of at most sqrt(K) 2^-24 of the result's size (4.7e-6 at K = 6144).
+"""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def tiled(x):
+    """fp16 [M, K] -> the tiled operand [ceil(M/64)][K/64][8][64][8], padding rows zero."""
+    M, K = x.shape
+    p = torch.zeros((M + 63) // 64 * 64, K, dtype=torch.float16, device=x.device)
+    p[:M] = x
+    return p.reshape(-1, 64, K // 64, 8, 8).permute(0, 2, 3, 1, 4).contiguous()
+
+
+def close(got, ref, K, what):
+    rel = ((got.double() - ref).norm() / ref.norm()).item()
+    print(f"[parity] {what}: rel-L2 {rel:.2e}", flush=True)
+    assert torch.isfinite(got).all() and rel <= math.sqrt(K) * 2.0**-24, what
+
+
+CASES = [
+    # tile, M, N, K, resid, LoRA rank
+    ("64x64", 33, 1536, 256, False, 0),
+    ("64x64 split K", 65, 1536, 4096, True, 0),
+    ("64x64 split K", 120, 1536, 6144, False, 32),
+    ("64x64", 64, 64, 1536, True, 32),
+    ("64x128, two k groups", 1025, 1536, 1536, True, 0),
+    ("64x128, two k groups", 999, 1536, 1536, False, 32),
+    ("64x128", 511, 4672, 1536, False, 0),
+    ("64x128", 513, 4672, 1536, True, 32),
+    ("128x128", 1537, 4672, 1536, False, 0),
+    ("128x128", 1800, 4608, 256, False, 32),
+    ("128x192", 2305, 4672, 1536, False, 0),
+    ("128x192", 2433, 4608, 1536, True, 32),
+    ("128x192, two k groups", 3951, 1536, 4096, True, 0),
+    ("128x192, two k groups", 2867, 1600, 6144, False, 32),
+    ("192x384", 3951, 4672, 1536, False, 0),
+    ("192x384", 3800, 4608, 256, False, 0),
+    ("256x256", 3329, 4672, 1536, False, 0),
+]
+
+
+@pytest.mark.parametrize("tile,M,N,K,resid,rank", CASES)
+def test_i8_tiles(ns2lib, tile, M, N, K, resid, rank):
+    print(f"[case] {tile} {M}x{N}x{K} resid {resid} rank {rank}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    bias = torch.randn(N, generator=g, device=DEV)
+    gate = torch.randn(N, generator=g, device=DEV)
+    wt = torch.empty_like(q)
+    ns2lib.tile_i8_weight(q, wt, N, K)
+    ref = (x.double() @ q.double().T) * s.double() + bias.double()
+    lora = None
+    if rank:
+        a = (torch.randn(rank, K, generator=g, device=DEV) / math.sqrt(K)).half()
+        b = (torch.randn(N, rank, generator=g, device=DEV) / math.sqrt(rank)).half()
+        lora = (a, b, rank)
+        # the term's own rounding: t = x a^T is rounded to fp16 for the second product
+        ref = ref + (x.double() @ a.double().T).half().double() @ b.double().T
+    buf = torch.randn(M + 300, N, generator=g, device=DEV)
+    before = buf.clone()
+    ns2lib.linear_i8_tiled(tiled(x), wt, s, buf, M, N, K, bias=bias, resid=resid, gate=gate if resid else None, lora=lora)
+    torch.cuda.synchronize()
+    assert torch.equal(buf[M:], before[M:]), "rows past M were written"
+    if resid:
+        ref = before[:M].double() + gate.double() * ref
+    if rank:
+        # t computed in fp32 may round to the other fp16 neighbour: 2^-11 of the term in few places
+        rel = ((buf[:M].double() - ref).norm() / ref.norm()).item()
+        assert rel <= 2.0**-12, f"{tile}: {rel:.2e}"
+    else:
+        close(buf[:M], ref, K, f"{tile} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("tile,M,N,K,resid", [("64x64", 70, 64, 64, False), ("64x64 split K", 65, 1536, 1600, True),
+                                              ("64x128", 1000, 1536, 64, False), ("128x192", 3951, 1600, 1536, True)])
+def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
+    print(f"[case] {tile} {M}x{N}x{K} resid {resid}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    wt = torch.empty_like(w)
+    ns2lib.tile_bf16_weight(w, wt, N, K)
+    buf = torch.randn(M + 200, N, generator=g, device=DEV)
+    before = buf.clone()
+    ns2lib.linear_f16w_tiled(tiled(x), wt, buf, M, N, K, resid=resid)
+    torch.cuda.synchronize()
+    assert torch.equal(buf[M:], before[M:]), "rows past M were written"
+    ref = x.double() @ w.half().double().T
+    close(buf[:M], before[:M].double() + ref if resid else ref, max(K, 1024), f"{tile} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("M,act", [(96, "silu"), (1000, "gelu_tanh")])
+def test_i8_activation(ns2lib, M, act):
+    N, K = 1536, 512
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    wt, y = torch.empty_like(q), torch.empty(M, N, device=DEV)
+    ns2lib.tile_i8_weight(q, wt, N, K)
+    ns2lib.linear_i8_tiled(tiled(x), wt, s, y, M, N, K, act=act)
+    torch.cuda.synchronize()
+    z = (x.double() @ q.double().T) * s.double()
+    ref = torch.nn.functional.silu(z) if act == "silu" else torch.nn.functional.gelu(z, approximate="tanh")
+    close(y, ref, 1024, act)
+
+
+# head dims and counts whose value columns start inside a wave's columns (3200 is no multiple of 96)
+@pytest.mark.parametrize("M,N,K,H,HD", [(3952, 4608, 512, 22, 64), (3328, 4608, 512, 16, 96), (2304, 4608, 512, 22, 64),
+                                        (1536, 4608, 512, 16, 96), (48, 4608, 512, 22, 64)])
+def test_vpack_tiles(ns2lib, M, N, K, H, HD):
+    """The packed values equal the fp16 roundings of the plain store's columns, key by key, and the
+    other columns equal the plain store's."""
+    print(f"[case] vpack {M}x{N}x{K} heads {H}x{HD}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = tiled(torch.randn(M, K, generator=g, device=DEV).half())
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    wt = torch.empty_like(q)
+    ns2lib.tile_i8_weight(q, wt, N, K)
+    Lk, vcol0 = M + 20, N - H * HD
+    tiles = (Lk + 63) // 64
+    plain, y = torch.empty(M, N, device=DEV), torch.zeros(M, N, device=DEV)
+    vpk = torch.zeros(H * tiles * 64 * HD, dtype=torch.float16, device=DEV)
+    ns2lib.linear_i8_tiled(x, wt, s, plain, M, N, K)
+    ns2lib.linear_i8_tiled_vpack(x, wt, s, y, M, N, K, vpk, vcol0=vcol0, H=H, D=HD, Lk=Lk)
+    torch.cuda.synchronize()
+    assert torch.equal(y[:, :vcol0], plain[:, :vcol0])
+    # [head][tile][chunk][dim][8]: chunk 2g + hi holds keys 16g + 4hi + {0..3}, 16g + 8 + 4hi + {0..3}
+    v = vpk.reshape(H, tiles, 4, 2, HD, 2, 4).permute(1, 2, 5, 3, 6, 0, 4).reshape(tiles * 64, H * HD)
+    # no K split with packed values, so where the plain launch splits K the sums differ in association
+    if torch.equal(v[:M], plain[:, vcol0:].half()):
+        return
+    close(v[:M].float(), plain[:, vcol0:].double(), 2.0**26, "packed values")  # fp16: 2^-11
