@@ -120,6 +120,41 @@ def test_i8_activation(ns2lib, M, act):
     close(y, ref, 1024, act)
 
 
+# 1030: 17 row blocks of 64, so the last 128-row tile holds one real block; 1090: a ragged second one
+@pytest.mark.parametrize("tile,M,N,K,rank", [("128x512", 1030, 8192, 256, 0), ("128x512", 1090, 8192, 1536, 32),
+                                             ("64x512", 1024, 8192, 256, 0), ("64x512", 2100, 8192, 256, 32)])
+def test_glu_tiles(ns2lib, tile, M, N, K, rank):
+    """The GLU + rotation epilogue's block tiles: one fp16 rounding of the result (2^-11 of a value at
+    most), with a LoRA the rounding of its down-projection too; rows past the last row block stay."""
+    print(f"[case] glu {tile} {M}x{N}x{K} rank {rank}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    h = (x.double() @ q.double().T) * s.double()
+    lora = None
+    if rank:
+        a = (torch.randn(rank, K, generator=g, device=DEV) / math.sqrt(K)).half()
+        b = (torch.randn(N, rank, generator=g, device=DEV) / math.sqrt(rank)).half()
+        lora = (a, b, rank)
+        h = h + (x.double() @ a.double().T).half().double() @ b.double().T
+    I, rows = N // 2, (M + 63) // 64 * 64
+    y = (torch.nn.functional.silu(h[:, :I]) * h[:, I:]).reshape(M, I // 256, 256)
+    h4 = torch.tensor([[1, 1, 1, -1], [1, 1, -1, 1], [1, -1, 1, 1], [-1, 1, 1, 1]], dtype=torch.float64, device=DEV)
+    had = torch.kron(torch.kron(h4, h4), torch.kron(h4, h4)) / 16
+    ref = (y @ had).reshape(M, I)
+    wt = torch.empty_like(q)
+    ns2lib.tile_i8_weight_glu(q, wt, N, K)
+    out = torch.full((rows + 64, I), -7.0, dtype=torch.float16, device=DEV)
+    ns2lib.linear_i8_glu_rot_tiled(tiled(x), wt, s, out, M, N, K, act="silu", lora=lora)
+    torch.cuda.synchronize()
+    assert (out[rows:] == -7.0).all(), "rows past the last row block were written"
+    got = out[:rows].reshape(rows // 64, I // 64, 8, 64, 8).permute(0, 3, 1, 2, 4).reshape(rows, I)[:M]
+    rel = ((got.double() - ref).norm() / ref.norm()).item()
+    print(f"[parity] glu {tile}: rel-L2 {rel:.2e}", flush=True)
+    assert torch.isfinite(got).all() and rel <= (2.0**-10 if rank else 2.0**-11)
+
+
 # head dims and counts whose value columns start inside a wave's columns (3200 is no multiple of 96)
 @pytest.mark.parametrize("M,N,K,H,HD", [(3952, 4608, 512, 22, 64), (3328, 4608, 512, 16, 96), (2304, 4608, 512, 22, 64),
                                         (1536, 4608, 512, 16, 96), (48, 4608, 512, 22, 64)])
