@@ -256,8 +256,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma_kernel(G
   // epilogue
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * WN + j * 32 + lrow;
-    if (n >= p.N) continue;
+    const int nr = n0 + wn * WN + j * 32 + lrow;
+    if (!LORA && nr >= p.N) continue;
+    // the LoRA products take rows of t from every lane: lanes past N stay in, on the last column
+    const int n = nr < p.N ? nr : p.N - 1;
     const float rs = p.scale ? p.scale[n] : 1.0f;
     const float bi = p.bias ? p.bias[n] : 0.0f;
     const float gt = p.gate ? p.gate[p.gOff + n] : 1.0f;
@@ -271,7 +273,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma_kernel(G
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < p.M) epilogue_store(p, m, n, acc[i][j][r], rs, bi, gt, LORA ? d[r] : 0.f);
+        if (m < p.M && (!LORA || nr < p.N)) epilogue_store(p, m, n, acc[i][j][r], rs, bi, gt, LORA ? d[r] : 0.f);
       }
     }
   }

@@ -104,6 +104,24 @@ def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
     close(buf[:M], before[:M].double() + ref if resid else ref, max(K, 1024), f"{tile} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(1001, 1616, 768), (65, 4120, 256)])
+def test_lora_ragged_columns(ns2lib, M, N, K):
+    """Row-major kernel, LoRA, N no multiple of 32: the last columns' low-rank term takes every lane's
+    rows (t's fp16 rounding: 2^-12 of the result)."""
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    a = (torch.randn(32, K, generator=g, device=DEV) / math.sqrt(K)).half()
+    b = (torch.randn(N, 32, generator=g, device=DEV) / math.sqrt(32)).half()
+    y = torch.empty(M, N, device=DEV)
+    ns2lib.linear_i8(x, 1, K, q, s, y, M, N, K, lora=(a, b, 32))
+    ref = (x.double() @ q.double().T) * s.double() + (x.double() @ a.double().T).half().double() @ b.double().T
+    for cols in (slice(0, N), slice(N // 32 * 32, N)):
+        rel = ((y[:, cols].double() - ref[:, cols]).norm() / ref[:, cols].norm()).item()
+        assert rel <= 2.0**-12, f"columns {cols}: {rel:.2e}"
+
+
 @pytest.mark.parametrize("M,act", [(96, "silu"), (1000, "gelu_tanh")])
 def test_i8_activation(ns2lib, M, act):
     N, K = 1536, 512
