@@ -792,6 +792,21 @@ __global__ __launch_bounds__(256) void tile_w16_kernel(const uint16_t* __restric
   *reinterpret_cast<uint4*>(Wt + i * 8) = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
+// x [M][ldx] row-major fp16 -> the tiled operand [ceil(M/64)][K/64][8][64][8], one thread per 16-byte
+// chunk; rows past M repeat the last one (their products are dropped).
+__global__ __launch_bounds__(256) void tile_x16_kernel(const uint16_t* __restrict__ x, int ldx, uint16_t* __restrict__ xt,
+                                                        int M, int K) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;  // output chunk index
+  const int row = (int)(i % 64);
+  const int c = (int)((i / 64) % 8);
+  const long long rest = i / 512;  // mb * (K/64) + kb
+  const int kb = (int)(rest % (K / 64));
+  const long long m = rest / (K / 64) * 64 + row;
+  if (m >= ((M + 63) & ~63)) return;
+  *reinterpret_cast<uint4*>(xt + i * 8) =
+      *reinterpret_cast<const uint4*>(x + (m < M ? m : M - 1) * ldx + kb * 64 + c * 8);
+}
+
 // Weight bytes per column band of the tile order: half of an XCD's 4 MB L2.
 constexpr long long kBandBytes = 2ll << 20;
 
@@ -1000,6 +1015,24 @@ int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, 
 }
 
 }  // namespace
+
+int ns2::linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, const float* scale,
+                           const float* bias, float* C, int M, int N, int K, int ldc, long long cOff, float alpha,
+                           int act, int resid, const float* gate, long long gOff, const uint16_t* lora_a,
+                           const uint16_t* lora_b, int lora_r) {
+  if (x16) {
+    const long long chunks = (long long)((M + 63) / 64) * 64 * K / 8;
+    ns2::ProfScope prof_("tile_f16_rows");
+    tile_x16_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, ns2::stream()>>>(x16, ldx, At, M, K);
+    NS2_LAUNCHED("tile_f16_rows");
+  }
+  int8_t* Wt = static_cast<int8_t*>(ns2::workspace(7, (size_t)N * K));
+  if (!Wt) return ns2::set_error(NS2_ERR_OOM, "ns2_linear_i8: weight workspace allocation failed");
+  int rc = ns2_tile_i8_weight(W, Wt, N, K);
+  if (rc) return rc;
+  return linear_tiled("ns2_linear_i8", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate, gOff,
+                      lora_a, lora_b, lora_r);
+}
 
 int ns2::linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_t* Wt, int M, int N, int K,
                                float** part, int* splits) {

@@ -104,6 +104,59 @@ def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
     close(buf[:M], before[:M].double() + ref if resid else ref, max(K, 1024), f"{tile} {M}x{N}x{K}")
 
 
+# both sides of the rule that re-tiles file-layout operands: rows, work, 64-row weight blocks
+@pytest.mark.parametrize("route,M,N,K,resid,rank,act", [
+    ("tiled", 400, 2560, 1024, True, 0, "none"), ("rows", 399, 2560, 1024, True, 0, "none"),
+    ("tiled", 1001, 1600, 768, False, 32, "none"), ("rows", 1001, 1616, 768, False, 32, "none"),
+    ("tiled", 3953, 64, 4096, True, 0, "silu"), ("rows", 3953, 64, 3840, True, 0, "silu"),
+])
+def test_i8_file_layout(ns2lib, route, M, N, K, resid, rank, act):
+    """The int8 linear on a file-layout weight (every int8 value, strided rows, a column window of C) for
+    its three input formats; fp16-exact inputs, so the error is that of fp32 sums."""
+    print(f"[case] file layout {route} {M}x{N}x{K} resid {resid} rank {rank} {act}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    lda, ldc = K + 64, N + 32
+    x = torch.randn(M, lda, generator=g, device=DEV).half()
+    q = torch.randint(-128, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    bias, gate = torch.randn(N, generator=g, device=DEV), torch.randn(N, generator=g, device=DEV)
+    xk = x[:, :K].double()
+    ref = (xk @ q.double().T) * s.double() + bias.double()
+    lora = None
+    if rank:
+        a = (torch.randn(rank, K, generator=g, device=DEV) / math.sqrt(K)).half()
+        b = (torch.randn(N, rank, generator=g, device=DEV) / math.sqrt(rank)).half()
+        lora = (a, b, rank)
+        ref = ref + (xk @ a.double().T).half().double() @ b.double().T
+    if act == "silu":
+        ref = torch.nn.functional.silu(ref)
+    base = torch.randn(M, ldc, generator=g, device=DEV)
+    if resid:
+        ref = base[:, 32:].double() + gate.double() * ref
+    kw = dict(bias=bias, resid=resid, gate=gate if resid else None, lora=lora, ldc=ldc, cOff=32, act=act)
+    outs = {}
+    for fmt, src in ((1, x), (2, x.float())):
+        y = base.clone()
+        ns2lib.linear_i8(src, fmt, lda, q, s, y, M, N, K, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(y[:, :32], base[:, :32]), "columns left of the window were written"
+        outs[fmt] = y
+    assert torch.equal(outs[1], outs[2])
+    got = outs[1][:, 32:]
+    if rank:  # t = x a^T may round to the other fp16 neighbour
+        assert ((got.double() - ref).norm() / ref.norm()).item() <= 2.0**-12
+    else:
+        close(got, ref, K, f"file layout {route} {M}x{N}x{K}")
+    # unrotated fp32 input: the same as the rotated rows given as fp16
+    xr = torch.empty(M, K, dtype=torch.float16, device=DEV)
+    ns2lib.rotate_f16(x.float(), lda, xr, K, M, K)
+    y0, y1 = base.clone(), base.clone()
+    ns2lib.linear_i8(x.float(), 0, lda, q, s, y0, M, N, K, **kw)
+    ns2lib.linear_i8(xr, 1, K, q, s, y1, M, N, K, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(y0, y1)
+
+
 @pytest.mark.parametrize("M,N,K", [(1001, 1616, 768), (65, 4120, 256)])
 def test_lora_ragged_columns(ns2lib, M, N, K):
     """Row-major kernel, LoRA, N no multiple of 32: the last columns' low-rank term takes every lane's
