@@ -560,10 +560,12 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[qt][dt][r] = 0.f;
   float m_ref[QT], l_run[QT];
+  bool fresh[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     m_ref[qt] = 0.f;
     l_run[qt] = 0.f;
+    fresh[qt] = true;
   }
 
   TileLoader<D, NW> loader(Kt, Vt, Bg, lds_addr(ks), lds_addr(vts), lds_addr(kbias), wave, lane);
@@ -692,19 +694,22 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
         if (MORE && first + r < ntiles) dma(first + r, (first + r) % NSLOT);
     }
 
-    // ---- move the reference when a score exceeds it by more than 2^kRebase, or when nothing
-    // has been accumulated yet (l = 0: the tile maximum becomes the reference, so the largest
-    // p is 1 and l >= 1 afterwards); the running sum and output scale by 2^-shift and the
-    // tile's relative scores drop by shift
+    // ---- move the reference when a score exceeds it by more than 2^kRebase, or when the query has
+    // seen no finite score yet (fresh: the tile maximum becomes the reference, so the largest p is
+    // 1); the running sum and output scale by 2^-shift and the tile's relative scores drop by shift.
+    // mx and fresh are those of the query, the same in its two lanes: a lane's own row sum says
+    // nothing (the 32 keys of one lane may all round to p = 0 while the other's do not)
     {
       bool need = false;
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) need |= (mx_cur[qt] > kRebase) || (l_run[qt] == 0.f);
+      for (int qt = 0; qt < QT; ++qt) need |= (mx_cur[qt] > kRebase) || fresh[qt];
       if (__builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-          const float shift = (l_run[qt] == 0.f) ? mx_cur[qt] : fmaxf(mx_cur[qt], 0.f);
-          const float alpha = __builtin_amdgcn_exp2f(-shift);
+          const bool seen = mx_cur[qt] > -INFINITY;
+          const float shift = fresh[qt] ? (seen ? mx_cur[qt] : 0.f) : fmaxf(mx_cur[qt], 0.f);
+          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift);
+          fresh[qt] = fresh[qt] && !seen;
           m_ref[qt] += shift;
           l_run[qt] *= alpha;
 #pragma unroll
@@ -926,11 +931,13 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[qt][dt][r] = 0.f;
   float m_ref[QT], l_run[QT];
+  bool fresh[QT];
   float16_t minit[QT];  // -m_ref in every accumulator slot: the C operand of each score chain
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     m_ref[qt] = 0.f;
     l_run[qt] = 0.f;
+    fresh[qt] = true;
 #pragma unroll
     for (int r = 0; r < 16; ++r) minit[qt][r] = 0.f;
   }
@@ -1016,20 +1023,23 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
           }
         }
     }
-    // ---- the reference moves when a score exceeds it by more than 2^kRebase, or on the first
-    // tile (nothing accumulated yet: the reference becomes the tile maximum)
+    // ---- the reference moves when a score exceeds it by more than 2^kRebase, or on the query's first
+    // tile with a finite score (fresh: the reference becomes the tile maximum); as in flash_kernel,
+    // the same in the query's two lanes
     {
       float mx[QT];
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) mx[qt] = col_max(__builtin_fmaxf(half_max(s[0][qt]), half_max(s[1][qt])));
       bool need = false;
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) need |= (mx[qt] > kRebase) || (l_run[qt] == 0.f);
+      for (int qt = 0; qt < QT; ++qt) need |= (mx[qt] > kRebase) || fresh[qt];
       if (__builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-          const float shift = (l_run[qt] == 0.f) ? mx[qt] : fmaxf(mx[qt], 0.f);
-          const float alpha = __builtin_amdgcn_exp2f(-shift);
+          const bool seen = mx[qt] > -INFINITY;
+          const float shift = fresh[qt] ? (seen ? mx[qt] : 0.f) : fmaxf(mx[qt], 0.f);
+          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift);
+          fresh[qt] = fresh[qt] && !seen;
           m_ref[qt] += shift;
           l_run[qt] *= alpha;
 #pragma unroll

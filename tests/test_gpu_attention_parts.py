@@ -1,0 +1,62 @@
+"""The flash kernels' softmax state: references that must agree between the two lanes of a query.
+
+The reference is the same attention in float64 on the fp32 inputs. q, k, v and P are rounded to fp16
+(2^-11 each): a score is off by about |q||k| 2^-11 / sqrt(D), which stays below 2^-9 for unit inputs,
+and the output by that plus P's and v's rounding, under 2^-8 of its size in all.
+"""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def reference(q, k, v, bias, start):
+    """q [B, Lq, H, D], k and v [B, Lk, H, D] -> [B, Lq, H, D] in float64."""
+    s = (q.double().transpose(1, 2).unsqueeze(3) * k.double().transpose(1, 2).unsqueeze(2)).sum(-1) / math.sqrt(q.shape[-1])
+    if bias is not None:
+        s[..., start:] += bias.double()[:, None, None, :]
+    return (torch.softmax(s, -1).unsqueeze(-1) * v.double().transpose(1, 2).unsqueeze(2)).sum(3).transpose(1, 2)
+
+
+def run(lib, q, k, v, bias=None, start=0):
+    B, Lq, H, D = q.shape
+    Lk = k.shape[1]
+    o = torch.full((B, Lq + 3, H, D), 9.0, device=DEV)
+    W = H * D
+    lib.attention(q, k, v, o, Lq=Lq, Lk=Lk, H=H, D=D, ldq=W, ldk=W, ldv=W, ldo=W, batch=B, qBatch=Lq * W, kBatch=Lk * W,
+                  vBatch=Lk * W, oBatch=(Lq + 3) * W, key_bias=bias, biasStart=start, biasBatch=Lk - start if bias is not None else 0)
+    torch.cuda.synchronize()
+    assert (o[:, Lq:] == 9.0).all(), "rows past Lq were written"
+    return o[:, :Lq]
+
+
+def check(got, ref, what):
+    rel = ((got.double() - ref).norm() / ref.norm()).item()
+    print(f"[parity] {what}: rel-L2 {rel:.2e}", flush=True)
+    assert torch.isfinite(got).all() and rel <= 2.0**-8, what
+
+
+# (batch, heads, queries): the 256-query and the 512-query kernel
+ROUTES = {"256 queries": (2, 120, 129), "512 queries": (2, 128, 65)}
+
+
+@pytest.mark.parametrize("route", ROUTES)
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_half_of_a_tile_vanishes(ns2lib, route, D):
+    """The keys one lane of a query holds all underflow in the first tile, and no later score reaches the
+    first tile's maximum: the lanes' references have to stay together all the same."""
+    B, H, Lq = ROUTES[route]
+    Lk = 256
+    g = torch.Generator(device=DEV).manual_seed(D)
+    v = torch.randn(B, Lk, H, D, generator=g, device=DEV)
+    q = torch.ones(B, Lq, H, D, device=DEV)
+    key = torch.arange(Lk, device=DEV)
+    for lane in (0, 4):
+        score = torch.where(key < 64, torch.where((key & 4) == lane, 0.0, -40.0), -3.0)  # of sqrt(D)-scaled q k
+        k = (score / math.sqrt(D))[None, :, None, None].expand(B, Lk, H, D).contiguous()
+        check(run(ns2lib, q, k, v), reference(q, k, v, None, 0), f"{route} D={D} lane bit {lane}")
+
