@@ -505,17 +505,21 @@ struct TileLoader {
 // rescale. Any reference gives the same softmax, and p <= 2^kRebase stays in fp16 range.
 constexpr float kRebase = 8.0f;
 
-// SUPER: 64-key tiles per LDS stage. The loads of a stage are issued together and waited for
-// with one barrier, so a barrier falls on every SUPER-th step and a stage's loads are issued
-// (STAGES - 2) * SUPER + 1 .. (STAGES - 1) * SUPER steps before its K fragments are read.
-template <int D, int QT, int NW, int STAGES, int SUPER>
+// KS: key parts. The NW waves of a block are NW / KS query waves times KS key parts: a stage holds KS
+// consecutive tiles and part g works on tile u KS + g of stage u; the parts' outputs, references and
+// row sums are merged through LDS at the end. Two parts halve a block's queries and its chain of tiles,
+// for grids whose 256-query blocks leave CUs idle (launch_flash_auto).
+template <int D, int QT, int NW, int KS>
 __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
-  constexpr int DC = D / 16;             // k-steps of S
-  constexpr int DT = D / 32;             // dim tiles of O
-  constexpr int TILE = KB * D;           // halfs per K (or V) tile image
-  constexpr int NSLOT = STAGES * SUPER;  // tile slots in LDS; tile t lives in slot t % NSLOT
-  static_assert(STAGES == 3 || (STAGES == 4 && SUPER == 1), "three stages, or four of one tile");
-  static_assert(SUPER == 1 || SUPER == 2, "one or two tiles per stage");
+  constexpr int DC = D / 16;          // k-steps of S
+  constexpr int DT = D / 32;          // dim tiles of O
+  constexpr int TILE = KB * D;        // halfs per K (or V) tile image
+  constexpr int STAGES = 3;
+  constexpr int NSLOT = STAGES * KS;  // tile slots in LDS; tile t lives in slot t % NSLOT
+  constexpr int QW = NW / KS;         // query waves
+  static_assert((KS == 1 || KS == 2) && NW % KS == 0, "one or two key parts");
+  static_assert((size_t)(KS - 1) * QW * QT * DT * 4096 <= (size_t)NSLOT * TILE * 2, "merge buffer: the K slots");
+  static_assert(QW * QT * 512 <= NSLOT * TILE * 2, "references and row sums: the V slots");
 
   // K of tile t+1 and V of tile t are read while the later stages land
   __shared__ __attribute__((aligned(16))) half_t ks[NSLOT][TILE];
@@ -541,9 +545,12 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
   const int b = pair / a.H, h = pair % a.H, bh = pair;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = qb * (NW * QT * 32) + wave * QT * 32;
+  const int kg = KS > 1 ? wave / QW : 0, wq = KS > 1 ? wave % QW : wave;
+  const int q0 = qb * (QW * QT * 32) + wq * QT * 32;
   const int lq = lane & 31, hi = lane >> 5;
   const int ntiles = a.Lk_pad / KB;
+  // stages, and this part's tiles (at least one: two parts need two tiles)
+  const int stages = (ntiles + KS - 1) / KS, n = (ntiles - kg + KS - 1) / KS;
 
   const half_t* Kt = a.Kc + (long long)bh * ntiles * TILE;
   const half_t* Vt = a.Vc + (long long)bh * ntiles * TILE;
@@ -640,24 +647,24 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
     return __builtin_fmaxf(lo, hi2);
   };
 
-  // Software pipeline, one barrier per tile. Step t:
-  //   wait for this wave's loads of tile t+1, barrier (every wave's loads of tile t+1 have
-  //   landed; every wave is done with step t-1), start loading tile t+STAGES-1 into the stage
-  //   that held tile t-1;
+  // Software pipeline, one barrier per stage. Step u, t = u KS + kg this part's tile:
+  //   wait for this wave's loads of stage u+1, barrier (every wave's loads of stage u+1 have
+  //   landed; every wave is done with step u-1), start loading stage u+STAGES-1 into the slots
+  //   that held stage u-1;
   //   move the softmax reference if tile t needs it (rare);
-  //   phase A: scores of tile t+1 on the MFMA pipe, K fragments read two MFMA groups ahead,
+  //   phase A: scores of tile t+KS on the MFMA pipe, K fragments read two MFMA groups ahead,
   //            the exp/convert/sum of tile t spread between the MFMA groups;
   //   phase B: O += V_t P_t on the MFMA pipe, V fragments read two MFMA groups ahead, the key
-  //            bias (for the tiles that have one) and row max of tile t+1 between them.
-  // Steps alternate the two score buffers (A holds tile t, B receives tile t+1).
+  //            bias (for the tiles that have one) and row max of tile t+KS between them.
+  // Steps alternate the two score buffers (A holds tile t, B receives tile t+KS).
   float16_t sA[2][QT], sB[2][QT];
   float mA[QT], mB[QT];
-  const int issued = (STAGES - 1) * SUPER < ntiles ? (STAGES - 1) * SUPER : ntiles;
+  const int issued = (STAGES - 1) * KS < ntiles ? (STAGES - 1) * KS : ntiles;
   for (int i = 0; i < issued; ++i) dma(i, i);
   {
-    // the first stage (tiles 0 .. SUPER-1) has landed once at most the tiles issued after it
-    // remain in flight
-    const int newer = issued - (SUPER < ntiles ? SUPER : ntiles);
+    // the first stage (tiles 0 .. KS-1) has landed once at most the tiles issued after it remain
+    // in flight
+    const int newer = issued - (KS < ntiles ? KS : ntiles);
     if (newer >= 2) wait_newer(W2_{});
     else if (newer == 1) wait_newer(W1_{});
     else wait_newer(W0_{});
@@ -668,31 +675,43 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
   for (int i = 0; i < NK; ++i) qk_mfma(sA, i, read_k(i, 0));
   if (0 >= a.bias_block0) add_bias(sA, 0);
 
+  auto row_max = [&]() {
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
-    const float m = fmaxf(half_max(sA, 0, qt), half_max(sA, 1, qt));
-    mA[qt] = col_max(m);
+    for (int qt = 0; qt < QT; ++qt) {
+      const float m = fmaxf(half_max(sA, 0, qt), half_max(sA, 1, qt));
+      mA[qt] = col_max(m);
+    }
+  };
+  row_max();
+  if (KS == 2 && kg == 1) {
+    // part 1 takes its reference from tile 0 as part 0 does, so that P is rounded as one part would
+    // round it (unless the reference moves), then scores its own first tile
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      fresh[qt] = !(mA[qt] > -INFINITY);
+      m_ref[qt] = fresh[qt] ? 0.f : mA[qt];
+    }
+    set_minit();
+#pragma unroll
+    for (int i = 0; i < NK; ++i) qk_mfma(sA, i, read_k(i, 1));
+    if (1 >= a.bias_block0) add_bias(sA, 1);
+    row_max();
   }
 
-  auto step = [&](int t, float16_t (&s_cur)[2][QT], float16_t (&s_nxt)[2][QT], float (&mx_cur)[QT],
-                  float (&mx_nxt)[QT], auto more_c, auto bias_c, auto sync_c) {
+  auto step = [&](int u, float16_t (&s_cur)[2][QT], float16_t (&s_nxt)[2][QT], float (&mx_cur)[QT],
+                  float (&mx_nxt)[QT], auto more_c, auto bias_c) {
     constexpr bool MORE = decltype(more_c)::value;
-    constexpr bool BIAS = decltype(bias_c)::value;  // tile t+1 carries a key bias
-    constexpr bool SYNC = decltype(sync_c)::value;  // t is the first tile of its stage
-    const int vbuf = t % NSLOT, kbuf = (t + 1) % NSLOT;
-    // On the first step of stage u: the next stage (which holds tile t+1 for SUPER = 1, and the
-    // K of tile t+SUPER that step t+SUPER-1 reads) has landed once at most the tiles issued after
-    // it remain in flight; the barrier then covers every wave's loads, and every wave's reads of
-    // stage u-1, which the loads of stage u+STAGES-1 overwrite
-    if (SYNC) {
-      if (MORE && STAGES == 4 && t + 2 < ntiles) wait_newer(W1_{});
-      else wait_newer(W0_{});
-      __syncthreads();
-      const int first = (t / SUPER + STAGES - 1) * SUPER;
+    constexpr bool BIAS = decltype(bias_c)::value;  // the next tile carries a key bias
+    const int vbuf = (u * KS + kg) % NSLOT, kbuf = ((u + 1) * KS + kg) % NSLOT;
+    // this wave's loads of stage u+1 have landed; the barrier then covers every wave's loads, and
+    // every wave's reads of stage u-1, which the loads of stage u+STAGES-1 overwrite (a part that
+    // ends here, !MORE, is in one of the last two stages: nothing is left to load)
+    wait_newer(W0_{});
+    __syncthreads();
+    const int first = (u + STAGES - 1) * KS;
 #pragma unroll
-      for (int r = 0; r < SUPER; ++r)
-        if (MORE && first + r < ntiles) dma(first + r, (first + r) % NSLOT);
-    }
+    for (int r = 0; r < KS; ++r)
+      if (MORE && first + r < ntiles) dma(first + r, (first + r) % NSLOT);
 
     // ---- move the reference when a score exceeds it by more than 2^kRebase, or when the query has
     // seen no finite score yet (fresh: the tile maximum becomes the reference, so the largest p is
@@ -819,25 +838,64 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
   using F_ = std::integral_constant<bool, false>;
   // Steps before tb feed tiles without a key bias; tb is rounded down to even (adding the zero
   // bias of image keys is harmless) so the first loop ends on the A buffer.
-  int tb = a.bias_block0 - 1;
-  tb = tb < 0 ? 0 : (tb > ntiles - 1 ? ntiles - 1 : tb);
+  int tb = a.bias_block0 / KS - 1;
+  tb = tb < 0 ? 0 : (tb > n - 1 ? n - 1 : tb);
   tb &= ~1;
-  // steps go in pairs from an even t, so with SUPER = 2 the first step of a pair starts a stage
-  using S2_ = std::integral_constant<bool, SUPER == 1>;
-  int t = 0;
-  for (; t < tb; t += 2) {
-    step(t, sA, sB, mA, mB, T_{}, F_{}, T_{});
-    step(t + 1, sB, sA, mB, mA, T_{}, F_{}, S2_{});
+  int u = 0;
+  for (; u < tb; u += 2) {
+    step(u, sA, sB, mA, mB, T_{}, F_{});
+    step(u + 1, sB, sA, mB, mA, T_{}, F_{});
   }
-  for (; t + 2 < ntiles; t += 2) {
-    step(t, sA, sB, mA, mB, T_{}, T_{}, T_{});
-    step(t + 1, sB, sA, mB, mA, T_{}, T_{}, S2_{});
+  for (; u + 2 < n; u += 2) {
+    step(u, sA, sB, mA, mB, T_{}, T_{});
+    step(u + 1, sB, sA, mB, mA, T_{}, T_{});
   }
-  if (t + 1 < ntiles) {
-    step(t, sA, sB, mA, mB, T_{}, T_{}, T_{});
-    step(t + 1, sB, sA, mB, mA, F_{}, F_{}, S2_{});
+  if (u + 1 < n) {
+    step(u, sA, sB, mA, mB, T_{}, T_{});
+    step(u + 1, sB, sA, mB, mA, F_{}, F_{});
   } else {
-    step(t, sA, sB, mA, mB, F_{}, F_{}, T_{});
+    step(u, sA, sB, mA, mB, F_{}, F_{});
+  }
+
+  if constexpr (KS == 2) {
+    // ---- merge: part 1 hands its output, reference and row sum to part 0 of the same queries
+    // through the K and V slots (16 bytes per lane and plane), part 0 stores
+    if (n < stages) __syncthreads();  // the other part's last step
+    __syncthreads();                  // every wave is done with the slots
+    float4* X = reinterpret_cast<float4*>(ks);
+    float* R = reinterpret_cast<float*>(vts);
+    if (kg == 1) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            X[(((wq * QT + qt) * DT + dt) * 4 + g) * 64 + lane] =
+                make_float4(o[qt][dt][4 * g], o[qt][dt][4 * g + 1], o[qt][dt][4 * g + 2], o[qt][dt][4 * g + 3]);
+        R[(wq * QT + qt) * 128 + lane] = fresh[qt] ? -INFINITY : m_ref[qt];
+        R[(wq * QT + qt) * 128 + 64 + lane] = l_run[qt];
+      }
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const float m1 = R[(wq * QT + qt) * 128 + lane], l1 = R[(wq * QT + qt) * 128 + 64 + lane];
+      const float m0 = fresh[qt] ? -INFINITY : m_ref[qt], m = fmaxf(m0, m1);
+      const float s0 = __builtin_amdgcn_exp2f(m0 - m), s1 = __builtin_amdgcn_exp2f(m1 - m);
+      l_run[qt] = l_run[qt] * s0 + l1 * s1;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 x = X[(((wq * QT + qt) * DT + dt) * 4 + g) * 64 + lane];
+          o[qt][dt][4 * g + 0] = o[qt][dt][4 * g + 0] * s0 + x.x * s1;
+          o[qt][dt][4 * g + 1] = o[qt][dt][4 * g + 1] * s0 + x.y * s1;
+          o[qt][dt][4 * g + 2] = o[qt][dt][4 * g + 2] * s0 + x.z * s1;
+          o[qt][dt][4 * g + 3] = o[qt][dt][4 * g + 3] * s0 + x.w * s1;
+        }
+    }
   }
 
   // ---- normalise and store: o[qt][dt][r] = O[query lq][dim dt*32 + 8(r/4) + 4hi + r%4]
@@ -1124,13 +1182,13 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
   }
 }
 
-template <int D, int QT, int NW, int STAGES = 3, int SUPER = 1>
+template <int D, int NW, int KS>
 void launch_flash(FlashArgs fa, hipStream_t s) {
-  constexpr int BQ = NW * QT * 32;
+  constexpr int BQ = NW / KS * 32;
   fa.qblocks = (fa.Lq + BQ - 1) / BQ;
   const int blocks = fa.qblocks * fa.pairs;
   fa.xcd_order = (fa.pairs % 8 == 0) ? 1 : 0;
-  flash_kernel<D, QT, NW, STAGES, SUPER><<<blocks, NW * 64, 0, s>>>(fa);
+  flash_kernel<D, 1, NW, KS><<<blocks, NW * 64, 0, s>>>(fa);
 }
 
 // The wide kernel where its grid of 512-query blocks covers every CU of the chip (D = 96: its
@@ -1148,9 +1206,19 @@ void launch_flash_auto(FlashArgs fa, hipStream_t s) {
     fa.qblocks = (fa.Lq + kWideQueries - 1) / kWideQueries;
     fa.xcd_order = (fa.pairs % 8 == 0) ? 1 : 0;
     flash_wide_kernel<96><<<wide_blocks, 512, 0, s>>>(fa);
-  } else {
-    launch_flash<D, 1, 8>(fa, s);
+    return;
   }
+  // Two key parts where the blocks still fit the chip once: 64-query blocks of four waves, else
+  // 128-query blocks of eight; a second round would cost what the halved chain gains. us with one part ->
+  // two (pack included): 16 heads x 144 queries 14.9 -> 12.8, 300 21.3 -> 15.2, 1024 38.1 -> 27.8 (64-query), 1200
+  // 39.6 -> 30.6, 2048 59.2 -> 48.2 (128-query); 2100 queries would go 61.2 -> 75.2.
+  if constexpr (D <= 96) {
+    if (fa.Lk > KB) {
+      if ((long long)((fa.Lq + 63) / 64) * fa.pairs <= kChipCUs) return launch_flash<D, 4, 2>(fa, s);
+      if ((long long)((fa.Lq + 127) / 128) * fa.pairs <= kChipCUs) return launch_flash<D, 8, 2>(fa, s);
+    }
+  }
+  launch_flash<D, 8, 1>(fa, s);
 }
 
 template <int D>

@@ -1,4 +1,5 @@
-"""The flash kernels' softmax state: references that must agree between the two lanes of a query.
+"""The flash kernels' softmax state: two key parts per block (small grids) against one, at the edges of
+tiles, parts and query blocks, and references that must agree between the two lanes of a query.
 
 The reference is the same attention in float64 on the fp32 inputs. q, k, v and P are rounded to fp16
 (2^-11 each): a score is off by about |q||k| 2^-11 / sqrt(D), which stays below 2^-9 for unit inputs,
@@ -40,8 +41,8 @@ def check(got, ref, what):
     assert torch.isfinite(got).all() and rel <= 2.0**-8, what
 
 
-# (batch, heads, queries): the 256-query and the 512-query kernel
-ROUTES = {"256 queries": (2, 120, 129), "512 queries": (2, 128, 65)}
+# (batch, heads, queries): 64-query blocks in two parts, 128-query blocks in two parts, one part, wide
+ROUTES = {"parts, 64 queries": (1, 4, 65), "parts, 128 queries": (2, 64, 129), "one part": (2, 120, 129), "wide": (2, 128, 65)}
 
 
 @pytest.mark.parametrize("route", ROUTES)
@@ -60,3 +61,32 @@ def test_half_of_a_tile_vanishes(ns2lib, route, D):
         k = (score / math.sqrt(D))[None, :, None, None].expand(B, Lk, H, D).contiguous()
         check(run(ns2lib, q, k, v), reference(q, k, v, None, 0), f"{route} D={D} lane bit {lane}")
 
+
+@pytest.mark.parametrize("D", [32, 64, 96])
+@pytest.mark.parametrize("Lq,Lk,start", [(1, 65, None), (63, 128, None), (64, 129, 65), (65, 129, 64), (33, 192, 100),
+                                         (200, 193, 128), (17, 256, 255), (129, 257, 70), (64, 64, 10), (5, 449, 66)])
+def test_key_parts(ns2lib, Lq, Lk, start, D):
+    """Tiles that split evenly or not between the parts, and biases from the first key of a part on:
+    text weights, keys masked by -inf and by the lowest fp32 value."""
+    B, H = 2, 3
+    g = torch.Generator(device=DEV).manual_seed(Lq + Lk + D)
+    q, k, v = (torch.randn(B, L, H, D, generator=g, device=DEV) for L in (Lq, Lk, Lk))
+    bias = None
+    if start is not None:
+        bias = torch.rand(B, Lk - start, generator=g, device=DEV).log()
+        bias[0, ::2] = -math.inf
+        bias[1, 1::3] = torch.finfo(torch.float32).min
+    check(run(ns2lib, q, k, v, bias, start or 0), reference(q, k, v, bias, start or 0), f"{Lq}x{Lk} from {start} D={D}")
+
+
+def test_key_parts_large_scores(ns2lib):
+    """Scores far from 0 in both directions and different in each part (the merge weighs the parts)."""
+    B, H, D, Lq, Lk = 1, 2, 96, 70, 330
+    g = torch.Generator(device=DEV).manual_seed(1)
+    v = torch.randn(B, Lk, H, D, generator=g, device=DEV)
+    q = torch.ones(B, Lq, H, D, device=DEV)
+    tile = torch.arange(Lk, device=DEV) // 64
+    for even, odd in ((-300.0, -299.0), (250.0, 248.5), (-300.0, 200.0), (90.0, -90.0)):
+        score = torch.where(tile % 2 == 0, even, odd) + (torch.arange(Lk, device=DEV) % 5) * 0.25
+        k = (score / math.sqrt(D)).half().float()[None, :, None, None].expand(B, Lk, H, D).contiguous()
+        check(run(ns2lib, q, k, v), reference(q, k, v, None, 0), f"scores {even} / {odd}")
