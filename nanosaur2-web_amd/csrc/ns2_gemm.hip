@@ -317,13 +317,17 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm_kernel(GemmArgs p, int
   const int N = p.N, tid = threadIdx.x;
   const long long mn = (long long)p.M * N, row = (long long)blockIdx.x * N;
   int col[C];
-  float acc[C], xv[C];
+  float acc[C], xv[C], wa[C], wo[C];
+  const bool out = rn.y || rn.yt;
 #pragma unroll
   for (int j = 0; j < C; ++j) {
     const int n = tid + 256 * j;
     col[j] = n < N ? n : N - 1;
     acc[j] = 0.f;
     xv[j] = rn.x[row + col[j]];
+    // the norm weights with the first loads: behind the reductions each would be a round trip more
+    wa[j] = rn.w_add[col[j]];
+    wo[j] = out ? rn.w_out[col[j]] : 0.f;
   }
   for (int z0 = 0; z0 < splits; z0 += ZB) {
     float v[ZB][C];
@@ -353,19 +357,19 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm_kernel(GemmArgs p, int
   float sx = 0.f;
 #pragma unroll
   for (int j = 0; j < C; ++j) {
-    const float v = xv[j] + t[j] * r1 * rn.w_add[col[j]];
+    const float v = xv[j] + t[j] * r1 * wa[j];
     t[j] = v;
     if (tid + 256 * j < N) {
       rn.x[row + col[j]] = v;
       sx += v * v;
     }
   }
-  if (!rn.y && !rn.yt) return;
+  if (!out) return;
   const float r2 = rsqrtf(block_sum(sx, red) / (float)N + rn.eps);
 #pragma unroll
   for (int j = 0; j < C; ++j)
     if (tid + 256 * j < N) {
-      float v = t[j] * r2 * rn.w_out[col[j]];
+      float v = t[j] * r2 * wo[j];
       if (rn.yt) {
         asm volatile("" : "+v"(v));  // the fp32 value, then one rounding (no fused conversion)
         reinterpret_cast<half_t*>(rn.yt)[tiled_off(blockIdx.x, col[j], N)] = (half_t)v;
