@@ -8,6 +8,8 @@
 // loader. The per-row int8 scale is applied in the epilogue, in the reference's order
 // (app/gpu/gemm.js:159-164). Small M (GEMV-like, e.g. the adaLN projections of one
 // conditioning vector) runs on a fp32-FMA kernel that streams the weights once.
+#include <type_traits>
+
 #include "ns2_common.h"
 
 using namespace ns2dev;
@@ -631,6 +633,329 @@ __global__ __launch_bounds__(512) void splitk_glu_down_kernel(GemmArgs p, int sp
   }
 }
 
+// ---- short sequences: a tiled fp16 linear and its row kernel in one launch --------------------
+//
+// A block owns 16 RT rows and the output columns its row operation needs (a whole head, or 128 GLU
+// columns with both halves), so nothing but the result leaves the chip: the split-K sums' round trip
+// through memory and a second launch were half the time of these calls. What bounds them is one
+// latency and the weight bytes through one CU, which takes 64 bytes per clock from L2 and about 25
+// from memory (one CU's misses in flight cover 100 KB). So every wave has the weight fragments of
+// two chunks of k-tiles in flight as 16-byte register loads (the tiled layout gives a fragment of
+// v_mfma_f32_16x16x32_f16 as four 256-byte runs) while the rows are placed in LDS in fragment order, one
+// 1 KB plane per 16 rows and 32 columns of K; the blocks of one weight slice run on one XCD
+// (few_rows_tile) and start at different k-steps, so that each brings another part of the slice into
+// their L2; and calls of few row tiles launch blocks without rows that only fetch (kFewRowsTiles).
+// us per encoder pass of 17 layers with weights from memory, 256 / 37 tokens: two launches each 915 / 734,
+// one launch 836 / 761, with the turned starts 785 / 722, with the fetching blocks 784 / 700. With
+// 4-byte loads that touch the down weights' lines at the start 841 / 771.
+constexpr int kFewRowsTiles = 8;  // row tiles launched at least
+
+inline __host__ __device__ int few_rows_tiles(int M, int rt) {
+  const int t = (M + 16 * rt - 1) / (16 * rt);
+  return t < kFewRowsTiles ? kFewRowsTiles : t;
+}
+
+// Block id -> (row tile, column group): XCD x = id % 8 owns a contiguous range of the groups' row tiles.
+__device__ __forceinline__ void few_rows_tile(int row_tiles, int groups, int& rt, int& cg) {
+  const int tiles = row_tiles * groups, x = blockIdx.x % 8, q = tiles / 8, r = tiles % 8;
+  const int t = x * q + (x < r ? x : r) + blockIdx.x / 8;
+  rt = t % row_tiles;
+  cg = t / row_tiles;
+}
+
+// acc[r][c] = rows 16 (RT rt + r) .. +15 of At [M][K] times weight rows n[c] .. n[c]+15 of Wt (both tiled
+// fp16), K in chunks of CH 64-wide k-tiles (K % (64 CH) == 0), from k-step K / 32 * rt / row_tiles round to the
+// one before it; acc[r][c][i]: row 4 (lane / 16) + i of the tile, column n[c] + lane % 16. frags: RT K / 32 KB of
+// LDS. Every wave of the block calls it (one barrier). loads_out() is called behind the first two
+// chunks' loads, before_last() where the loads of the last chunk have gone out and one chunk's
+// registers are free. Row tiles past M take row tile 0's rows (their results are dropped).
+template <int RT, int CH, class L, class F>
+__device__ __forceinline__ void few_rows_product(const half_t* At, const half_t* Wt, int M, int K, int rt, int row_tiles,
+                                                 const int (&n)[2], float4_t (&acc)[RT][2], char* frags, L loads_out,
+                                                 F before_last) {
+  constexpr int S = 2 * CH;  // 32-wide steps per chunk
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int l16 = lane & 15, grp = lane >> 4;
+  const int steps = K / 32, chunks = steps / S, start = steps * rt / row_tiles;
+  auto turn = [&](int s) { return s + start < steps ? s + start : s + start - steps; };
+  // step s of a row or weight row r: tiled_off(r, 8 grp, K) + 2048 s
+  const half_t* ap[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int m0 = 16 * (RT * rt + r);
+    ap[r] = At + tiled_off((m0 < M ? m0 : 0) + l16, 8 * grp, K);
+  }
+  const half_t* wp[2] = {Wt + tiled_off(n[0] + l16, 8 * grp, K), Wt + tiled_off(n[1] + l16, 8 * grp, K)};
+  half8_t b0[2][S], b1[2][S];
+  auto load = [&](half8_t (&b)[2][S], int c) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) b[t][s] = *reinterpret_cast<const half8_t*>(wp[t] + (long long)turn(c * S + s) * 2048);
+  };
+  auto products = [&](const half8_t (&b)[2][S], int c) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const half8_t a = *reinterpret_cast<const half8_t*>(frags + (turn(c * S + s) * RT + r) * 1024 + lane * 16);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[t][s], acc[r][t], 0, 0, 0);
+      }
+  };
+  // the rows first (they arrive first), up to AP planes per wave and row tile in flight
+  constexpr int AP = RT == 1 ? 4 : 3;
+  half8_t a[AP][RT];
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int s = wave + i * waves;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) a[i][r] = *reinterpret_cast<const half8_t*>(ap[r] + (long long)(s < steps ? s : 0) * 2048);
+  }
+  load(b0, 0);
+  if (chunks > 1) load(b1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  loads_out();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int s = wave + i * waves;
+    if (s < steps)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) *reinterpret_cast<half8_t*>(frags + (s * RT + r) * 1024 + lane * 16) = a[i][r];
+  }
+  for (int s = wave + AP * waves; s < steps; s += waves)
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      *reinterpret_cast<half8_t*>(frags + (s * RT + r) * 1024 + lane * 16) =
+          *reinterpret_cast<const half8_t*>(ap[r] + (long long)s * 2048);
+  // LDS writes done, then the barrier; the weight loads stay in flight
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) acc[r][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+  int c = 0;
+  for (; c + 2 < chunks; c += 2) {
+    products(b0, c);
+    load(b0, c + 2);
+    products(b1, c + 1);
+    if (c + 3 < chunks) load(b1, c + 3);
+  }
+  products(b0, c);
+  before_last();
+  if (c + 1 < chunks) products(b1, c + 1);
+}
+
+// The q|k|v linear with its head norms, RoPE and fp16 keys and values (splitk_head_norm_kernel's
+// arithmetic on unsplit sums): block (16 RT rows, head), wave w of D/32 has columns 16w .. 16w+15 and their
+// RoPE partners D/2 + 16w .. of the head. 96 blocks at 256 rows x 6 heads.
+template <int D, int RT, int CH>
+__global__ __launch_bounds__(2 * D) void few_rows_head_norm_kernel(const half_t* __restrict__ At, const half_t* __restrict__ Wt, GemmArgs p,
+                                                                   HeadNorm hn) {
+  constexpr int NW = D / 32;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ float red[NW][16 * RT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, grp = lane >> 4;
+  const int row_tiles = few_rows_tiles(p.M, RT);
+  int rt, h;
+  few_rows_tile(row_tiles, p.N / D, rt, h);
+  const int m0 = rt * 16 * RT + 4 * grp, c0 = 16 * wave + l16;  // the lane's first row; its first column within the head
+  const bool normed = h < hn.H1 + hn.H2;                        // uniform
+  float bi[2] = {0.f, 0.f}, w[2] = {1.f, 1.f};
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (p.bias) bi[t] = p.bias[h * D + c0 + t * (D / 2)];
+    if (normed) w[t] = (h < hn.H1 ? hn.w1 : hn.w2)[c0 + t * (D / 2)];
+  }
+  float cs[RT][4], sn[RT][4];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + 16 * r + i;
+      const bool rope = normed && hn.cs && m < hn.rope_rows && m < p.M;
+      const long long at = rope ? (long long)m * (D / 2) + c0 : 0;
+      cs[r][i] = rope ? hn.cs[at] : 1.f;
+      sn[r][i] = rope ? hn.cs[hn.sin_off + at] : 0.f;
+    }
+  float4_t acc[RT][2];
+  const int n[2] = {h * D + 16 * wave, h * D + D / 2 + 16 * wave};
+  few_rows_product<RT, CH>(At, Wt, p.M, p.K, rt, row_tiles, n, acc, smem, [] {}, [] {});
+  float v[RT][2][4];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[r][t][i] = acc[r][t][i] * p.alpha + bi[t];
+  if (normed) {
+    // sums of squares of the rows: the 16 lanes of a row group, then the waves in order
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float q = v[r][0][i] * v[r][0][i] + v[r][1][i] * v[r][1][i];
+        q += dpp<kDppXor1>(q);
+        q += dpp<kDppXor2>(q);
+        q += dpp<kDppHalfMirror>(q);
+        q += dpp<kDppRowMirror>(q);
+        if (l16 == 0) red[wave][16 * r + 4 * grp + i] = q;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float q = 0.f;
+#pragma unroll
+        for (int u = 0; u < NW; ++u) q += red[u][16 * r + 4 * grp + i];
+        const float rs = rsqrtf(q / (float)D + hn.eps);
+        const float a = v[r][0][i] * rs * w[0], b = v[r][1][i] * rs * w[1];
+        const bool rope = hn.cs && m0 + 16 * r + i < hn.rope_rows;
+        v[r][0][i] = rope ? a * cs[r][i] - b * sn[r][i] : a;
+        v[r][1][i] = rope ? b * cs[r][i] + a * sn[r][i] : b;
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 16 * r + i, c = c0 + t * (D / 2);
+        if (m >= p.M) continue;
+        float x = v[r][t][i];
+        if (hn.kv16 && h >= hn.H1) {  // uniform
+          // the fp32 value as the fp32 store would hold it (no multiply-add fused with the conversion)
+          asm volatile("" : "+v"(x));
+          hn.kv16[m * hn.ldkv + (long long)(h - hn.H1) * D + c] = (half_t)x;
+        } else {
+          p.C[p.cOff + (long long)m * p.ldc + h * D + c] = x;
+        }
+      }
+}
+
+// The gate/up linear, its GLU and the GLU group's share of the down projection (the arithmetic of
+// splitk_glu_down_kernel on unsplit sums): block (16 RT rows, group of GS GLU columns), wave w of 8 has gate
+// and up columns 16w .. 16w+15 of the group, then column tiles w, w + 8, ... of the down product, whose
+// weight fragments go out behind the gate/up loads and the products before the last chunk. 256 blocks
+// at 256 rows x 2048 GLU columns.
+template <int GS, int RT, int CH>
+__global__ __launch_bounds__(GS * 4) void few_rows_glu_down_kernel(const half_t* __restrict__ At, const half_t* __restrict__ Wt, GemmArgs p,
+                                                                   GluDown gd) {
+  // waves, 32-wide steps of the down product, its tiles per round trip, those that go out at the start
+  constexpr int NW = GS / 16, DS = GS / 32, JC = 5, JE = RT == 1 ? 3 : 1;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ __attribute__((aligned(16))) half_t g16[RT * 16 * GS];  // the GLU output in fragment order
+  const int I = p.N / 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, grp = lane >> 4;
+  const int row_tiles = few_rows_tiles(p.M, RT);
+  int rt, cg;
+  few_rows_tile(row_tiles, I / GS, rt, cg);
+  const int j0 = cg * GS, j = j0 + 16 * wave + l16, nt = gd.Nd / 16;
+  const float bg = p.bias ? p.bias[j] : 0.f, bu = p.bias ? p.bias[j + I] : 0.f;
+  half8_t bf[JC][DS];
+  auto load_w = [&](int jt0, auto lo, auto hi) {
+#pragma unroll
+    for (int c = lo.value; c < hi.value; ++c) {
+      const int jt = jt0 + c * NW < nt ? jt0 + c * NW : nt - 1;
+      const half_t* wrow = gd.wd + tiled_off(16 * jt + l16, j0 + 8 * grp, I);
+#pragma unroll
+      for (int s = 0; s < DS; ++s) bf[c][s] = *reinterpret_cast<const half8_t*>(wrow + 2048 * s);
+    }
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using CE = std::integral_constant<int, JE>;
+  using CJ = std::integral_constant<int, JC>;
+  float4_t acc[RT][2];
+  const int n[2] = {j0 + 16 * wave, I + j0 + 16 * wave};
+  few_rows_product<RT, CH>(At, Wt, p.M, p.K, rt, row_tiles, n, acc, smem, [&] { load_w(wave, C0{}, CE{}); },
+                           [&] { load_w(wave, CE{}, CJ{}); });
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float y = apply_act(acc[r][0][i] * p.alpha + bg, gd.act) * (acc[r][1][i] * p.alpha + bu);
+      // the fp32 value first, as the GLU kernel stores it: no multiply fused into the conversion
+      asm volatile("" : "+v"(y));
+      // row 4 grp + i, column c = 16 wave + l16: plane c / 32, lane 16 (c % 32 / 8) + row, element c % 8
+      const int c = 16 * wave + l16;
+      g16[(c / 32 * RT + r) * 512 + ((c % 32 / 8) * 16 + 4 * grp + i) * 8 + c % 8] = (half_t)y;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  half8_t af[RT][DS];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int s = 0; s < DS; ++s) af[r][s] = *reinterpret_cast<const half8_t*>(&g16[(s * RT + r) * 512 + lane * 8]);
+  for (int jt0 = wave; jt0 < nt; jt0 += JC * NW) {
+    if (jt0 != wave) load_w(jt0, C0{}, CJ{});
+#pragma unroll
+    for (int c = 0; c < JC; ++c) {
+      const int jt = jt0 + c * NW;
+      if (jt >= nt) continue;  // uniform per wave
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        float4_t d = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < DS; ++s) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[r][s], bf[c][s], d, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 16 * (RT * rt + r) + 4 * grp + i;
+          if (m < p.M) gd.out[((long long)cg * p.M + m) * gd.Nd + 16 * jt + l16] = d[i];
+        }
+      }
+    }
+  }
+}
+
+// Rows up to which the one-launch kernels take a call, 16 rows per block up to one block per CU of the
+// GLU kernel at the encoder's width, then 32. us per pass with two launches -> one: 256 tokens 913 ->
+// 726, 512 1135 -> 919, 600 1342 -> 1145, 1000 1680 -> 1380 (the norm kernels' weights included).
+constexpr int kFewRows = 1024, kFewRows16 = 256;
+constexpr int kFewRowsPlanes = 60 * 1024;  // LDS bytes of the rows' planes: with the GLU output 64 KB in all
+inline bool few_rows(int M, int K) {
+  return M <= kFewRows && K % 64 == 0 && (M <= kFewRows16 ? 1 : 2) * (long long)K * 32 <= kFewRowsPlanes;
+}
+
+// Whether an output of the call overlaps its tiled rows: one launch would overwrite rows that other
+// blocks still read, so such a call keeps the two launches, of which only the second stores.
+inline bool overlaps(const void* out, size_t out_bytes, const uint16_t* At, int M, int K) {
+  const uintptr_t o = (uintptr_t)out, a = (uintptr_t)At;
+  return o < a + ((size_t)M + 63) / 64 * 64 * K * 2 && a < o + out_bytes;
+}
+
+// f(RT, CH) with the row tiles per block and the chunk of a call
+template <class F>
+void few_rows_dispatch(int M, int K, F f) {
+  using std::integral_constant;
+  if (M <= kFewRows16) {
+    if (K % 320 == 0) f(integral_constant<int, 1>{}, integral_constant<int, 5>{});
+    else f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  } else {
+    if (K % 320 == 0) f(integral_constant<int, 2>{}, integral_constant<int, 5>{});
+    else f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  }
+}
+
+template <int D>
+void launch_few_rows_head_norm(const half_t* At, const half_t* Wt, const GemmArgs& p, const HeadNorm& hn, hipStream_t s) {
+  few_rows_dispatch(p.M, p.K, [&](auto rt, auto ch) {
+    constexpr int RT = decltype(rt)::value, CH = decltype(ch)::value;
+    const int blocks = few_rows_tiles(p.M, RT) * (p.N / D);
+    few_rows_head_norm_kernel<D, RT, CH><<<blocks, 2 * D, RT * p.K * 32, s>>>(At, Wt, p, hn);
+  });
+}
+
+void launch_few_rows_glu_down(const half_t* At, const half_t* Wt, const GemmArgs& p, const GluDown& gd, hipStream_t s) {
+  few_rows_dispatch(p.M, p.K, [&](auto rt, auto ch) {
+    constexpr int RT = decltype(rt)::value, CH = decltype(ch)::value;
+    const int blocks = few_rows_tiles(p.M, RT) * (p.N / 2 / kGluDownGroup);
+    few_rows_glu_down_kernel<kGluDownGroup, RT, CH><<<blocks, 512, RT * p.K * 32, s>>>(At, Wt, p, gd);
+  });
+}
+
 // Small-M path: one wave per output column n, all M (<= MR <= 8) rows, fp32 FMA.
 // A: fp32 [M, lda] (bf16 layers) or rotated fp16 [M, lda] (int8 layers).
 template <bool W_BF16, int MR>
@@ -1022,6 +1347,13 @@ inline bool retile_i8(const GemmArgs& p) {
   return p.M >= kRetileRows && p.N > 0 && p.K >= kRetileK && (double)p.M * p.N * p.K >= kRetileWork && p.N % 64 == 0 && !p.add;
 }
 
+// The operands of a tiled fp16 linear, as the tiled kernel's entry points check them.
+int check_tiled_f16(const char* fn, const uint16_t* At, const uint16_t* Wt, int M, int N, int K) {
+  NS2_REQUIRE(At && Wt && M > 0 && N > 0 && N % 64 == 0 && K > 0 && K % 64 == 0 && aligned16(At) && aligned16(Wt),
+              "%s: At, Wt, M=%d, N=%d (N %% 64 == 0), K=%d (K %% 64 == 0) or alignment", fn, M, N, K);
+  return NS2_OK;
+}
+
 int check_common(const GemmArgs& p, const char* name) {
   NS2_REQUIRE(p.A && p.W && p.C, "%s: null A, W or C", name);
   NS2_REQUIRE(p.M >= 0 && p.N > 0 && p.K > 0, "%s: bad sizes M=%d N=%d K=%d", name, p.M, p.N, p.K);
@@ -1284,15 +1616,26 @@ int ns2_linear_f16w_tiled_head_norm_f16kv(const uint16_t* At, const uint16_t* Wt
               "%s: N=%d (at most %d heads of %d), H1=%d, H2=%d or their weights", fn, N, kHeadNormMaxHeads, D, H1,
               H2);
   NS2_REQUIRE(ldkv >= N - H1 * D, "%s: ldkv=%d is below the %d fp16 key/value columns", fn, ldkv, N - H1 * D);
+  const HeadNorm hn{w1, H1, w2, H2, D, cs, sin_off, cs ? rope_rows : 0, eps, reinterpret_cast<half_t*>(kv16), ldkv};
+  GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, C, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
+  hipStream_t s = ns2::stream();
+  if (few_rows(M, K) && !overlaps(C, (size_t)M * N * 4, At, M, K) && !overlaps(kv16, (size_t)M * ldkv * 2, At, M, K)) {
+    int rc = check_tiled_f16(fn, At, Wt, M, N, K);
+    if (rc) return rc;
+    const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);
+    ns2::ProfScope prof_("linear_head_norm_f16kv");
+    if (D == 64) launch_few_rows_head_norm<64>(a, w, q, hn, s);
+    else if (D == 128) launch_few_rows_head_norm<128>(a, w, q, hn, s);
+    else launch_few_rows_head_norm<256>(a, w, q, hn, s);
+    NS2_LAUNCHED("linear_head_norm_f16kv");
+    return NS2_OK;
+  }
   float* part = nullptr;
   int splits = 1;
   int rc = ns2::linear_f16w_tiled_raw(fn, At, Wt, M, N, K, &part, &splits);
   if (rc) return rc;
-  GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, C, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   q.part = part;
-  const HeadNorm hn{w1, H1, w2, H2, D, cs, sin_off, cs ? rope_rows : 0, eps, reinterpret_cast<half_t*>(kv16), ldkv};
   ns2::ProfScope prof_("head_norm_f16kv");
-  hipStream_t s = ns2::stream();
   if (D == 64) splitk_head_norm_kernel<64><<<M, 64, 0, s>>>(q, splits, hn);
   else if (D == 128) splitk_head_norm_kernel<128><<<M, 128, 0, s>>>(q, splits, hn);
   else splitk_head_norm_kernel<256><<<M, 256, 0, s>>>(q, splits, hn);
@@ -1311,13 +1654,22 @@ int ns2_linear_f16w_tiled_glu_down(const uint16_t* At, const uint16_t* Wt, const
               kGluDownGroup, Nd);
   NS2_REQUIRE(act >= NS2_ACT_NONE && act <= NS2_ACT_GELU_TANH, "%s: unknown act %d", fn, act);
   NS2_REQUIRE(aligned16(wd_tiled), "%s: wd_tiled must be 16-byte aligned", fn);
+  GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, part, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
+  const GluDown gd{reinterpret_cast<const half_t*>(wd_tiled), part, Nd, act, glu_down_ranges(M, N, Nd)};
+  if (few_rows(M, K) && !overlaps(part, (size_t)(N / 2 / kGluDownGroup) * M * Nd * 4, At, M, K)) {
+    int rc = check_tiled_f16(fn, At, Wt, M, N, K);
+    if (rc) return rc;
+    const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);
+    ns2::ProfScope prof_("linear_glu_down");
+    launch_few_rows_glu_down(a, w, q, gd, ns2::stream());
+    NS2_LAUNCHED("linear_glu_down");
+    return NS2_OK;
+  }
   float* gu = nullptr;
   int splits = 1;
   int rc = ns2::linear_f16w_tiled_raw(fn, At, Wt, M, N, K, &gu, &splits);
   if (rc) return rc;
-  GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, part, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   q.part = gu;
-  const GluDown gd{reinterpret_cast<const half_t*>(wd_tiled), part, Nd, act, glu_down_ranges(M, N, Nd)};
   ns2::ProfScope prof_("glu_down");
   splitk_glu_down_kernel<kGluDownGroup>
       <<<dim3((M + 15) / 16, N / 2 / kGluDownGroup, gd.ncs), 512, 0, ns2::stream()>>>(q, splits, gd);
