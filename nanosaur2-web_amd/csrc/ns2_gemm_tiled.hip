@@ -358,7 +358,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
   constexpr int A_BYTES = BM * 64 * KT * 2, W_BYTES = BN * 64 * KT * WB;
   static_assert(BM % 64 == 0 && BN % 64 == 0 && WTM % 32 == 0 && WTN % 32 == 0, "tile shape");
   static_assert(NS % 2 == 0, "an even number of steps per k-tile");
-  static_assert(STAGES == 2 || STAGES == 3, "two or three LDS stages");
+  static_assert(STAGES == 2 || (STAGES == 3 && SPREAD == 1), "two or three LDS stages");
   static_assert(!WF16 || EPI == 0, "fp16 weights take the plain epilogue");
   __shared__ __attribute__((aligned(16))) char smem[STAGES * (A_BYTES + W_BYTES)];
   char* const as = smem;
@@ -880,21 +880,27 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
 // 1536/4096/6144, weights cycled through 8 copies); choosing by the model costs 1.1 % on average
 // against the best tile of each of those launches.
 //   64x64, 4 waves (2 k groups)   few tiles: each block's k chain halved, three 128-wide stages
-//   64x128, 8 waves (2 k groups)  at most two tiles per CU (1024 x 1536 x 1536 +=: 14.4 -> 11.5 us)
+//   64x128, 8 waves (2 k groups)  two tiles per CU (1900 x 1536 x 1536 +=: 17.9 us)
+//   the same, three stages        one tile per CU: with the block alone on its CU, one k-tile ahead does not
+//                                 cover a weight's way from memory (weights cycled through 600 MB, two ->
+//                                 three stages: 1024 x 1536 x 1536 +=: 14.3 -> 11.8 us, x 4096 29.8 -> 22.5, x 6144
+//                                 42.1 -> 32.4, 250 x 4608 x 1536 13.6 -> 11.3; six stages of the 64x64 tile
+//                                 or five of 128x192 gained nothing more)
 //   64x128, 4 waves               3 or 4 tiles per CU
 //   128x128, 4 waves              3 tiles per CU (1792 x 4608 x 1536: 35.4 -> 30.1 us)
 //   128x192, 4 waves              2 tiles per CU (2432 x 4608 x 1536: 47.2 -> 39.1 us)
 //   128x192, 8 waves (2 k groups) one tile per CU, long K (3952 x 1536 x 4096 +=: 62.2 -> 54.7 us)
 //   192x384, 8 waves              one tile per CU (3952 x 4608 x 1536: 70.3 -> 57.5 us)
 //   256x256, 8 waves              one tile per CU (3328 x 4608 x 1536: 51.9 -> 49.6 us)
-enum Tile { T64x64, T64x128K2, T64x128, T128x128, T128x192, T128x192K2, T192x384, T256x256, kTiles };
+enum Tile { T64x64, T64x128K2, T64x128K2S3, T64x128, T128x128, T128x192, T128x192K2, T192x384, T256x256, kTiles };
 struct TileCfg {
   int bm, bn, occ;
   float L, e[4], c[4];
 };
 constexpr TileCfg kCfgs[kTiles] = {
     {64, 64, 2, 1.8f, {1.86f, 2.65f}, {0.210f, 0.322f}},
-    {64, 128, 2, 1.5f, {2.40f, 4.34f}, {0.294f, 0.474f}},
+    {64, 128, 2, 1.5f, {2.56f, 4.34f}, {0.398f, 0.474f}},
+    {64, 128, 1, 1.5f, {3.20f}, {0.263f}},
     {64, 128, 4, 3.8f, {0.f, 1.49f, 3.17f, 0.f}, {0.413f, 0.510f, 0.731f, 1.147f}},
     {128, 128, 3, 2.9f, {2.49f, 5.20f, 0.f}, {0.513f, 0.790f, 1.550f}},
     {128, 192, 2, 0.9f, {5.77f, 0.f}, {0.696f, 1.497f}},
@@ -1005,6 +1011,7 @@ int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, 
   switch (tile) {
     case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, 0, false, true, true, true>(p, splits);
     case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4>(p);
+    case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 2, 3, 1, 2>(p);
     case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, 0, false, true, true, true>(p);
     case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, 0, false, false>(p);
     case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2>(p);

@@ -36,8 +36,11 @@ CASES = [
     ("64x64 split K", 65, 1536, 4096, True, 0),
     ("64x64 split K", 120, 1536, 6144, False, 32),
     ("64x64", 64, 64, 1536, True, 32),
-    ("64x128, two k groups", 1025, 1536, 1536, True, 0),
-    ("64x128, two k groups", 999, 1536, 1536, False, 32),
+    ("64x128, two k groups", 1501, 1536, 1536, True, 0),
+    ("64x128, two k groups", 1460, 1536, 1536, False, 32),
+    ("64x128, two k groups, three stages", 1025, 1536, 1536, True, 0),
+    ("64x128, two k groups, three stages", 999, 1536, 1536, False, 32),
+    ("64x128, two k groups, three stages", 1000, 1472, 1536, False, 0),
     ("64x128", 511, 4672, 1536, False, 0),
     ("64x128", 513, 4672, 1536, True, 32),
     ("128x128", 1537, 4672, 1536, False, 0),
