@@ -192,8 +192,9 @@ __global__ __launch_bounds__(256) void attn_pack_kernel(PackArgs a) {
   }
 }
 
-// One key row's share for four lanes (adjacent, within a quad): lane part q owns rope pairs
-// [q D/8, (q+1) D/8), i.e. dims q D/8 .. +D/8 of each half. Every load is issued first (the
+// One key row's share for four lanes (adjacent, within a quad): lane part q owns dims 16 i + 4q .. +3 of
+// each half, so that the four lanes' loads of 16 bytes are adjacent, and so are the 8-byte halves of the
+// chunks they store (x[4 i + e]: dim 16 i + 4q + e). Every load is issued first (the
 // row, the norm weights, the rope table): none depends on another, so their latencies overlap
 // instead of following the row's reduction.
 template <int D>
@@ -201,20 +202,20 @@ __device__ __forceinline__ void prep_quarter_row(const float* __restrict__ src, 
                                                  const float* __restrict__ cs, long long sinOff, int row,
                                                  bool rope, float eps, int q, float* x1, float* x2) {
   constexpr int HALF = D / 2, PER = D / 8;
-  const int i0 = q * PER;
+  const int i0 = 4 * q;
   float w1[PER], w2[PER], c[PER], sn[PER];
 #pragma unroll
   for (int j = 0; j < PER; j += 4) {
-    const float4 a = *reinterpret_cast<const float4*>(src + i0 + j);
-    const float4 b = *reinterpret_cast<const float4*>(src + HALF + i0 + j);
+    const float4 a = *reinterpret_cast<const float4*>(src + i0 + 4 * j);
+    const float4 b = *reinterpret_cast<const float4*>(src + HALF + i0 + 4 * j);
     x1[j] = a.x, x1[j + 1] = a.y, x1[j + 2] = a.z, x1[j + 3] = a.w;
     x2[j] = b.x, x2[j + 1] = b.y, x2[j + 2] = b.z, x2[j + 3] = b.w;
   }
   if (nw) {
 #pragma unroll
     for (int j = 0; j < PER; j += 4) {
-      const float4 a = *reinterpret_cast<const float4*>(nw + i0 + j);
-      const float4 b = *reinterpret_cast<const float4*>(nw + HALF + i0 + j);
+      const float4 a = *reinterpret_cast<const float4*>(nw + i0 + 4 * j);
+      const float4 b = *reinterpret_cast<const float4*>(nw + HALF + i0 + 4 * j);
       w1[j] = a.x, w1[j + 1] = a.y, w1[j + 2] = a.z, w1[j + 3] = a.w;
       w2[j] = b.x, w2[j + 1] = b.y, w2[j + 2] = b.z, w2[j + 3] = b.w;
     }
@@ -224,8 +225,8 @@ __device__ __forceinline__ void prep_quarter_row(const float* __restrict__ src, 
     const float* sp = cs + sinOff + (long long)row * HALF + i0;
 #pragma unroll
     for (int j = 0; j < PER; j += 4) {
-      const float4 a = *reinterpret_cast<const float4*>(cp + j);
-      const float4 b = *reinterpret_cast<const float4*>(sp + j);
+      const float4 a = *reinterpret_cast<const float4*>(cp + 4 * j);
+      const float4 b = *reinterpret_cast<const float4*>(sp + 4 * j);
       c[j] = a.x, c[j + 1] = a.y, c[j + 2] = a.z, c[j + 3] = a.w;
       sn[j] = b.x, sn[j + 1] = b.y, sn[j + 2] = b.z, sn[j + 3] = b.w;
     }
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(256) void attn_pack_vec_kernel(PackArgs a) {
     half_t* kdst = a.Kc + ((long long)bh * tiles + tile) * (KB * D) + rl * 8;
 #pragma unroll
     for (int j = 0; j < PER; j += 4) {
-      const int d1 = q * PER + j, d2 = HALF + d1;
+      const int d1 = 4 * q + 4 * j, d2 = HALF + d1;
       *reinterpret_cast<uint2*>(kdst + (d1 / 8) * (KB * 8) + d1 % 8) =
           make_uint2(pack_half2(x1[j], x1[j + 1]), pack_half2(x1[j + 2], x1[j + 3]));
       *reinterpret_cast<uint2*>(kdst + (d2 / 8) * (KB * 8) + d2 % 8) =
