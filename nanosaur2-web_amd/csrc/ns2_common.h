@@ -36,12 +36,13 @@ int lora_prepare(const float** t, const uint16_t* lora_a, const uint16_t* lora_b
 int linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_t* Wt, int M, int N, int K, float** part,
                           int* splits);
 // The int8 ConvRot linear on a file-layout weight W [N][K] through the tiled kernel: W is re-tiled
-// into library scratch (slot 7) by each call, and so is a row-major fp16 input x16 [M][ldx] into
+// into Wt (library scratch) by each call, and so is a row-major fp16 input x16 [M][ldx] into
 // At. At: the rotated input as the tiled fp16 operand, already filled where x16 is null.
 // Returns a status code.
-int linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, const float* scale, const float* bias, float* C, int M,
-                      int N, int K, int ldc, long long cOff, float alpha, int act, int resid, const float* gate,
-                      long long gOff, const uint16_t* lora_a, const uint16_t* lora_b, int lora_r);
+int linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, int8_t* Wt, const float* scale,
+                      const float* bias, float* C, int M, int N, int K, int ldc, long long cOff, float alpha, int act,
+                      int resid, const float* gate, long long gOff, const uint16_t* lora_a, const uint16_t* lora_b,
+                      int lora_r);
 
 // Kernel profiler (ns2_profile_*): when enabled, stream events bracket every launch and are
 // aggregated by kernel name on ns2_profile_report.

@@ -914,7 +914,7 @@ __global__ __launch_bounds__(GS * 4) void few_rows_glu_down_kernel(const half_t*
 // GLU kernel at the encoder's width, then 32. us per pass with two launches -> one: 256 tokens 913 ->
 // 726, 512 1135 -> 919, 600 1342 -> 1145, 1000 1680 -> 1380 (the norm kernels' weights included).
 constexpr int kFewRows = 1024, kFewRows16 = 256;
-constexpr int kFewRowsPlanes = 60 * 1024;  // LDS bytes of the rows' planes: with the GLU output 64 KB in all
+constexpr int kFewRowsPlanes = 60 * 1024;  // LDS bytes of the rows' planes (the GLU output takes 4 KB per 16 rows more)
 inline bool few_rows(int M, int K) {
   return M <= kFewRows && K % 64 == 0 && (M <= kFewRows16 ? 1 : 2) * (long long)K * 32 <= kFewRowsPlanes;
 }
@@ -1429,19 +1429,19 @@ int ns2_linear_i8_lora(const void* A, int a_fmt, int lda, const int8_t* W, const
               "ns2_linear_i8: a_fmt must be 0 (fp32), 1 (rotated fp16) or 2 (rotated fp32)");
   NS2_REQUIRE(scale != nullptr, "ns2_linear_i8: null scale");
   NS2_REQUIRE(K % 256 == 0, "ns2_linear_i8: K=%d must be a multiple of 256 (ConvRot groups)", K);
-  const bool retile = retile_i8(p);
+  // without memory for the re-tiled operands the call keeps the row-major kernel
+  int8_t* Wt = retile_i8(p) ? static_cast<int8_t*>(ns2::workspace(7, (size_t)N * K)) : nullptr;
   if (a_fmt != 1) {
     // fp32 input: rotate (ops.linear without xr, app/gpu/ops.js:54) or just cast a
     // pre-rotated xr, into library scratch
     NS2_REQUIRE(A && lda >= K && lda % 4 == 0 && aligned16(A), "ns2_linear_i8: bad fp32 A / lda=%d", lda);
   }
-  uint16_t* xr = nullptr;
-  if (a_fmt != 1 || retile) {
-    const size_t rows = retile ? ((size_t)M + 63) / 64 * 64 : (size_t)M;
-    xr = static_cast<uint16_t*>(ns2::workspace(0, rows * K * sizeof(uint16_t)));
-    if (!xr) return ns2::set_error(NS2_ERR_OOM, "ns2_linear_i8: workspace allocation failed");
-  }
+  uint16_t* xr = Wt ? static_cast<uint16_t*>(ns2::workspace(0, ((size_t)M + 63) / 64 * 64 * K * sizeof(uint16_t))) : nullptr;
+  const bool retile = xr != nullptr;
+  if (!retile && retile_i8(p)) (void)hipGetLastError();  // the failed allocation's
   if (a_fmt != 1) {
+    if (!retile) xr = static_cast<uint16_t*>(ns2::workspace(0, (size_t)M * K * sizeof(uint16_t)));
+    if (!xr) return ns2::set_error(NS2_ERR_OOM, "ns2_linear_i8: workspace allocation failed");
     if (a_fmt == 0) {
       int rc = ns2_rotate_f16(static_cast<const float*>(A), lda, xr, K, M, K, retile);
       if (rc) return rc;
@@ -1460,8 +1460,8 @@ int ns2_linear_i8_lora(const void* A, int a_fmt, int lda, const int8_t* W, const
   int rc = check_common(p, "ns2_linear_i8");
   if (rc) return rc;
   if (retile)
-    return ns2::linear_i8_retiled(xr, a_fmt == 1 ? static_cast<const uint16_t*>(A) : nullptr, lda, W, scale, bias, C, M,
-                                  N, K, ldc, cOff, alpha, act, resid, gate, gOff, lora_a, lora_b, lora_r);
+    return ns2::linear_i8_retiled(xr, a_fmt == 1 ? static_cast<const uint16_t*>(A) : nullptr, lda, W, Wt, scale, bias, C,
+                                  M, N, K, ldc, cOff, alpha, act, resid, gate, gOff, lora_a, lora_b, lora_r);
   if (lora_r) {
     // the LoRA down-projections take the rotated input (rotated A for int8 weights)
     rc = ns2::lora_prepare(&p.lt, lora_a, lora_b, lora_r, p.A, 1, p.lda, M, K, "ns2_linear_i8_lora");

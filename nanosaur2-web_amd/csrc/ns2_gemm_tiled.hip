@@ -1023,18 +1023,16 @@ int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, 
 
 }  // namespace
 
-int ns2::linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, const float* scale,
-                           const float* bias, float* C, int M, int N, int K, int ldc, long long cOff, float alpha,
-                           int act, int resid, const float* gate, long long gOff, const uint16_t* lora_a,
-                           const uint16_t* lora_b, int lora_r) {
+int ns2::linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, int8_t* Wt,
+                           const float* scale, const float* bias, float* C, int M, int N, int K, int ldc,
+                           long long cOff, float alpha, int act, int resid, const float* gate, long long gOff,
+                           const uint16_t* lora_a, const uint16_t* lora_b, int lora_r) {
   if (x16) {
     const long long chunks = (long long)((M + 63) / 64) * 64 * K / 8;
     ns2::ProfScope prof_("tile_f16_rows");
     tile_x16_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, ns2::stream()>>>(x16, ldx, At, M, K);
     NS2_LAUNCHED("tile_f16_rows");
   }
-  int8_t* Wt = static_cast<int8_t*>(ns2::workspace(7, (size_t)N * K));
-  if (!Wt) return ns2::set_error(NS2_ERR_OOM, "ns2_linear_i8: weight workspace allocation failed");
   int rc = ns2_tile_i8_weight(W, Wt, N, K);
   if (rc) return rc;
   return linear_tiled("ns2_linear_i8", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate, gOff,
