@@ -1211,8 +1211,9 @@ void launch_flash_auto(FlashArgs fa, hipStream_t s) {
   }
   // Two key parts where the blocks still fit the chip once: 64-query blocks of four waves, else
   // 128-query blocks of eight; a second round would cost what the halved chain gains. us with one part ->
-  // two (pack included): 16 heads x 144 queries 14.9 -> 12.8, 300 21.3 -> 15.2, 1024 38.1 -> 27.8 (64-query), 1200
-  // 39.6 -> 30.6, 2048 59.2 -> 48.2 (128-query); 2100 queries would go 61.2 -> 75.2.
+  // two (pack included): 16 heads x 144 queries 14.9 -> 13.2, 300 21.3 -> 15.7, 1024 38.1 -> 28.3 (64-query), 1200
+  // 39.6 -> 29.7, 2048 59.2 -> 46.8 (128-query); 2100 queries would go 61.2 -> 75.2. D = 128 has no LDS
+  // for two parts' stages.
   if constexpr (D <= 96) {
     if (fa.Lk > KB) {
       if ((long long)((fa.Lq + 63) / 64) * fa.pairs <= kChipCUs) return launch_flash<D, 4, 2>(fa, s);
