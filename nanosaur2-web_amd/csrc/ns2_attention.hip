@@ -505,6 +505,11 @@ struct TileLoader {
 // score exceeds it by more than 2^kRebase; between moves the output accumulator needs no
 // rescale. Any reference gives the same softmax, and p <= 2^kRebase stays in fp16 range.
 constexpr float kRebase = 8.0f;
+// A tile whose maximum is more than this above the reference makes what came before it vanish (2^-256 is
+// 0 in fp32), and its scores, formed on top of -m_ref, have lost the bits that a reference far below them
+// takes: after a first tile masked with -1e9 the next tile's scores would be multiples of 128. Such a
+// tile is scored again from 0, as a query's first tile.
+constexpr float kRescore = 256.0f;
 
 // KS: key parts. The NW waves of a block are NW / KS query waves times KS key parts: a stage holds KS
 // consecutive tiles and part g works on tile u KS + g of stage u; the parts' outputs, references and
@@ -723,12 +728,32 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
       bool need = false;
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) need |= (mx_cur[qt] > kRebase) || fresh[qt];
-      if (__builtin_amdgcn_ballot_w64(need)) {
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) != 0, 0)) {
+        bool any_far = false, far[QT];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          far[qt] = (mx_cur[qt] > kRescore) && !fresh[qt];
+          any_far |= far[qt];
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_far) != 0, 0)) {
+          // K and the biases of tile t are in LDS until the end of the step
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) {
+            m_ref[qt] = far[qt] ? 0.f : m_ref[qt];
+            fresh[qt] |= far[qt];
+          }
+          set_minit();
+#pragma unroll
+          for (int i = 0; i < NK; ++i) qk_mfma(s_cur, i, read_k(i, vbuf));
+          if (u * KS + kg >= a.bias_block0) add_bias(s_cur, vbuf);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) mx_cur[qt] = col_max(fmaxf(half_max(s_cur, 0, qt), half_max(s_cur, 1, qt)));
+        }
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           const bool seen = mx_cur[qt] > -INFINITY;
           const float shift = fresh[qt] ? (seen ? mx_cur[qt] : 0.f) : fmaxf(mx_cur[qt], 0.f);
-          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift);
+          const float alpha = far[qt] ? 0.f : (fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift));
           fresh[qt] = fresh[qt] && !seen;
           m_ref[qt] += shift;
           l_run[qt] *= alpha;
@@ -1042,7 +1067,7 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
     }
     // ---- S^T = K Q^T - m_ref
     float16_t s[2][QT];
-    {
+    auto scores = [&]() {
       half8_t kf[2][2], qf[2][QT];
       kf[0][0] = read_k(0, 0, buf);
       kf[0][1] = read_k(0, 1, buf);
@@ -1066,38 +1091,59 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
                                                                0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    if constexpr (BIAS) {
+      if constexpr (BIAS) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const float4 bb = *reinterpret_cast<const float4*>(&kbias[buf][kt * 32 + 8 * g + 4 * hi]);
+          for (int g = 0; g < 4; ++g) {
+            const float4 bb = *reinterpret_cast<const float4*>(&kbias[buf][kt * 32 + 8 * g + 4 * hi]);
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt) {
-            s[kt][qt][4 * g + 0] += bb.x;
-            s[kt][qt][4 * g + 1] += bb.y;
-            s[kt][qt][4 * g + 2] += bb.z;
-            s[kt][qt][4 * g + 3] += bb.w;
+            for (int qt = 0; qt < QT; ++qt) {
+              s[kt][qt][4 * g + 0] += bb.x;
+              s[kt][qt][4 * g + 1] += bb.y;
+              s[kt][qt][4 * g + 2] += bb.z;
+              s[kt][qt][4 * g + 3] += bb.w;
+            }
           }
-        }
-    }
+      }
+    };
+    scores();
     // ---- the reference moves when a score exceeds it by more than 2^kRebase, or on the query's first
     // tile with a finite score (fresh: the reference becomes the tile maximum); as in flash_kernel,
     // the same in the query's two lanes
     {
       float mx[QT];
+      auto row_max = [&]() {
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) mx[qt] = col_max(__builtin_fmaxf(half_max(s[0][qt]), half_max(s[1][qt])));
+        for (int qt = 0; qt < QT; ++qt) mx[qt] = col_max(__builtin_fmaxf(half_max(s[0][qt]), half_max(s[1][qt])));
+      };
+      row_max();
       bool need = false;
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) need |= (mx[qt] > kRebase) || fresh[qt];
-      if (__builtin_amdgcn_ballot_w64(need)) {
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) != 0, 0)) {
+        bool any_far = false, far[QT];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          far[qt] = (mx[qt] > kRescore) && !fresh[qt];
+          any_far |= far[qt];
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_far) != 0, 0)) {
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) {
+            m_ref[qt] = far[qt] ? 0.f : m_ref[qt];
+            fresh[qt] |= far[qt];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) minit[qt][r] = -m_ref[qt];
+          }
+          scores();
+          row_max();
+        }
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           const bool seen = mx[qt] > -INFINITY;
           const float shift = fresh[qt] ? (seen ? mx[qt] : 0.f) : fmaxf(mx[qt], 0.f);
-          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift);
+          const float alpha = far[qt] ? 0.f : (fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift));
           fresh[qt] = fresh[qt] && !seen;
           m_ref[qt] += shift;
           l_run[qt] *= alpha;

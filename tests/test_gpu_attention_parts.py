@@ -90,3 +90,19 @@ def test_key_parts_large_scores(ns2lib):
         score = torch.where(tile % 2 == 0, even, odd) + (torch.arange(Lk, device=DEV) % 5) * 0.25
         k = (score / math.sqrt(D)).half().float()[None, :, None, None].expand(B, Lk, H, D).contiguous()
         check(run(ns2lib, q, k, v), reference(q, k, v, None, 0), f"scores {even} / {odd}")
+
+
+@pytest.mark.parametrize("route", ROUTES)
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("low", [-3000.0, -1e9, -1e30])
+def test_first_tiles_masked(ns2lib, route, D, low):
+    """A finite low mask over whole key tiles in front of the others: the reference taken from them must not
+    swallow the scores of the tiles behind (fp32 spacing at 1.4e9: 128)."""
+    B, H, Lq = ROUTES[route]
+    Lk = 300
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.randn(B, L, H, D, generator=g, device=DEV) for L in (Lq, Lk, Lk))
+    key = torch.arange(Lk, device=DEV)
+    for what, masked in (("first tile", key < 64), ("first two tiles", key < 128), ("even tiles", key // 64 % 2 == 0)):
+        bias = torch.where(masked, low, 0.0).expand(B, Lk).contiguous()
+        check(run(ns2lib, q, k, v, bias, 0), reference(q, k, v, bias, 0), f"{route} D={D} {what} masked by {low}")
