@@ -229,6 +229,36 @@ def test_glu_tiles(ns2lib, tile, M, N, K, rank):
     assert torch.isfinite(got).all() and rel <= (2.0**-10 if rank else 2.0**-11)
 
 
+@pytest.mark.parametrize("M", [100, 1100])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "none"])
+def test_glu_activation(ns2lib, M, act):
+    """The fused GLU launch computes the activation of the plain epilogue, bit for bit: small integers make
+    the products' fp32 sums exact in any order, act(h1) comes from the plain linear, and the modulation
+    producer (scale -1, the row as its shift) rotates act(h1) * h2 as the GLU epilogue does."""
+    print(f"[case] glu activation {M} {act}", flush=True)
+    I, K = 4096, 256
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randint(-8, 9, (M, K), generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (2 * I, K), generator=g, device=DEV, dtype=torch.int8)
+    s = torch.full((2 * I,), 2.0**-12, device=DEV)
+    wt, wg = torch.empty_like(q), torch.empty_like(q)
+    ns2lib.tile_i8_weight(q, wt, 2 * I, K)
+    ns2lib.tile_i8_weight_glu(q, wg, 2 * I, K)
+    a, h = torch.empty(M, I, device=DEV), torch.empty(M, 2 * I, device=DEV)
+    ns2lib.linear_i8_tiled(tiled(x), wt, s, a, M, I, K, act=act)  # the first I weight rows are the first tiles
+    ns2lib.linear_i8_tiled(tiled(x), wt, s, h, M, 2 * I, K)
+    out = torch.empty((M + 63) // 64, I // 64, 8, 64, 8, dtype=torch.float16, device=DEV)
+    ns2lib.linear_i8_glu_rot_tiled(tiled(x), wg, s, out, M, 2 * I, K, act=act)
+    got = out.permute(0, 3, 1, 2, 4).reshape(-1, I)[:M]
+    one, minus = torch.ones(I, device=DEV), torch.full((I,), -1.0, device=DEV)
+    ref = torch.empty(M, I, dtype=torch.float16, device=DEV)
+    for m in range(0, M, 7):
+        ns2lib.norm_mod_rotate_f16(one, torch.cat([a[m] * h[m, I:], minus]), 0, I, 1, I, one, ref[m])
+    torch.cuda.synchronize()
+    differ = (got[::7] != ref[::7]).sum().item()
+    assert differ == 0, f"{differ} values differ"
+
+
 # head dims and counts whose value columns start inside a wave's columns (3200 is no multiple of 96)
 @pytest.mark.parametrize("M,N,K,H,HD", [(3952, 4608, 512, 22, 64), (3328, 4608, 512, 16, 96), (2304, 4608, 512, 22, 64),
                                         (1536, 4608, 512, 16, 96), (48, 4608, 512, 22, 64)])
