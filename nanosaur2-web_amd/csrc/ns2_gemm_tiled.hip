@@ -358,10 +358,10 @@ void gemm_tiled_kernel(TGemmArgs p) {
   constexpr int WB = WF16 ? 2 : 1;   // bytes per weight element
   constexpr int A_BLOCKS = BM / 64 * 8 * KT, W_BLOCKS = BN / 64 * WCH * KT;  // 1 KB blocks per stage
   constexpr int BLOCKS = A_BLOCKS + W_BLOCKS;
-  constexpr int PER_WAVE = (BLOCKS + NW - 1) / NW;  // copies per wave and k-tile, at most
-  constexpr int FULL_WAVES = BLOCKS % NW ? BLOCKS % NW : NW;  // waves that issue that many; the others one less
+  constexpr int PER_WAVE = BLOCKS / NW;  // copies per wave and k-tile
   constexpr int A_BYTES = BM * 64 * KT * 2, W_BYTES = BN * 64 * KT * WB;
   static_assert(BM % 64 == 0 && BN % 64 == 0 && WTM % 32 == 0 && WTN % 32 == 0, "tile shape");
+  static_assert(BLOCKS % NW == 0, "copies must split evenly over the waves");
   static_assert(NS % 2 == 0, "an even number of steps per k-tile");
   static_assert(STAGES == 2 || (STAGES == 3 && SPREAD == 1), "two or three LDS stages");
   static_assert(!WF16 || EPI == 0, "fp16 weights take the plain epilogue");
@@ -415,14 +415,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
     }
   }
   auto dma_one = [&](int i, int kt, int st) {
-    if (i + 1 < PER_WAVE || FULL_WAVES == NW || wave < FULL_WAVES)
-      dma16(g_src[i] + (long long)kt * g_step[i] + lane * 16, __builtin_amdgcn_readfirstlane(l_dst[i] + st * l_step[i]));
-  };
-  // wait until at most this wave's copies of the n most recent tiles are in flight
-  auto wait_newer = [&](auto n_c) {
-    constexpr int N = decltype(n_c)::value;
-    if (FULL_WAVES == NW || wave < FULL_WAVES) vm_wait<N * PER_WAVE>();
-    else vm_wait<N * (PER_WAVE - 1)>();
+    dma16(g_src[i] + (long long)kt * g_step[i] + lane * 16, __builtin_amdgcn_readfirstlane(l_dst[i] + st * l_step[i]));
   };
 
   float16_t acc[TM][TN];
@@ -489,13 +482,8 @@ void gemm_tiled_kernel(TGemmArgs p) {
     }
   // tile 0 has landed; the copies of later tiles may be in flight
   constexpr int FIRST = [] { int n = 0; for (int i = 0; i < PER_WAVE; ++i) n += i * SLOTS / PER_WAVE < TN; return n; }();
-  if (kblocks >= STAGES) {
-    // the short waves' last copy is never in the first part unless SPREAD is 1
-    if (FULL_WAVES == NW || wave < FULL_WAVES) vm_wait<(STAGES - 2) * PER_WAVE + FIRST>();
-    else vm_wait<(STAGES - 2) * (PER_WAVE - 1) + (FIRST < PER_WAVE ? FIRST : PER_WAVE - 1)>();
-  } else {
-    vm_wait<0>();
-  }
+  if (kblocks >= STAGES) vm_wait<(STAGES - 2) * PER_WAVE + FIRST>();
+  else vm_wait<0>();
   __syncthreads();
   half8_t a[2][TM];
   WRaw w[2][TN];
@@ -514,7 +502,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
         // this wave's copies of tile kt+1 have landed once at most the later tiles' remain in
         // flight; the barrier then covers every wave's copies, and every wave's reads of tile
         // kt (waited for here), whose stage the next copies overwrite
-        if (STAGES == 3 && kt + 2 < kblocks) wait_newer(std::integral_constant<int, 1>{});
+        if (STAGES == 3 && kt + 2 < kblocks) vm_wait<PER_WAVE>();
         else vm_wait<0>();
         __syncthreads();
         read_frags(nst, 0, a[0], w[0]);
