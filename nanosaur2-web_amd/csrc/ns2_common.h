@@ -19,7 +19,7 @@ bool initialised();
 // Stream-ordered scratch owned by the library, grown on demand and reused by later calls
 // (one slot per concurrent use inside a single entry point).
 void* workspace(int slot, size_t bytes);
-constexpr int kWorkspaceSlots = 8;
+constexpr int kWorkspaceSlots = 7;
 // Device address of the current device's copy of the fixed scratch array that the
 // allocation-free entry points use (NS2_NOALLOC_SCRATCH_BYTES bytes, resolved by ns2_init), or
 // null before ns2_init has run on that device.
@@ -35,14 +35,11 @@ int lora_prepare(const float** t, const uint16_t* lora_a, const uint16_t* lora_b
 // in split order by the caller's row kernel). At fp16 tiled [ceil(M/64)*64][K]. Returns a status code.
 int linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_t* Wt, int M, int N, int K, float** part,
                           int* splits);
-// The int8 ConvRot linear on a file-layout weight W [N][K] through the tiled kernel: W is re-tiled
-// into Wt (library scratch) by each call, and so is a row-major fp16 input x16 [M][ldx] into
-// At. At: the rotated input as the tiled fp16 operand, already filled where x16 is null.
-// Returns a status code.
-int linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, int8_t* Wt, const float* scale,
-                      const float* bias, float* C, int M, int N, int K, int ldc, long long cOff, float alpha, int act,
-                      int resid, const float* gate, long long gOff, const uint16_t* lora_a, const uint16_t* lora_b,
-                      int lora_r);
+// The int8 ConvRot linear on a file-layout weight W [N][K] and rotated fp16 rows x [M][ldx] through the
+// tiled kernel, which reads both as they lie (no scratch but the LoRA term's). Returns a status code.
+int linear_i8_rows(const uint16_t* x, int ldx, const int8_t* W, const float* scale, const float* bias, float* C, int M,
+                   int N, int K, int ldc, long long cOff, float alpha, int act, int resid, const float* gate,
+                   long long gOff, const uint16_t* lora_a, const uint16_t* lora_b, int lora_r);
 
 // Kernel profiler (ns2_profile_*): when enabled, stream events bracket every launch and are
 // aggregated by kernel name on ns2_profile_report.

@@ -1334,17 +1334,21 @@ int launch_gemm(const GemmArgs& p, const char* name, const RowNorm* rn = nullptr
   return NS2_OK;
 }
 
-// Whether an int8 linear on a file-layout weight re-tiles its operands for the tiled kernel, which
-// multiplies at about twice the row-major kernel's rate. The re-tile costs a launch and one pass over
-// the weight (5-8 us), so it takes rows enough to share that and work enough to gain it. us row-major -> re-tiled,
-// N x K: 4608 x 1536: 300 rows 26.8 -> 22.8, 2432 rows 92.5 -> 53.4; 1536 x 1536: 300 17.8 -> 16.1, 2432 38.6 ->
-// 30.8; 8192 x 1536: 300 28.6 -> 30.4, 500 35.1 -> 33.7, 2432 135 -> 84; 1536 x 6144: 300 32.7 -> 33.7, 500
-// 50.6 -> 41.1, 2432 120 -> 80; 512 x 512: 4096 19.4 -> 13.8; 4608 x 256 with fp16 rows: 1000 15.7 -> 16.1. The tiled
-// kernel takes whole 64-row weight blocks and no added matrix.
-constexpr int kRetileRows = 400, kRetileK = 512;
-constexpr double kRetileWork = 1e9;
-inline bool retile_i8(const GemmArgs& p) {
-  return p.M >= kRetileRows && p.N > 0 && p.K >= kRetileK && (double)p.M * p.N * p.K >= kRetileWork && p.N % 64 == 0 && !p.add;
+// Whether an int8 linear on a file-layout weight runs on the tiled kernel's block tiles (linear_i8_rows), which
+// multiply at about twice the row-major kernel's rate and read rows and weights as they lie. us
+// row-major -> tiles, rotated fp16 rows, N x K: 4608 x 1536: 400 rows 22.4 -> 13.0, 2432 87.0 -> 41.0; 1536 x 1536: 450 rows
+// 17.3 -> 9.4, 2432 31.9 -> 19.2; 8192 x 1536: 400 28.7 -> 19.3, 2432 134 -> 69.6; 1536 x 6144: 400 32.9 -> 24.0, 2432 103 -> 58.9;
+// 512 x 512: 8192 17.8 -> 10.2. They do not split K, as the row-major kernel does where its 64x64 tiles leave
+// the chip idle: with fewer of those tiles than kRowsTiles a long K is faster there (x 64 x 4096: 1024 rows
+// 13.0 -> 16.8, 3952 (62 tiles) 15.7 -> 16.8, 8192 (128) 21.4 -> 17.3; x 256 x 4096: 1024 (64 tiles) 15.4 -> 17.0, 1536
+// (96) 19.0 -> 17.1). Fewer rows or less work stay with it as well: long K loses there
+// (1536 x 6144: 33 rows 14.7 -> 23.4, 300 rows 26.3 -> 23.9), short K would gain (4608 x 1536: 33 rows 11.1 -> 8.9). The tiles take
+// whole 64-row weight blocks and no added matrix.
+constexpr int kRowsM = 400, kRowsK = 512, kRowsTiles = 96;
+constexpr double kRowsWork = 1e9;
+inline bool rows_i8(const GemmArgs& p) {
+  return p.M >= kRowsM && p.N > 0 && p.N % 64 == 0 && p.K >= kRowsK && (double)p.M * p.N * p.K >= kRowsWork &&
+         (p.M + 63LL) / 64 * (p.N / 64) >= kRowsTiles && !p.add;
 }
 
 // The operands of a tiled fp16 linear, as the tiled kernel's entry points check them.
@@ -1429,24 +1433,14 @@ int ns2_linear_i8_lora(const void* A, int a_fmt, int lda, const int8_t* W, const
               "ns2_linear_i8: a_fmt must be 0 (fp32), 1 (rotated fp16) or 2 (rotated fp32)");
   NS2_REQUIRE(scale != nullptr, "ns2_linear_i8: null scale");
   NS2_REQUIRE(K % 256 == 0, "ns2_linear_i8: K=%d must be a multiple of 256 (ConvRot groups)", K);
-  // without memory for the re-tiled operands the call keeps the row-major kernel
-  int8_t* Wt = retile_i8(p) ? static_cast<int8_t*>(ns2::workspace(7, (size_t)N * K)) : nullptr;
   if (a_fmt != 1) {
     // fp32 input: rotate (ops.linear without xr, app/gpu/ops.js:54) or just cast a
     // pre-rotated xr, into library scratch
     NS2_REQUIRE(A && lda >= K && lda % 4 == 0 && aligned16(A), "ns2_linear_i8: bad fp32 A / lda=%d", lda);
-  }
-  uint16_t* xr = Wt ? static_cast<uint16_t*>(ns2::workspace(0, ((size_t)M + 63) / 64 * 64 * K * sizeof(uint16_t))) : nullptr;
-  const bool retile = xr != nullptr;
-  if (!retile && retile_i8(p)) (void)hipGetLastError();  // the failed allocation's
-  if (a_fmt != 1) {
-    if (!retile) xr = static_cast<uint16_t*>(ns2::workspace(0, (size_t)M * K * sizeof(uint16_t)));
+    uint16_t* xr = static_cast<uint16_t*>(ns2::workspace(0, (size_t)M * K * sizeof(uint16_t)));
     if (!xr) return ns2::set_error(NS2_ERR_OOM, "ns2_linear_i8: workspace allocation failed");
     if (a_fmt == 0) {
-      int rc = ns2_rotate_f16(static_cast<const float*>(A), lda, xr, K, M, K, retile);
-      if (rc) return rc;
-    } else if (retile) {
-      int rc = ns2_to_tiled_f16(static_cast<const float*>(A), lda, nullptr, 0, xr, M, K);
+      int rc = ns2_rotate_f16(static_cast<const float*>(A), lda, xr, K, M, K, 0);
       if (rc) return rc;
     } else {
       const long long quads = (long long)M * K / 4;
@@ -1459,9 +1453,9 @@ int ns2_linear_i8_lora(const void* A, int a_fmt, int lda, const int8_t* W, const
   }
   int rc = check_common(p, "ns2_linear_i8");
   if (rc) return rc;
-  if (retile)
-    return ns2::linear_i8_retiled(xr, a_fmt == 1 ? static_cast<const uint16_t*>(A) : nullptr, lda, W, Wt, scale, bias, C,
-                                  M, N, K, ldc, cOff, alpha, act, resid, gate, gOff, lora_a, lora_b, lora_r);
+  if (rows_i8(p))
+    return ns2::linear_i8_rows(static_cast<const uint16_t*>(p.A), p.lda, W, scale, bias, C, M, N, K, ldc, cOff, alpha, act,
+                               resid, gate, gOff, lora_a, lora_b, lora_r);
   if (lora_r) {
     // the LoRA down-projections take the rotated input (rotated A for int8 weights)
     rc = ns2::lora_prepare(&p.lt, lora_a, lora_b, lora_r, p.A, 1, p.lda, M, K, "ns2_linear_i8_lora");

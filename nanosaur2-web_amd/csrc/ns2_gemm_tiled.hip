@@ -25,8 +25,8 @@ using namespace ns2dev;
 namespace {
 
 struct TGemmArgs {
-  const half_t* At;
-  const uint8_t* Wt;
+  const half_t* At;   // tiled, or the rows of kI8Rows (lda halfs apart)
+  const uint8_t* Wt;  // tiled, or the int8 rows of kI8Rows
   const float* scale;
   const float* bias;
   float* C;
@@ -56,7 +56,12 @@ struct TGemmArgs {
   // vpk = nullptr: off. vcol0 and vD are multiples of 32 and M of 16.
   half_t* vpk;
   int vcol0, vD, vtiles;
+  int lda;
 };
+
+// A launch's operands: tiled fp16 rows with int8 or fp16 weight tiles, or fp16 rows and int8 weight rows as
+// they lie (K contiguous).
+enum Ops { kI8, kF16, kI8Rows };
 
 // 8 biased bytes (two dwords) -> 8 halfs: byte u -> half(0x6400 | u) - 1152 = u - 128 = w.
 // v_perm picks bytes of {x, 0x64646464}: selector bytes 4..7 are x's bytes, 0 is 0x64.
@@ -344,12 +349,17 @@ __device__ __forceinline__ void finish(const TGemmArgs& p, const float16_t (&acc
 // (ns2_tile_i8_weight_glu), so 64 columns of a wave hold 32 columns of each GLU half; the
 // block's 512 columns give 256 consecutive outputs act(h1) * h2, one rotation group, which is
 // rotated and written to Y as the tiled fp16 operand of the next int8 linear.
-// WF16: fp16 weight tiles (the plain bf16 linears, re-tiled as fp16; no per-row scale unless
+// OPS kF16: fp16 weight tiles (the plain bf16 linears, re-tiled as fp16; no per-row scale unless
 // given): 8 KB per 64x64 weight tile, read straight into the MFMA B operand.
+// OPS kI8Rows: nothing is re-tiled. A copy of 1 KB takes 8 rows x 128 bytes of A or 16 rows x 64 bytes of W
+// (whole lines), and each lane fetches the 16-byte piece whose index is XORed with its row's (row % 8
+// for A, row / 4 % 4 for W), so that the fragment reads of consecutive rows fall in different banks as
+// those of the tiled layout do. The sums have the order of the tiled launch.
 // WPE: waves per SIMD the registers must leave room for.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int KG, int KT, int STAGES, int SPREAD, int EPI, int ACT, int RM, bool LORA, bool WF16, int WPE>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int KG, int KT, int STAGES, int SPREAD, int EPI, int ACT, int RM, bool LORA, Ops OPS, int WPE>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * KG * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void gemm_tiled_kernel(TGemmArgs p) {
+  constexpr bool WF16 = OPS == kF16, ROWS = OPS == kI8Rows;
   constexpr int NW = WAVES_M * WAVES_N * KG;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -364,7 +374,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
   static_assert(BLOCKS % NW == 0, "copies must split evenly over the waves");
   static_assert(NS % 2 == 0, "an even number of steps per k-tile");
   static_assert(STAGES == 2 || (STAGES == 3 && SPREAD == 1), "two or three LDS stages");
-  static_assert(!WF16 || EPI == 0, "fp16 weights take the plain epilogue");
+  static_assert(OPS == kI8 || EPI == 0, "the GLU epilogue takes int8 weight tiles");
   __shared__ __attribute__((aligned(16))) char smem[STAGES * (A_BYTES + W_BYTES)];
   char* const as = smem;
   char* const ws = smem + STAGES * A_BYTES;
@@ -394,11 +404,30 @@ void gemm_tiled_kernel(TGemmArgs p) {
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
       const int j = wave + i * NW;
-      if (j < A_BLOCKS) {
+      if (ROWS && j < A_BLOCKS) {
+        // block (64 rows, k-tile, 8 rows); rows past M re-read the last one
+        const int c = j % (8 * KT);
+        const int mr = m0 + 64 * (j / (8 * KT)) + 8 * (c % 8) + (lane >> 3), m = mr < p.M ? mr : p.M - 1;
+        g_src[i] = reinterpret_cast<const char*>(p.At + (long long)m * p.lda + 64 * (kt0 + c / 8)) +
+                   ((lane & 7) ^ (lane >> 3)) * 16;
+        l_dst[i] = as_base + j * 1024;
+        g_step[i] = 128 * KT;
+        l_step[i] = A_BYTES;
+      } else if (ROWS) {
+        // block (64 weight rows, k-tile, 16 rows)
+        const int jw = j - A_BLOCKS, c = jw % (4 * KT);
+        int nb = n0 / 64 + jw / (4 * KT);
+        nb = nb < p.nblocks ? nb : p.nblocks - 1;
+        g_src[i] = reinterpret_cast<const char*>(p.Wt) + (long long)(64 * nb + 16 * (c % 4) + (lane >> 2)) * p.K +
+                   64 * (kt0 + c / 4) + ((lane & 3) ^ (lane >> 4)) * 16;
+        l_dst[i] = ws_base + jw * 1024;
+        g_step[i] = 64 * KT;
+        l_step[i] = W_BYTES;
+      } else if (j < A_BLOCKS) {
         const int mbi = j / (8 * KT), c = j % (8 * KT);
         int mb = m0 / 64 + mbi;
         mb = mb < p.mblocks ? mb : p.mblocks - 1;
-        g_src[i] = reinterpret_cast<const char*>(p.At) + ((long long)mb * kall * 8 + (long long)kt0 * 8 + c) * 1024;
+        g_src[i] = reinterpret_cast<const char*>(p.At) + ((long long)mb * kall * 8 + (long long)kt0 * 8 + c) * 1024 + lane * 16;
         l_dst[i] = as_base + j * 1024;
         g_step[i] = 8 * KT * 1024;
         l_step[i] = A_BYTES;
@@ -407,7 +436,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
         const int nbi = jw / (WCH * KT), c = jw % (WCH * KT);
         int nb = n0 / 64 + nbi;
         nb = nb < p.nblocks ? nb : p.nblocks - 1;
-        g_src[i] = reinterpret_cast<const char*>(p.Wt) + ((long long)nb * kall * WCH + (long long)kt0 * WCH + c) * 1024;
+        g_src[i] = reinterpret_cast<const char*>(p.Wt) + ((long long)nb * kall * WCH + (long long)kt0 * WCH + c) * 1024 + lane * 16;
         l_dst[i] = ws_base + jw * 1024;
         g_step[i] = WCH * KT * 1024;
         l_step[i] = W_BYTES;
@@ -415,7 +444,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
     }
   }
   auto dma_one = [&](int i, int kt, int st) {
-    dma16(g_src[i] + (long long)kt * g_step[i] + lane * 16, __builtin_amdgcn_readfirstlane(l_dst[i] + st * l_step[i]));
+    dma16(g_src[i] + (long long)kt * g_step[i], __builtin_amdgcn_readfirstlane(l_dst[i] + st * l_step[i]));
   };
 
   float16_t acc[TM][TN];
@@ -447,7 +476,22 @@ void gemm_tiled_kernel(TGemmArgs p) {
   // fp16 weights, read as the B operand itself)
   using WRaw = std::conditional_t<WF16, half8_t, uint2>;
   auto read_frags = [&](int st, int s, half8_t (&a)[TM], WRaw (&w)[TN]) {
-    const int kc = 2 * (s * KG + kg) + hi;
+    const int ks = s * KG + kg, kc = 2 * ks + hi;
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int col = wn * WTN + 32 * j;
+        w[j] = *reinterpret_cast<const WRaw*>(ws + st * W_BYTES + (col / 64 * KT + ks / 4) * 4096 + (col % 64 + lq) * 64 +
+                                              (((ks % 4) ^ (lq >> 2 & 3)) * 16 + hi * 8));
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int row = wm * WTM + 32 * i;
+        a[i] = *reinterpret_cast<const half8_t*>(as + st * A_BYTES + (row / 64 * KT + ks / 4) * 8192 + (row % 64 + lq) * 128 +
+                                                 ((kc % 8) ^ (lq & 7)) * 16);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int col = wn * WTN + 32 * j;
@@ -461,6 +505,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
   };
   auto decode = [&](const WRaw& w) {
     if constexpr (WF16) return w;
+    else if constexpr (ROWS) return u8x8_to_h8(make_uint2(w.x ^ 0x80808080u, w.y ^ 0x80808080u));
     else return u8x8_to_h8(w);
   };
 
@@ -785,25 +830,10 @@ __global__ __launch_bounds__(256) void tile_w16_kernel(const uint16_t* __restric
   *reinterpret_cast<uint4*>(Wt + i * 8) = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
-// x [M][ldx] row-major fp16 -> the tiled operand [ceil(M/64)][K/64][8][64][8], one thread per 16-byte
-// chunk; rows past M repeat the last one (their products are dropped).
-__global__ __launch_bounds__(256) void tile_x16_kernel(const uint16_t* __restrict__ x, int ldx, uint16_t* __restrict__ xt,
-                                                        int M, int K) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;  // output chunk index
-  const int row = (int)(i % 64);
-  const int c = (int)((i / 64) % 8);
-  const long long rest = i / 512;  // mb * (K/64) + kb
-  const int kb = (int)(rest % (K / 64));
-  const long long m = rest / (K / 64) * 64 + row;
-  if (m >= ((M + 63) & ~63)) return;
-  *reinterpret_cast<uint4*>(xt + i * 8) =
-      *reinterpret_cast<const uint4*>(x + (m < M ? m : M - 1) * ldx + kb * 64 + c * 8);
-}
-
 // Weight bytes per column band of the tile order: half of an XCD's 4 MB L2.
 constexpr long long kBandBytes = 2ll << 20;
 
-template <int BM, int BN, int WM, int WN, int KG, int KT, int STAGES, int SPREAD, int WPE, int EPI = 0, bool WF16 = false, bool RESID = true,
+template <int BM, int BN, int WM, int WN, int KG, int KT, int STAGES, int SPREAD, int WPE, int EPI = 0, Ops OPS = kI8, bool RESID = true,
           bool LORA = true, bool ANY_ACT = false>
 int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   p.tiles_m = (p.M + BM - 1) / BM;
@@ -815,7 +845,7 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   // with a few row tiles read each weight tile about once whatever the order.
   p.bands = 1;
   if (p.tiles_m >= 8) {
-    const double a_bytes = (double)p.tiles_m * BM * p.K * 2, w_bytes = (double)p.N * p.K * (WF16 ? 2 : 1);
+    const double a_bytes = (double)p.tiles_m * BM * p.K * 2, w_bytes = (double)p.N * p.K * (OPS == kF16 ? 2 : 1);
     double best = 0;
     for (int b = 1; b <= 8 && b <= p.tiles_n; b *= 2) {
       const double slice = w_bytes / b;
@@ -833,11 +863,11 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
     constexpr int A = decltype(act_c)::value, R = decltype(rm_c)::value;
     if constexpr (LORA) {
       if (p.lr) {
-        gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, true, WF16, WPE><<<grid, block, 0, s>>>(p);
+        gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, true, OPS, WPE><<<grid, block, 0, s>>>(p);
         return;
       }
     }
-    gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, false, WF16, WPE><<<grid, block, 0, s>>>(p);
+    gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, false, OPS, WPE><<<grid, block, 0, s>>>(p);
   };
   using std::integral_constant;
   if constexpr (EPI == 1) {
@@ -946,16 +976,40 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 namespace {
 
-// wf16: Wt holds fp16 weight tiles (ns2_tile_bf16_weight) and scale may be null; otherwise
-// int8 ConvRot tiles with their per-row scales (K a whole number of rotation groups).
-int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, const float* scale, const float* bias,
+// Launches block tile t; the tiles that OPS has no kernel for are not picked.
+template <Ops OPS>
+int launch_tile(Tile t, const TGemmArgs& p, int splits) {
+  if constexpr (OPS == kF16) {
+    switch (t) {
+      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 1, 3, 1, 2, 0, OPS, true, true, true>(p, splits);
+      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 3, 0, OPS, true, true, true>(p);
+      default: return launch_tiled<128, 192, 2, 2, 2, 1, 2, 1, 2, 0, OPS>(p);
+    }
+  } else {
+    switch (t) {
+      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, 0, OPS, true, true, true>(p, splits);
+      case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4, 0, OPS>(p);
+      case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 2, 3, 1, 2, 0, OPS>(p);
+      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, 0, OPS, true, true, true>(p);
+      case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, 0, OPS, false>(p);
+      case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2, 0, OPS>(p);
+      case T128x192K2: return launch_tiled<128, 192, 2, 2, 2, 2, 2, 2, 2, 0, OPS>(p);
+      case T192x384: return launch_tiled<192, 384, 2, 4, 1, 1, 2, 2, 2, 0, OPS, false, false>(p);
+      default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, 0, OPS, false, false>(p);
+    }
+  }
+}
+
+// ops kF16: Wt holds fp16 weight tiles (ns2_tile_bf16_weight) and scale may be null; otherwise int8 ConvRot
+// weights with their per-row scales (K a whole number of rotation groups). lda: row stride of kI8Rows.
+int linear_tiled(const char* fn, Ops ops, const uint16_t* At, int lda, const void* Wt, const float* scale, const float* bias,
                  float* C, int M, int N, int K, int ldc, long long cOff, float alpha, int act, int resid,
                  const float* gate, long long gOff, const uint16_t* lora_a, const uint16_t* lora_b, int lora_r,
                  uint16_t* vpk = nullptr, int vcol0 = 0, int vD = 0, int vtiles = 0) {
   NS2_READY();
   if (M == 0) return NS2_OK;
-  NS2_REQUIRE(At && Wt && (scale || wf16) && C, "%s: null At, Wt, scale or C", fn);
-  const int kmul = wf16 ? 64 : 256;
+  NS2_REQUIRE(At && Wt && (scale || ops == kF16) && C, "%s: null At, Wt, scale or C", fn);
+  const int kmul = ops == kF16 ? 64 : 256;
   NS2_REQUIRE(M > 0 && N > 0 && N % 64 == 0 && K > 0 && K % kmul == 0,
               "%s: M=%d N=%d K=%d (N %% 64 == 0, K %% %d == 0 required)", fn, M, N, K, kmul);
   NS2_REQUIRE(ldc >= N && cOff >= 0 && gOff >= 0, "%s: bad ldc/offsets", fn);
@@ -967,68 +1021,44 @@ int linear_tiled(const char* fn, bool wf16, const uint16_t* At, const void* Wt, 
   p.vcol0 = vcol0;
   p.vD = vD;
   p.vtiles = vtiles;
+  p.lda = lda;
   if (lora_r) {
-    int rc = ns2::lora_prepare(&p.lt, lora_a, lora_b, lora_r, At, 2, K, M, K, fn);
+    int rc = ns2::lora_prepare(&p.lt, lora_a, lora_b, lora_r, At, ops == kI8Rows ? 1 : 2, ops == kI8Rows ? lda : K, M, K, fn);
     if (rc) return rc;
     p.lb = reinterpret_cast<const half_t*>(lora_b);
     p.lr = lora_r;
   }
-  ns2::ProfScope prof_(wf16 ? "gemm_f16_tiled" : "gemm_i8_tiled");
+  ns2::ProfScope prof_(ops == kF16 ? "gemm_f16_tiled" : ops == kI8 ? "gemm_i8_tiled" : "linear_i8");
   // The tiles a launch may take: activations (none of the models' tiled linears has one) are built
   // for the two small tiles; fp16 weights for three tiles of one 64-wide k-tile per stage; the two
   // largest tiles have no registers left for old outputs or the LoRA term, 128x128 (three blocks
   // per CU) none for old outputs.
   unsigned allowed = (1u << kTiles) - 1;
   if (act != NS2_ACT_NONE) allowed = 1u << T64x64 | 1u << T64x128;
-  else if (wf16) allowed = 1u << T64x64 | 1u << T64x128 | 1u << T128x192K2;
+  else if (ops == kF16) allowed = 1u << T64x64 | 1u << T64x128 | 1u << T128x192K2;
   else if (resid || lora_r) allowed &= ~(1u << T192x384 | 1u << T256x256 | (resid ? 1u << T128x128 : 0u));
   int splits;
-  const Tile tile = pick_tile(M, N, K, allowed, !vpk, &splits);
+  const Tile tile = pick_tile(M, N, K, allowed, ops != kI8Rows && !vpk, &splits);
   if (splits > 1) {
     const int kt = K / 64;
     p.ksplit = (kt + splits - 1) / splits;
-    if (!wf16) p.ksplit += p.ksplit & 1;  // whole 128-wide stages
+    if (ops != kF16) p.ksplit += p.ksplit & 1;  // whole 128-wide stages
     splits = (kt + p.ksplit - 1) / p.ksplit;
   }
   if (splits > 1) {
     p.part = static_cast<float*>(ns2::workspace(5, (size_t)splits * M * N * sizeof(float)));
     if (!p.part) return ns2::set_error(NS2_ERR_OOM, "%s: split-K workspace allocation failed", fn);
   }
-  if (wf16) {
-    switch (tile) {
-      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 1, 3, 1, 2, 0, true, true, true, true>(p, splits);
-      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 3, 0, true, true, true, true>(p);
-      default: return launch_tiled<128, 192, 2, 2, 2, 1, 2, 1, 2, 0, true>(p);
-    }
-  }
-  switch (tile) {
-    case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, 0, false, true, true, true>(p, splits);
-    case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4>(p);
-    case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 2, 3, 1, 2>(p);
-    case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, 0, false, true, true, true>(p);
-    case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, 0, false, false>(p);
-    case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2>(p);
-    case T128x192K2: return launch_tiled<128, 192, 2, 2, 2, 2, 2, 2, 2>(p);
-    case T192x384: return launch_tiled<192, 384, 2, 4, 1, 1, 2, 2, 2, 0, false, false, false>(p);
-    default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, 0, false, false, false>(p);
-  }
+  if (ops == kF16) return launch_tile<kF16>(tile, p, splits);
+  return ops == kI8 ? launch_tile<kI8>(tile, p, splits) : launch_tile<kI8Rows>(tile, p, 1);
 }
 
 }  // namespace
 
-int ns2::linear_i8_retiled(uint16_t* At, const uint16_t* x16, int ldx, const int8_t* W, int8_t* Wt,
-                           const float* scale, const float* bias, float* C, int M, int N, int K, int ldc,
-                           long long cOff, float alpha, int act, int resid, const float* gate, long long gOff,
-                           const uint16_t* lora_a, const uint16_t* lora_b, int lora_r) {
-  if (x16) {
-    const long long chunks = (long long)((M + 63) / 64) * 64 * K / 8;
-    ns2::ProfScope prof_("tile_f16_rows");
-    tile_x16_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, ns2::stream()>>>(x16, ldx, At, M, K);
-    NS2_LAUNCHED("tile_f16_rows");
-  }
-  int rc = ns2_tile_i8_weight(W, Wt, N, K);
-  if (rc) return rc;
-  return linear_tiled("ns2_linear_i8", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate, gOff,
+int ns2::linear_i8_rows(const uint16_t* x, int ldx, const int8_t* W, const float* scale, const float* bias, float* C, int M,
+                        int N, int K, int ldc, long long cOff, float alpha, int act, int resid, const float* gate,
+                        long long gOff, const uint16_t* lora_a, const uint16_t* lora_b, int lora_r) {
+  return linear_tiled("ns2_linear_i8", kI8Rows, x, ldx, W, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate, gOff,
                       lora_a, lora_b, lora_r);
 }
 
@@ -1053,7 +1083,7 @@ int ns2::linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_
   *part = p.part;
   *splits = s;
   ns2::ProfScope prof_("gemm_f16_tiled");
-  return launch_tiled<64, 64, 2, 2, 1, 1, 3, 1, 2, 0, true, false, false>(p, s, false);
+  return launch_tiled<64, 64, 2, 2, 1, 1, 3, 1, 2, 0, kF16, false, false>(p, s, false);
 }
 
 extern "C" {
@@ -1121,7 +1151,7 @@ int ns2_linear_i8_glu_rot_tiled_lora(const uint16_t* At, const int8_t* Wt, const
 int ns2_linear_i8_tiled(const uint16_t* At, const int8_t* Wt, const float* scale, const float* bias,
                         float* C, int M, int N, int K, int ldc, long long cOff, float alpha, int act,
                         int resid, const float* gate, long long gOff) {
-  return linear_tiled("ns2_linear_i8_tiled", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate,
+  return linear_tiled("ns2_linear_i8_tiled", kI8, At, 0, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid, gate,
                          gOff, nullptr, nullptr, 0);
 }
 
@@ -1129,7 +1159,7 @@ int ns2_linear_i8_tiled_lora(const uint16_t* At, const int8_t* Wt, const float* 
                              float* C, int M, int N, int K, int ldc, long long cOff, float alpha, int act,
                              int resid, const float* gate, long long gOff, const uint16_t* lora_a,
                              const uint16_t* lora_b, int lora_r) {
-  return linear_tiled("ns2_linear_i8_tiled_lora", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid,
+  return linear_tiled("ns2_linear_i8_tiled_lora", kI8, At, 0, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, resid,
                          gate, gOff, lora_a, lora_b, lora_r);
 }
 
@@ -1147,14 +1177,14 @@ int ns2_tile_bf16_weight(const uint16_t* W, uint16_t* Wt, int N, int K) {
 
 int ns2_linear_f16w_tiled(const uint16_t* At, const uint16_t* Wt, const float* bias, float* C, int M, int N, int K,
                           int ldc, long long cOff, float alpha, int act, int resid, const float* gate, long long gOff) {
-  return linear_tiled("ns2_linear_f16w_tiled", true, At, Wt, nullptr, bias, C, M, N, K, ldc, cOff, alpha, act, resid,
+  return linear_tiled("ns2_linear_f16w_tiled", kF16, At, 0, Wt, nullptr, bias, C, M, N, K, ldc, cOff, alpha, act, resid,
                       gate, gOff, nullptr, nullptr, 0);
 }
 
 int ns2_linear_f16w_tiled_lora(const uint16_t* At, const uint16_t* Wt, const float* bias, float* C, int M, int N,
                                int K, int ldc, long long cOff, float alpha, int act, int resid, const float* gate,
                                long long gOff, const uint16_t* lora_a, const uint16_t* lora_b, int lora_r) {
-  return linear_tiled("ns2_linear_f16w_tiled_lora", true, At, Wt, nullptr, bias, C, M, N, K, ldc, cOff, alpha, act,
+  return linear_tiled("ns2_linear_f16w_tiled_lora", kF16, At, 0, Wt, nullptr, bias, C, M, N, K, ldc, cOff, alpha, act,
                       resid, gate, gOff, lora_a, lora_b, lora_r);
 }
 
@@ -1170,7 +1200,7 @@ int ns2_linear_i8_tiled_vpack(const uint16_t* At, const int8_t* Wt, const float*
               "(vcol0=%d H=%d D=%d N=%d; vcol0 %% 64 == 0, D %% 32 == 0)", vcol0, H, D, N);
   NS2_REQUIRE(M % 16 == 0 && M <= Lk, "ns2_linear_i8_tiled_vpack: M=%d must be a multiple of 16 and at most Lk=%d",
               M, Lk);
-  return linear_tiled("ns2_linear_i8_tiled_vpack", false, At, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, 0,
+  return linear_tiled("ns2_linear_i8_tiled_vpack", kI8, At, 0, Wt, scale, bias, C, M, N, K, ldc, cOff, alpha, act, 0,
                          nullptr, 0, lora_a, lora_b, lora_r, vpk, vcol0, D, (Lk + 63) / 64);
 }
 

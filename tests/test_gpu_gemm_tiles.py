@@ -107,11 +107,14 @@ def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
     close(buf[:M], before[:M].double() + ref if resid else ref, max(K, 1024), f"{tile} {M}x{N}x{K}")
 
 
-# both sides of the rule that re-tiles file-layout operands: rows, work, 64-row weight blocks
+# both sides of the rule that takes file-layout operands to the block tiles: rows, work, 64-row weight blocks
+# ("tiled" 3953x64x4096 has too few tiles and 8193x64x4096 enough)
 @pytest.mark.parametrize("route,M,N,K,resid,rank,act", [
     ("tiled", 400, 2560, 1024, True, 0, "none"), ("rows", 399, 2560, 1024, True, 0, "none"),
     ("tiled", 1001, 1600, 768, False, 32, "none"), ("rows", 1001, 1616, 768, False, 32, "none"),
     ("tiled", 3953, 64, 4096, True, 0, "silu"), ("rows", 3953, 64, 3840, True, 0, "silu"),
+    ("tiled", 8193, 64, 4096, True, 0, "silu"), ("tiled", 2500, 4608, 1536, False, 0, "none"),
+    ("tiled", 3953, 1536, 1536, False, 0, "none"), ("tiled", 1025, 1536, 1536, True, 0, "none"),
 ])
 def test_i8_file_layout(ns2lib, route, M, N, K, resid, rank, act):
     """The int8 linear on a file-layout weight (every int8 value, strided rows, a column window of C) for
@@ -158,6 +161,35 @@ def test_i8_file_layout(ns2lib, route, M, N, K, resid, rank, act):
     ns2lib.linear_i8(xr, 1, K, q, s, y1, M, N, K, **kw)
     torch.cuda.synchronize()
     assert torch.equal(y0, y1)
+
+
+def test_i8_file_layout_rotated_rows_keep_to_themselves(ns2lib):
+    """The linear on rotated fp16 rows and a file-layout weight uses no memory but its operands: none is
+    allocated, and calls that overlap on two streams do not meet."""
+    M, N, K = 512, 8192, 8192
+    g = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = [torch.randint(-128, 128, (N, K), generator=g, device=DEV, dtype=torch.int8) for _ in range(2)]
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    y, alone = ([torch.empty(M, N, device=DEV) for _ in range(2)] for _ in range(2))
+    main, streams = torch.cuda.current_stream(), [torch.cuda.Stream() for _ in range(2)]
+    ns2lib.linear_i8(x, 1, K, q[0], s, alone[0], 64, N, K)  # the kernels' code is loaded
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for i in range(2):
+        ns2lib.linear_i8(x, 1, K, q[i], s, alone[i], M, N, K)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < N * K // 2, "device memory was allocated"
+    close(alone[0], (x.double() @ q[0].double().T) * s.double(), K, "file layout 512x8192x8192")
+    try:
+        for _ in range(8):
+            for i in range(2):
+                ns2lib.set_stream(streams[i].cuda_stream)
+                ns2lib.linear_i8(x, 1, K, q[i], s, y[i], M, N, K)
+    finally:
+        ns2lib.set_stream(main.cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], alone[0]) and torch.equal(y[1], alone[1])
 
 
 @pytest.mark.parametrize("M,N,K", [(1001, 1616, 768), (65, 4120, 256)])
