@@ -653,11 +653,13 @@ __global__ __launch_bounds__(512) void splitk_glu_down_kernel(GemmArgs p, int sp
 // us per encoder pass of 17 layers with weights from memory, 256 / 37 tokens: two launches each 915 / 734,
 // one launch 836 / 761, with the turned starts 785 / 722, with the fetching blocks 784 / 700. With
 // 4-byte loads that touch the down weights' lines at the start 841 / 771.
-constexpr int kFewRowsTiles = 8;  // row tiles launched at least
+constexpr int kFewRowsTiles = 8;     // row tiles launched at least,
+constexpr int kFewRowsBlocks = 128;  // while the blocks stay below this
 
-inline __host__ __device__ int few_rows_tiles(int M, int rt) {
+inline int few_rows_tiles(int M, int rt, int groups) {
   const int t = (M + 16 * rt - 1) / (16 * rt);
-  return t < kFewRowsTiles ? kFewRowsTiles : t;
+  const int fetch = kFewRowsBlocks / groups < kFewRowsTiles ? kFewRowsBlocks / groups : kFewRowsTiles;
+  return t < fetch ? fetch : t;
 }
 
 // Block id -> (row tile, column group): XCD x = id % 8 owns a contiguous range of the groups' row tiles.
@@ -757,12 +759,11 @@ __device__ __forceinline__ void few_rows_product(const half_t* At, const half_t*
 // RoPE partners D/2 + 16w .. of the head. 96 blocks at 256 rows x 6 heads.
 template <int D, int RT, int CH>
 __global__ __launch_bounds__(2 * D) void few_rows_head_norm_kernel(const half_t* __restrict__ At, const half_t* __restrict__ Wt, GemmArgs p,
-                                                                   HeadNorm hn) {
+                                                                   HeadNorm hn, int row_tiles) {
   constexpr int NW = D / 32;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float red[NW][16 * RT];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, grp = lane >> 4;
-  const int row_tiles = few_rows_tiles(p.M, RT);
   int rt, h;
   few_rows_tile(row_tiles, p.N / D, rt, h);
   const int m0 = rt * 16 * RT + 4 * grp, c0 = 16 * wave + l16;  // the lane's first row; its first column within the head
@@ -848,14 +849,13 @@ __global__ __launch_bounds__(2 * D) void few_rows_head_norm_kernel(const half_t*
 // at 256 rows x 2048 GLU columns.
 template <int GS, int RT, int CH>
 __global__ __launch_bounds__(GS * 4) void few_rows_glu_down_kernel(const half_t* __restrict__ At, const half_t* __restrict__ Wt, GemmArgs p,
-                                                                   GluDown gd) {
+                                                                   GluDown gd, int row_tiles) {
   // waves, 32-wide steps of the down product, its tiles per round trip, those that go out at the start
   constexpr int NW = GS / 16, DS = GS / 32, JC = 5, JE = RT == 1 ? 3 : 1;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ __attribute__((aligned(16))) half_t g16[RT * 16 * GS];  // the GLU output in fragment order
   const int I = p.N / 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, grp = lane >> 4;
-  const int row_tiles = few_rows_tiles(p.M, RT);
   int rt, cg;
   few_rows_tile(row_tiles, I / GS, rt, cg);
   const int j0 = cg * GS, j = j0 + 16 * wave + l16, nt = gd.Nd / 16;
@@ -920,8 +920,33 @@ __global__ __launch_bounds__(GS * 4) void few_rows_glu_down_kernel(const half_t*
 // 726, 512 1135 -> 919, 600 1342 -> 1145, 1000 1680 -> 1380 (the norm kernels' weights included).
 constexpr int kFewRows = 1024, kFewRows16 = 256;
 constexpr int kFewRowsPlanes = 60 * 1024;  // LDS bytes of the rows' planes (the GLU output takes 4 KB per 16 rows more)
-inline bool few_rows(int M, int K) {
+inline bool few_rows_fit(int M, int K) {
   return M <= kFewRows && K % 64 == 0 && (M <= kFewRows16 ? 1 : 2) * (long long)K * 32 <= kFewRowsPlanes;
+}
+
+// Which of those calls one launch is faster for. Each block streams its whole weight slice through one
+// CU, where the two launches split K over the chip: a slice may be the larger, the more there is to
+// save, that is the more columns (or groups and row tiles) the two launches would write and read back.
+// Lines through 3700 pairs of launches (head dims 64-256, 1-8 heads, 1-64 GLU groups, Nd 64-2048, K
+// 64-1920, 1-1024 rows), on the side where one launch is at most 3 % slower. Time of one launch over that of two: head
+// norm at 37 rows, 6 heads of 256: K = 640 0.91, 1024 0.98, 1280 1.15; one head of 256: 512 0.97, 640 1.06, 1536
+// 1.43; at 300 rows, one head: 256 0.99, 512 1.14. GLU + down, Nd = 640, K = 640: 16 groups 1 row 1.04, 37 rows 0.96,
+// 256 rows 0.67; one group 1.07; K = 1536: 16 groups 37 rows 1.19, 100 rows 0.91.
+inline bool few_rows_head_norm(int M, int N, int K, int D) {
+  if (!few_rows_fit(M, K)) return false;
+  const long long slice = (long long)D * K;
+  if (M > kFewRows16) return slice <= 20 * 1024 + 140LL * N;
+  return slice <= 92 * 1024 + 96LL * N && (D > 64 || K <= 832 + N);
+}
+inline bool few_rows_glu_down(int M, int N, int K, int Nd) {
+  if (!few_rows_fit(M, K)) return false;
+  const int groups = N / 2 / kGluDownGroup, tiles = (M + 15) / 16;
+  if (M > kFewRows16) return groups > 2 || K <= 320;
+  if (tiles > 4) return K <= (groups >= 8 ? 1152 : groups > 2 ? 768 : 512);
+  // bytes of a block's weights: 256 GLU columns of K, 128 columns of Nd
+  const long long slice = 512LL * K + 256LL * Nd, most = 400 * 1024;
+  if (tiles == 1 || groups <= 8) return slice <= most && K <= 512;
+  return slice <= most + 18 * 1024 * (groups - 8) && K <= 1024;
 }
 
 // Whether an output of the call overlaps its tiled rows: one launch would overwrite rows that other
@@ -948,16 +973,16 @@ template <int D>
 void launch_few_rows_head_norm(const half_t* At, const half_t* Wt, const GemmArgs& p, const HeadNorm& hn, hipStream_t s) {
   few_rows_dispatch(p.M, p.K, [&](auto rt, auto ch) {
     constexpr int RT = decltype(rt)::value, CH = decltype(ch)::value;
-    const int blocks = few_rows_tiles(p.M, RT) * (p.N / D);
-    few_rows_head_norm_kernel<D, RT, CH><<<blocks, 2 * D, RT * p.K * 32, s>>>(At, Wt, p, hn);
+    const int tiles = few_rows_tiles(p.M, RT, p.N / D);
+    few_rows_head_norm_kernel<D, RT, CH><<<tiles * (p.N / D), 2 * D, RT * p.K * 32, s>>>(At, Wt, p, hn, tiles);
   });
 }
 
 void launch_few_rows_glu_down(const half_t* At, const half_t* Wt, const GemmArgs& p, const GluDown& gd, hipStream_t s) {
   few_rows_dispatch(p.M, p.K, [&](auto rt, auto ch) {
     constexpr int RT = decltype(rt)::value, CH = decltype(ch)::value;
-    const int blocks = few_rows_tiles(p.M, RT) * (p.N / 2 / kGluDownGroup);
-    few_rows_glu_down_kernel<kGluDownGroup, RT, CH><<<blocks, 512, RT * p.K * 32, s>>>(At, Wt, p, gd);
+    const int groups = p.N / 2 / kGluDownGroup, tiles = few_rows_tiles(p.M, RT, groups);
+    few_rows_glu_down_kernel<kGluDownGroup, RT, CH><<<tiles * groups, 512, RT * p.K * 32, s>>>(At, Wt, p, gd, tiles);
   });
 }
 
@@ -1620,7 +1645,7 @@ int ns2_linear_f16w_tiled_head_norm_f16kv(const uint16_t* At, const uint16_t* Wt
   const HeadNorm hn{w1, H1, w2, H2, D, cs, sin_off, cs ? rope_rows : 0, eps, reinterpret_cast<half_t*>(kv16), ldkv};
   GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, C, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   hipStream_t s = ns2::stream();
-  if (few_rows(M, K) && !overlaps(C, (size_t)M * N * 4, At, M, K) && !overlaps(kv16, (size_t)M * ldkv * 2, At, M, K)) {
+  if (few_rows_head_norm(M, N, K, D) && !overlaps(C, (size_t)M * N * 4, At, M, K) && !overlaps(kv16, (size_t)M * ldkv * 2, At, M, K)) {
     int rc = check_tiled_f16(fn, At, Wt, M, N, K);
     if (rc) return rc;
     const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);
@@ -1657,7 +1682,7 @@ int ns2_linear_f16w_tiled_glu_down(const uint16_t* At, const uint16_t* Wt, const
   NS2_REQUIRE(aligned16(wd_tiled), "%s: wd_tiled must be 16-byte aligned", fn);
   GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, part, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   const GluDown gd{reinterpret_cast<const half_t*>(wd_tiled), part, Nd, act, glu_down_ranges(M, N, Nd)};
-  if (few_rows(M, K) && !overlaps(part, (size_t)(N / 2 / kGluDownGroup) * M * Nd * 4, At, M, K)) {
+  if (few_rows_glu_down(M, N, K, Nd) && !overlaps(part, (size_t)(N / 2 / kGluDownGroup) * M * Nd * 4, At, M, K)) {
     int rc = check_tiled_f16(fn, At, Wt, M, N, K);
     if (rc) return rc;
     const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);

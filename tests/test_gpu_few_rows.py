@@ -98,6 +98,37 @@ def test_glu_down(ns2lib, M, K, inner, Nd, act, bias):
         close(part[s * M:s * M + M], ref, 2.0**-11, f"share {s}")
 
 
+# M, D, heads, K of the q|k|v linear, or M, GLU columns, Nd, K: both sides of the rules that choose between one launch
+# and two, with the largest weight slices that one launch takes
+@pytest.mark.parametrize("one,M,D,heads,K", [(True, 16, 256, 6, 896), (False, 16, 256, 6, 1024), (True, 37, 64, 2, 960),
+                                             (False, 37, 64, 2, 1024), (True, 256, 128, 8, 1472), (False, 256, 128, 8, 1536),
+                                             (True, 257, 256, 6, 896), (False, 257, 256, 6, 960), (False, 300, 256, 1, 256)])
+def test_head_norm_route(ns2lib, one, M, D, heads, K):
+    ns2lib.profile_reset()
+    ns2lib.profile(True)
+    try:
+        test_head_norm(ns2lib, M, K, D, heads, heads - 1, 0, True)
+        names = ns2lib.profile_report()
+    finally:
+        ns2lib.profile(False)
+    assert ("linear_head_norm_f16kv" in names) == one and ("head_norm_f16kv" in names) != one
+
+
+@pytest.mark.parametrize("one,M,inner,Nd,K", [(True, 16, 2048, 640, 448), (False, 16, 2048, 640, 512), (True, 17, 8192, 64, 1024),
+                                              (False, 17, 8192, 64, 1088), (False, 64, 256, 640, 576), (True, 65, 1024, 64, 1152),
+                                              (False, 65, 1024, 64, 1216), (True, 65, 512, 64, 768), (False, 257, 256, 64, 384),
+                                              (True, 257, 384, 64, 960), (True, 10, 6144, 64, 512)])
+def test_glu_down_route(ns2lib, one, M, inner, Nd, K):
+    ns2lib.profile_reset()
+    ns2lib.profile(True)
+    try:
+        test_glu_down(ns2lib, M, K, inner, Nd, "silu", True)
+        names = ns2lib.profile_report()
+    finally:
+        ns2lib.profile(False)
+    assert ("linear_glu_down" in names) == one and ("glu_down" in names) != one
+
+
 def test_outputs_over_the_rows(ns2lib):
     """An output that overlaps the tiled rows (only the last launch of a call may store)."""
     M, K, N, D = 100, 640, 1536, 256
