@@ -949,11 +949,11 @@ inline bool few_rows_glu_down(int M, int N, int K, int Nd) {
   return slice <= most + 18 * 1024 * (groups - 8) && K <= 1024;
 }
 
-// Whether an output of the call overlaps its tiled rows: one launch would overwrite rows that other
-// blocks still read, so such a call keeps the two launches, of which only the second stores.
-inline bool overlaps(const void* out, size_t out_bytes, const uint16_t* At, int M, int K) {
-  const uintptr_t o = (uintptr_t)out, a = (uintptr_t)At;
-  return o < a + ((size_t)M + 63) / 64 * 64 * K * 2 && a < o + out_bytes;
+// Whether an output of the call overlaps its tiled rows or weights: one launch would overwrite what
+// other blocks still read, so such a call keeps the two launches, of which only the second stores.
+inline bool overlaps(const void* out, size_t out_bytes, const uint16_t* At, const uint16_t* Wt, int M, int N, int K) {
+  const uintptr_t o = (uintptr_t)out, a = (uintptr_t)At, w = (uintptr_t)Wt;
+  return (o < a + ((size_t)M + 63) / 64 * 64 * K * 2 && a < o + out_bytes) || (o < w + (size_t)N * K * 2 && w < o + out_bytes);
 }
 
 // f(RT, CH) with the row tiles per block and the chunk of a call
@@ -1645,7 +1645,8 @@ int ns2_linear_f16w_tiled_head_norm_f16kv(const uint16_t* At, const uint16_t* Wt
   const HeadNorm hn{w1, H1, w2, H2, D, cs, sin_off, cs ? rope_rows : 0, eps, reinterpret_cast<half_t*>(kv16), ldkv};
   GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, C, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   hipStream_t s = ns2::stream();
-  if (few_rows_head_norm(M, N, K, D) && !overlaps(C, (size_t)M * N * 4, At, M, K) && !overlaps(kv16, (size_t)M * ldkv * 2, At, M, K)) {
+  if (few_rows_head_norm(M, N, K, D) && !overlaps(C, (size_t)M * N * 4, At, Wt, M, N, K) &&
+      !overlaps(kv16, (size_t)M * ldkv * 2, At, Wt, M, N, K)) {
     int rc = check_tiled_f16(fn, At, Wt, M, N, K);
     if (rc) return rc;
     const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);
@@ -1682,7 +1683,7 @@ int ns2_linear_f16w_tiled_glu_down(const uint16_t* At, const uint16_t* Wt, const
   NS2_REQUIRE(aligned16(wd_tiled), "%s: wd_tiled must be 16-byte aligned", fn);
   GemmArgs q{nullptr, nullptr, nullptr, bias, nullptr, part, nullptr, 0, 0, 0, N, M, N, K, 1.0f, NS2_ACT_NONE, 0};
   const GluDown gd{reinterpret_cast<const half_t*>(wd_tiled), part, Nd, act, glu_down_ranges(M, N, Nd)};
-  if (few_rows_glu_down(M, N, K, Nd) && !overlaps(part, (size_t)(N / 2 / kGluDownGroup) * M * Nd * 4, At, M, K)) {
+  if (few_rows_glu_down(M, N, K, Nd) && !overlaps(part, (size_t)(N / 2 / kGluDownGroup) * M * Nd * 4, At, Wt, M, N, K)) {
     int rc = check_tiled_f16(fn, At, Wt, M, N, K);
     if (rc) return rc;
     const half_t *a = reinterpret_cast<const half_t*>(At), *w = reinterpret_cast<const half_t*>(Wt);

@@ -149,3 +149,27 @@ def test_outputs_over_the_rows(ns2lib):
         outs.append((c[:, :4 * D].clone(), kv))
     close(outs[1][0], outs[0][0].double(), 2.0**-19, "q over the rows")
     close(outs[1][1].float(), outs[0][1].double(), 2.0**-11, "k and v")
+
+
+def test_outputs_over_the_weights(ns2lib):
+    """An output that overlaps the weights, which only the first of two launches reads."""
+    M, K, inner, Nd = 200, 640, 1024, 640
+    g = torch.Generator(device=DEV).manual_seed(4)
+    x = tiled(torch.randn(M, K, generator=g, device=DEV).half())
+    _, wt = weight(ns2lib, 2 * inner, K, g)
+    _, wdt = weight(ns2lib, Nd, inner, g)
+    alone = torch.empty(inner // 128 * M, Nd, device=DEV)
+    ns2lib.linear_f16w_tiled_glu_down(x, wt, None, M, 2 * inner, K, wdt, Nd, alone)
+    part = torch.empty_like(alone)
+    part.view(-1)[:wt.numel() // 2] = wt.reshape(-1).view(torch.float32)
+    ns2lib.linear_f16w_tiled_glu_down(x, part, None, M, 2 * inner, K, wdt, Nd, part)
+    torch.cuda.synchronize()
+    close(part, alone.double(), 2.0**-11, "shares over the weights")
+    w, c = torch.randn(256, generator=g, device=DEV), torch.empty(M, 2 * inner, device=DEV)
+    kv, over = (torch.empty(M, 1024, dtype=torch.float16, device=DEV) for _ in range(2))
+    ns2lib.linear_f16w_tiled_head_norm_f16kv(x, wt, None, c, M, 2 * inner, K, w, 4, w, 1, 256, kv, 1024)
+    buf = wt.reshape(-1).view(torch.float16).clone()
+    ns2lib.linear_f16w_tiled_head_norm_f16kv(x, buf, None, c, M, 2 * inner, K, w, 4, w, 1, 256, buf, 1024)
+    torch.cuda.synchronize()
+    over.copy_(buf[:M * 1024].reshape(M, 1024))
+    close(over.float(), kv.double(), 2.0**-10, "k and v over the weights")
