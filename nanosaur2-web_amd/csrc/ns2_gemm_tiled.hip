@@ -139,22 +139,27 @@ __device__ __forceinline__ void block_tile(const TGemmArgs& p, int& tm, int& tn)
 
 // The epilogues below work on a wave's sums acc[i][j][r] = C[mw + 32i + 8(r/4) + 4hi + r%4][nw + 32j + lq]
 // (mw, nw the wave's first row and column, both uniform; lq = lane % 32, hi = lane / 32). Rows are
-// addressed as a uniform pointer plus a 32-bit lane offset. Every value loaded for an epilogue is
+// addressed as a uniform pointer plus a lane offset of 64 bits (4 ldc may exceed 32). Every value loaded for an epilogue is
 // waited for once, before the first store (pin): the stores then issue back to back. With the
 // wait inside a per-row branch the compiler drained every earlier store before each one, and the
 // stores of a wave ran one memory round trip after another.
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 
-// Old outputs of tile (i, j).
+// Old outputs of tile (i, j); rows past M read the last one (their results are dropped).
 __device__ __forceinline__ void load_old(const TGemmArgs& p, float (&old)[16], int mw, int nw, int lq, int hi) {
   const float* base = p.C + p.cOff + (long long)mw * p.ldc + nw;
   const int rows = p.M - mw;
+  if (rows >= 32) {
+    const long long lane_off = 4LL * hi * p.ldc + lq;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) old[r] = (base + (long long)(8 * (r >> 2) + (r & 3)) * p.ldc)[lane_off];
+    return;
+  }
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    // rows past M read the last one (their results are dropped)
     int dm = 8 * (r >> 2) + 4 * hi + (r & 3);
     dm = dm < rows ? dm : (rows > 0 ? rows - 1 : 0);
-    old[r] = base[(unsigned)(dm * p.ldc + lq)];
+    old[r] = base[(long long)dm * p.ldc + lq];
   }
 }
 
@@ -186,7 +191,7 @@ __device__ __forceinline__ void store_plain(const TGemmArgs& p, const float16_t 
     if (RM) pin(gt[j]);
   }
   float* base = p.C + p.cOff + (long long)mw * p.ldc + nw;
-  const unsigned lane_off = (unsigned)(4 * hi * p.ldc + lq);
+  const long long lane_off = 4LL * hi * p.ldc + lq;
 #pragma unroll
   for (int t = 0; t < TM * TN; ++t) {
     const int j = t / TM, i = t % TM;
@@ -283,7 +288,7 @@ __device__ __forceinline__ void store_vpack(const TGemmArgs& p, const float16_t 
         q.y = pack_half2(v[2], v[3]);
         q.z = pack_half2(v[4], v[5]);
         q.w = pack_half2(v[6], v[7]);
-        *reinterpret_cast<uint4*>(dst0 + (kt * 8 + kc) * p.vD * 8) = q;
+        *reinterpret_cast<uint4*>(dst0 + ((long long)kt * 8 + kc) * p.vD * 8) = q;
       }
     }
   }
@@ -297,7 +302,7 @@ __device__ __forceinline__ void finish(const TGemmArgs& p, const float16_t (&acc
   if (p.part) {
     // split-K: the raw partial products of split blockIdx.y
     float* base = p.part + ((long long)blockIdx.y * p.M + mw) * p.N + nw;
-    const unsigned lane_off = (unsigned)(4 * hi * p.N + lq);
+    const long long lane_off = 4LL * hi * p.N + lq;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if (nw + 32 * j >= p.N) continue;

@@ -89,6 +89,28 @@ def test_i8_tiles(ns2lib, tile, M, N, K, resid, rank):
         close(buf[:M], ref, K, f"{tile} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 64, 256), (40, 128, 4096), (70, 12288, 512)])
+def test_rows_far_apart(ns2lib, M, N, K):
+    """Old outputs and stores where 31 output rows span more than 2^31 (70 rows) or 2^32 (40 rows) elements, in
+    20 GB that are never filled."""
+    ldc = (1 << (32 if M == 40 else 31)) // 31 + 64
+    buf = torch.empty(M * ldc, device=DEV)
+    c = buf.as_strided((M, N), (ldc, 1))
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+    wt = torch.empty_like(q)
+    ns2lib.tile_i8_weight(q, wt, N, K)
+    old = torch.randn(M, N, generator=g, device=DEV)
+    c.copy_(old)
+    ns2lib.linear_i8_tiled(tiled(x), wt, s, buf, M, N, K, ldc=ldc, resid=True)
+    torch.cuda.synchronize()
+    close(c.contiguous(), old.double() + (x.double() @ q.double().T) * s.double(), K, f"{M}x{N}x{K} ldc {ldc}")
+    del buf, c
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("tile,M,N,K,resid", [("64x64", 70, 64, 64, False), ("64x64 split K", 65, 1536, 1600, True),
                                               ("64x128", 1000, 1536, 64, False), ("128x192", 3951, 1600, 1536, True)])
 def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
