@@ -1,0 +1,4 @@
+// The tiled GEMM's plain launches on int8 weight rows and fp16 rows as they lie.
+#include "ns2_gemm_tiled.h"
+
+template int ns2tiled::launch_tile<ns2tiled::kI8Rows>(ns2tiled::Tile, const ns2tiled::TGemmArgs&, int);
