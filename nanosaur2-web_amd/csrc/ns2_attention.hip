@@ -505,11 +505,11 @@ struct TileLoader {
 // score exceeds it by more than 2^kRebase; between moves the output accumulator needs no
 // rescale. Any reference gives the same softmax, and p <= 2^kRebase stays in fp16 range.
 constexpr float kRebase = 8.0f;
-// A tile whose maximum is more than this above the reference makes what came before it vanish (2^-256 is
-// 0 in fp32), and its scores, formed on top of -m_ref, have lost the bits that a reference far below them
-// takes: after a first tile masked with -1e9 the next tile's scores would be multiples of 128. Such a
-// tile is scored again from 0, as a query's first tile.
-constexpr float kRescore = 256.0f;
+// The part of the reference that the score chains start from is never below -kLowRef: scores formed on top
+// of a reference far below them lose the bits it takes (after a first tile masked with -1e9 the next
+// tile's would be multiples of 128). What is below is kept apart (m_low, 0 or negative, so that the reference is m_ref +
+// m_low) and subtracted from the finished scores, when the tile does not move the reference anyway.
+constexpr float kLowRef = 1024.0f;
 
 // KS: key parts. The NW waves of a block are NW / KS query waves times KS key parts: a stage holds KS
 // consecutive tiles and part g works on tile u KS + g of stage u; the parts' outputs, references and
@@ -572,11 +572,12 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[qt][dt][r] = 0.f;
-  float m_ref[QT], l_run[QT];
+  float m_ref[QT], m_low[QT], l_run[QT];
   bool fresh[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     m_ref[qt] = 0.f;
+    m_low[qt] = 0.f;
     l_run[qt] = 0.f;
     fresh[qt] = true;
   }
@@ -695,7 +696,8 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       fresh[qt] = !(mA[qt] > -INFINITY);
-      m_ref[qt] = fresh[qt] ? 0.f : mA[qt];
+      m_ref[qt] = fresh[qt] ? 0.f : fmaxf(mA[qt], -kLowRef);
+      m_low[qt] = fresh[qt] ? 0.f : mA[qt] - m_ref[qt];
     }
     set_minit();
 #pragma unroll
@@ -727,35 +729,17 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
     {
       bool need = false;
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) need |= (mx_cur[qt] > kRebase) || fresh[qt];
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) != 0, 0)) {
-        bool any_far = false, far[QT];
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-          far[qt] = (mx_cur[qt] > kRescore) && !fresh[qt];
-          any_far |= far[qt];
-        }
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_far) != 0, 0)) {
-          // K and the biases of tile t are in LDS until the end of the step
-#pragma unroll
-          for (int qt = 0; qt < QT; ++qt) {
-            m_ref[qt] = far[qt] ? 0.f : m_ref[qt];
-            fresh[qt] |= far[qt];
-          }
-          set_minit();
-#pragma unroll
-          for (int i = 0; i < NK; ++i) qk_mfma(s_cur, i, read_k(i, vbuf));
-          if (u * KS + kg >= a.bias_block0) add_bias(s_cur, vbuf);
-#pragma unroll
-          for (int qt = 0; qt < QT; ++qt) mx_cur[qt] = col_max(fmaxf(half_max(s_cur, 0, qt), half_max(s_cur, 1, qt)));
-        }
+      for (int qt = 0; qt < QT; ++qt) need |= (mx_cur[qt] > kRebase) || m_low[qt] != 0.f || fresh[qt];
+      if (__builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           const bool seen = mx_cur[qt] > -INFINITY;
-          const float shift = fresh[qt] ? (seen ? mx_cur[qt] : 0.f) : fmaxf(mx_cur[qt], 0.f);
-          const float alpha = far[qt] ? 0.f : (fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift));
+          const float shift = fresh[qt] ? (seen ? mx_cur[qt] : 0.f) : fmaxf(mx_cur[qt], m_low[qt]);
+          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(m_low[qt] - shift);
           fresh[qt] = fresh[qt] && !seen;
-          m_ref[qt] += shift;
+          const float ref = m_ref[qt] + shift;
+          m_ref[qt] = fmaxf(ref, -kLowRef);
+          m_low[qt] = ref - m_ref[qt];
           l_run[qt] *= alpha;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
@@ -899,7 +883,7 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
           for (int g = 0; g < 4; ++g)
             X[(((wq * QT + qt) * DT + dt) * 4 + g) * 64 + lane] =
                 make_float4(o[qt][dt][4 * g], o[qt][dt][4 * g + 1], o[qt][dt][4 * g + 2], o[qt][dt][4 * g + 3]);
-        R[(wq * QT + qt) * 128 + lane] = fresh[qt] ? -INFINITY : m_ref[qt];
+        R[(wq * QT + qt) * 128 + lane] = fresh[qt] ? -INFINITY : m_ref[qt] + m_low[qt];
         R[(wq * QT + qt) * 128 + 64 + lane] = l_run[qt];
       }
     }
@@ -908,7 +892,7 @@ __global__ __launch_bounds__(NW * 64) void flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       const float m1 = R[(wq * QT + qt) * 128 + lane], l1 = R[(wq * QT + qt) * 128 + 64 + lane];
-      const float m0 = fresh[qt] ? -INFINITY : m_ref[qt], m = fmaxf(m0, m1);
+      const float m0 = fresh[qt] ? -INFINITY : m_ref[qt] + m_low[qt], m = fmaxf(m0, m1);
       const float s0 = __builtin_amdgcn_exp2f(m0 - m), s1 = __builtin_amdgcn_exp2f(m1 - m);
       l_run[qt] = l_run[qt] * s0 + l1 * s1;
 #pragma unroll
@@ -1014,12 +998,13 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[qt][dt][r] = 0.f;
-  float m_ref[QT], l_run[QT];
+  float m_ref[QT], m_low[QT], l_run[QT];
   bool fresh[QT];
   float16_t minit[QT];  // -m_ref in every accumulator slot: the C operand of each score chain
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     m_ref[qt] = 0.f;
+    m_low[qt] = 0.f;
     l_run[qt] = 0.f;
     fresh[qt] = true;
 #pragma unroll
@@ -1067,7 +1052,7 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
     }
     // ---- S^T = K Q^T - m_ref
     float16_t s[2][QT];
-    auto scores = [&]() {
+    {
       half8_t kf[2][2], qf[2][QT];
       kf[0][0] = read_k(0, 0, buf);
       kf[0][1] = read_k(0, 1, buf);
@@ -1091,61 +1076,42 @@ __global__ __launch_bounds__(512) void flash_wide_kernel(FlashArgs a) {
                                                                0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (BIAS) {
+    }
+    if constexpr (BIAS) {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const float4 bb = *reinterpret_cast<const float4*>(&kbias[buf][kt * 32 + 8 * g + 4 * hi]);
+        for (int g = 0; g < 4; ++g) {
+          const float4 bb = *reinterpret_cast<const float4*>(&kbias[buf][kt * 32 + 8 * g + 4 * hi]);
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt) {
-              s[kt][qt][4 * g + 0] += bb.x;
-              s[kt][qt][4 * g + 1] += bb.y;
-              s[kt][qt][4 * g + 2] += bb.z;
-              s[kt][qt][4 * g + 3] += bb.w;
-            }
+          for (int qt = 0; qt < QT; ++qt) {
+            s[kt][qt][4 * g + 0] += bb.x;
+            s[kt][qt][4 * g + 1] += bb.y;
+            s[kt][qt][4 * g + 2] += bb.z;
+            s[kt][qt][4 * g + 3] += bb.w;
           }
-      }
-    };
-    scores();
+        }
+    }
     // ---- the reference moves when a score exceeds it by more than 2^kRebase, or on the query's first
     // tile with a finite score (fresh: the reference becomes the tile maximum); as in flash_kernel,
     // the same in the query's two lanes
     {
       float mx[QT];
-      auto row_max = [&]() {
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) mx[qt] = col_max(__builtin_fmaxf(half_max(s[0][qt]), half_max(s[1][qt])));
-      };
-      row_max();
+      for (int qt = 0; qt < QT; ++qt) mx[qt] = col_max(__builtin_fmaxf(half_max(s[0][qt]), half_max(s[1][qt])));
       bool need = false;
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) need |= (mx[qt] > kRebase) || fresh[qt];
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) != 0, 0)) {
-        bool any_far = false, far[QT];
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-          far[qt] = (mx[qt] > kRescore) && !fresh[qt];
-          any_far |= far[qt];
-        }
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_far) != 0, 0)) {
-#pragma unroll
-          for (int qt = 0; qt < QT; ++qt) {
-            m_ref[qt] = far[qt] ? 0.f : m_ref[qt];
-            fresh[qt] |= far[qt];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) minit[qt][r] = -m_ref[qt];
-          }
-          scores();
-          row_max();
-        }
+      for (int qt = 0; qt < QT; ++qt) need |= (mx[qt] > kRebase) || m_low[qt] != 0.f || fresh[qt];
+      if (__builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           const bool seen = mx[qt] > -INFINITY;
-          const float shift = fresh[qt] ? (seen ? mx[qt] : 0.f) : fmaxf(mx[qt], 0.f);
-          const float alpha = far[qt] ? 0.f : (fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(-shift));
+          const float shift = fresh[qt] ? (seen ? mx[qt] : 0.f) : fmaxf(mx[qt], m_low[qt]);
+          const float alpha = fresh[qt] ? 1.f : __builtin_amdgcn_exp2f(m_low[qt] - shift);
           fresh[qt] = fresh[qt] && !seen;
-          m_ref[qt] += shift;
+          const float ref = m_ref[qt] + shift;
+          m_ref[qt] = fmaxf(ref, -kLowRef);
+          m_low[qt] = ref - m_ref[qt];
           l_run[qt] *= alpha;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
