@@ -86,13 +86,10 @@ __device__ __forceinline__ half8_t u8x8_to_h8(uint2 w) {
 
 // One output: (acc * alpha) * rs + bi, activation, then store or add into the residual `old`
 // (gated by gt) in the reference's order (app/gpu/gemm.js:159-164).
-// Activation: compile-time for the launches the model makes, else by the argument.
-constexpr int kActAny = -1;  // chosen by the argument at run time
-
 template <int ACT>
-__device__ __forceinline__ float act_t(float x, int act) {
-  if (ACT == kActAny) return apply_act(x, act);
+__device__ __forceinline__ float act_t(float x) {
   if (ACT == NS2_ACT_SILU) return silu(x);
+  if (ACT == NS2_ACT_GELU_TANH) return gelu_tanh(x);
   return x;
 }
 
@@ -101,12 +98,12 @@ __device__ __forceinline__ float act_t(float x, int act) {
 // third of the epilogue's vector instructions; 3952 x 8192 x 1536: 102.6 -> 101.0 us, the uncorrected product 100.2). Compared with the division for
 // all 2^32 inputs: the same bits for every result above 1e-35, at most 1e-36 off below.
 template <int ACT>
-__device__ __forceinline__ float glu_act(float x, int act) {
+__device__ __forceinline__ float glu_act(float x) {
   if (ACT == NS2_ACT_SILU) {
     const float d = 1.0f + __expf(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
   }
-  return act_t<ACT>(x, act);
+  return act_t<ACT>(x);
 }
 
 // XCD-aware tile order: consecutive block ids go to different XCDs (round-robin dispatch);
@@ -216,7 +213,7 @@ __device__ __forceinline__ void store_plain(const TGemmArgs& p, const float16_t 
       x *= rs[j];
       x += bi[j];
       if constexpr (LORA) x += d[r];
-      x = act_t<ACT>(x, p.act);
+      x = act_t<ACT>(x);
       if (RM) x = (PRE_C ? cold[PRE_C ? i : 0][PRE_C ? j : 0][r] : old[t & 1][LOAD_OLD ? r : 0]) + gt[j] * x;
       v[r] = x;
       if (LORA || RM) pin(v[r]);
@@ -276,7 +273,7 @@ __device__ __forceinline__ void store_vpack(const TGemmArgs& p, const float16_t 
           x *= rs[j];
           x += bi[j];
           if constexpr (LORA) x += d[8 * g + e];
-          v[e] = act_t<ACT>(x, p.act);
+          v[e] = act_t<ACT>(x);
           // the fp32 value first, as the plain store writes it: the conversion must not fuse
           // with the multiply-add into one rounding to fp16 (v_fma_mix)
           pin(v[e]);
@@ -615,7 +612,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
               float h1 = acc[i][2 * jj][r] * p.alpha;
               h1 *= s1;
               h1 += b1;
-              T[row * 256 + gc] = glu_act<ACT>(h1 + d1[r], p.act);
+              T[row * 256 + gc] = glu_act<ACT>(h1 + d1[r]);
             }
             const float16_t d2 = lora_tile(p.lt, p.lb, p.lr, m, I + G, hi);
 #pragma unroll
@@ -637,7 +634,7 @@ void gemm_tiled_kernel(TGemmArgs p) {
               float h2 = acc[i][2 * jj + 1][r] * p.alpha;
               h2 *= s2;
               h2 += b2;
-              T[row * 256 + gc] = glu_act<ACT>(h1, p.act) * h2;
+              T[row * 256 + gc] = glu_act<ACT>(h1) * h2;
             }
           }
         }
@@ -734,8 +731,11 @@ int launch_splitk_reduce(const TGemmArgs& p, int splits);
 // Weight bytes per column band of the tile order: half of an XCD's 4 MB L2.
 constexpr long long kBandBytes = 2ll << 20;
 
-template <int BM, int BN, int WM, int WN, int KG, int KT, int STAGES, int SPREAD, int WPE, int EPI = 0, Ops OPS = kI8, bool RESID = true,
-          bool LORA = true, bool ANY_ACT = false>
+// What a block tile has kernels for, beside plain launches: old outputs (C +=), the LoRA term, both, and the
+// activations (one kernel each) of those.
+enum Forms : unsigned { kPlain = 0, kResid = 1, kLora = 2, kResidLora = 4, kAct = 8 };
+
+template <int BM, int BN, int WM, int WN, int KG, int KT, int STAGES, int SPREAD, int WPE, Ops OPS, unsigned FORMS, int EPI = 0>
 int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -760,29 +760,37 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
   }
   const dim3 grid(p.tiles_m * p.tiles_n, splits), block(WM * WN * KG * 64);
   hipStream_t s = ns2::stream();
+  using std::integral_constant;
+  // a form without a kernel is not picked (linear_tiled)
+  bool ran = false;
   auto run = [&](auto act_c, auto rm_c) {
     constexpr int A = decltype(act_c)::value, R = decltype(rm_c)::value;
-    if constexpr (LORA) {
+    if constexpr ((FORMS & (R ? kResidLora : kLora)) != 0) {
       if (p.lr) {
         gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, true, OPS, WPE><<<grid, block, 0, s>>>(p);
-        return;
+        ran = true;
       }
     }
-    gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, false, OPS, WPE><<<grid, block, 0, s>>>(p);
-  };
-  using std::integral_constant;
-  if constexpr (EPI == 1) {
-    if (p.act == NS2_ACT_SILU) run(integral_constant<int, NS2_ACT_SILU>{}, integral_constant<int, 0>{});
-    else run(integral_constant<int, kActAny>{}, integral_constant<int, 0>{});
-  } else if (p.act == NS2_ACT_NONE) {
-    if constexpr (RESID) {
-      if (p.resid) run(integral_constant<int, NS2_ACT_NONE>{}, integral_constant<int, 1>{});
+    if constexpr (!R || (FORMS & kResid)) {
+      if (!p.lr) {
+        gemm_tiled_kernel<BM, BN, WM, WN, KG, KT, STAGES, SPREAD, EPI, A, R, false, OPS, WPE><<<grid, block, 0, s>>>(p);
+        ran = true;
+      }
     }
-    if (!p.resid) run(integral_constant<int, NS2_ACT_NONE>{}, integral_constant<int, 0>{});
-  } else if constexpr (ANY_ACT) {
-    if (p.resid) run(integral_constant<int, kActAny>{}, integral_constant<int, 1>{});
-    else run(integral_constant<int, kActAny>{}, integral_constant<int, 0>{});
+  };
+  auto run_act = [&](auto act_c) {
+    if constexpr (EPI == 0 && (FORMS & kResid)) {
+      if (p.resid) return run(act_c, integral_constant<int, 1>{});
+    }
+    if (!p.resid) run(act_c, integral_constant<int, 0>{});
+  };
+  if (p.act == NS2_ACT_NONE) {
+    run_act(integral_constant<int, NS2_ACT_NONE>{});
+  } else if constexpr (EPI == 1 || (FORMS & kAct)) {
+    if (p.act == NS2_ACT_SILU) run_act(integral_constant<int, NS2_ACT_SILU>{});
+    else run_act(integral_constant<int, NS2_ACT_GELU_TANH>{});
   }
+  if (!ran) return ns2::set_error(NS2_ERR_INVALID, "gemm_tiled: a block tile without a kernel for the call");
   NS2_LAUNCHED("gemm_tiled");
   if (p.part && reduce) return launch_splitk_reduce(p, splits);
   return NS2_OK;
@@ -792,26 +800,54 @@ int launch_tiled(TGemmArgs p, int splits = 1, bool reduce = true) {
 // one instantiation per operand kind, each compiled in a file of its own.
 enum Tile { T64x64, T64x128K2, T64x128K2S3, T64x128, T128x128, T128x192, T128x192K2, T192x384, T256x256, kTiles };
 
-// Launches block tile t; the tiles that OPS has no kernel for are not picked.
+// The forms of each tile. Each activation has its own kernels, although none of the models' tiled linears
+// has one: chosen at run time it cost small launches 2 us (33 x 64 x 1536 with SiLU: 7.2 -> 9.3) and spilled on the
+// largest tiles. 192x384 gains over the other tiles by 4 % at most with old outputs or a LoRA,
+// so it is plain only; 128x128 has no registers for old outputs beside the LoRA term at three blocks
+// per CU; fp16 weights have the six tiles that any launch gains from.
+constexpr unsigned kNotBuilt = ~0u;
+template <Ops OPS>
+constexpr unsigned tile_forms(Tile t) {
+  if (OPS == kF16 && (t == T64x128K2 || t == T128x192K2 || t == T192x384)) return kNotBuilt;
+  return t == T192x384 ? kPlain : t == T128x128 ? kResid | kLora | kAct : kResid | kLora | kResidLora | kAct;
+}
+
+// The tiles with a kernel for the call, bit t for tile t.
+template <Ops OPS>
+inline unsigned allowed_tiles(int act, int resid, int lora_r) {
+  unsigned m = 0;
+  for (int t = 0; t < kTiles; ++t) {
+    const unsigned f = tile_forms<OPS>((Tile)t);
+    if (f == kNotBuilt) continue;
+    const unsigned need = (act != NS2_ACT_NONE ? kAct : 0u) | (resid ? kResid : 0u) | (lora_r ? kLora : 0u) |
+                          (resid && lora_r ? kResidLora : 0u);
+    if ((f & need) == need) m |= 1u << t;
+  }
+  return m;
+}
+
 template <Ops OPS>
 int launch_tile(Tile t, const TGemmArgs& p, int splits) {
   if constexpr (OPS == kF16) {
     switch (t) {
-      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 1, 3, 1, 2, 0, OPS, true, true, true>(p, splits);
-      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 3, 0, OPS, true, true, true>(p);
-      default: return launch_tiled<128, 192, 2, 2, 2, 1, 2, 1, 2, 0, OPS>(p);
+      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 1, 3, 1, 2, OPS, tile_forms<OPS>(T64x64)>(p, splits);
+      case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 1, 3, 1, 2, OPS, tile_forms<OPS>(T64x128K2S3)>(p);
+      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 3, OPS, tile_forms<OPS>(T64x128)>(p);
+      case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 2, OPS, tile_forms<OPS>(T128x128)>(p);
+      case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2, OPS, tile_forms<OPS>(T128x192)>(p);
+      default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, OPS, tile_forms<OPS>(T256x256)>(p);
     }
   } else {
     switch (t) {
-      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, 0, OPS, true, true, true>(p, splits);
-      case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4, 0, OPS>(p);
-      case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 2, 3, 1, 2, 0, OPS>(p);
-      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, 0, OPS, true, true, true>(p);
-      case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, 0, OPS, false>(p);
-      case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2, 0, OPS>(p);
-      case T128x192K2: return launch_tiled<128, 192, 2, 2, 2, 2, 2, 2, 2, 0, OPS>(p);
-      case T192x384: return launch_tiled<192, 384, 2, 4, 1, 1, 2, 2, 2, 0, OPS, false, false>(p);
-      default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, 0, OPS, false, false>(p);
+      case T64x64: return launch_tiled<64, 64, 1, 2, 2, 2, 3, 1, 2, OPS, tile_forms<OPS>(T64x64)>(p, splits);
+      case T64x128K2: return launch_tiled<64, 128, 1, 4, 2, 2, 2, 1, 4, OPS, tile_forms<OPS>(T64x128K2)>(p);
+      case T64x128K2S3: return launch_tiled<64, 128, 1, 4, 2, 2, 3, 1, 2, OPS, tile_forms<OPS>(T64x128K2S3)>(p);
+      case T64x128: return launch_tiled<64, 128, 1, 4, 1, 1, 2, 1, 4, OPS, tile_forms<OPS>(T64x128)>(p);
+      case T128x128: return launch_tiled<128, 128, 2, 2, 1, 1, 2, 1, 3, OPS, tile_forms<OPS>(T128x128)>(p);
+      case T128x192: return launch_tiled<128, 192, 2, 2, 1, 1, 2, 2, 2, OPS, tile_forms<OPS>(T128x192)>(p);
+      case T128x192K2: return launch_tiled<128, 192, 2, 2, 2, 2, 2, 2, 2, OPS, tile_forms<OPS>(T128x192K2)>(p);
+      case T192x384: return launch_tiled<192, 384, 2, 4, 1, 1, 2, 2, 2, OPS, tile_forms<OPS>(T192x384)>(p);
+      default: return launch_tiled<256, 256, 2, 4, 1, 1, 2, 2, 2, OPS, tile_forms<OPS>(T256x256)>(p);
     }
   }
 }

@@ -8,7 +8,7 @@ using namespace ns2tiled;
 namespace {
 
 // The splits of a split-K launch summed in z order (deterministic), then the plain epilogue of
-// store_plain (scale, bias, the LoRA term, activation, store / += / += gate times).
+// store_plain (scale, bias, activation, store / += / += gate times).
 __global__ __launch_bounds__(256) void tiled_splitk_reduce_kernel(TGemmArgs p, int splits) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   const long long mn = (long long)p.M * p.N;
@@ -19,55 +19,12 @@ __global__ __launch_bounds__(256) void tiled_splitk_reduce_kernel(TGemmArgs p, i
   float v = acc * p.alpha;
   if (p.scale) v *= p.scale[n];
   v += p.bias ? p.bias[n] : 0.0f;
-  if (p.lr) v += lora_dot(p.lt, p.lb, p.lr, m, n);
   if (p.act == NS2_ACT_SILU) v = silu(v);
   else if (p.act == NS2_ACT_GELU_TANH) v = gelu_tanh(v);
   float* c = p.C + p.cOff + (long long)m * p.ldc + n;
   if (!p.resid) *c = v;
   else if (!p.gate) *c = *c + v;
   else *c = *c + p.gate[p.gOff + n] * v;
-}
-
-// The same for launches with a LoRA term, one wave per 32x32 output tile: the lane sums the
-// splits of its 16 elements (the v_mfma_f32_32x32x16_f16 accumulator layout, rows 8(r/4) +
-// 4hi + r%4 of the tile, column lq), adds the tile's LoRA term on the matrix cores (lora_tile,
-// as the unsplit epilogues do) and applies the epilogue. An element-wise reduce would take the
-// LoRA term as R scalar products per element: 51.7 us for 256 x 3072 at rank 32.
-__global__ __launch_bounds__(256) void tiled_splitk_reduce_lora_kernel(TGemmArgs p, int splits) {
-  const int lane = threadIdx.x & 63, lq = lane & 31, hi = lane >> 5;
-  const int tn_count = p.N / 32;
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= ((p.M + 31) / 32) * tn_count) return;  // uniform per wave
-  const int m0 = (tile / tn_count) * 32, n = (tile % tn_count) * 32 + lq;
-  const long long mn = (long long)p.M * p.N;
-  float acc[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-    float a = 0.f;
-    if (m < p.M)
-      for (int z = 0; z < splits; ++z) a += p.part[z * mn + (long long)m * p.N + n];
-    acc[r] = a;
-  }
-  const int mrow = m0 + lq < p.M ? m0 + lq : p.M - 1;
-  const float16_t d = lora_tile(p.lt, p.lb, p.lr, mrow, n, hi);
-  const float rs = p.scale ? p.scale[n] : 1.0f;
-  const float bi = p.bias ? p.bias[n] : 0.0f;
-  const float gt = p.gate ? p.gate[p.gOff + n] : 1.0f;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-    if (m >= p.M) continue;
-    float v = acc[r] * p.alpha;
-    v *= rs;
-    v += bi;
-    v += d[r];
-    if (p.act == NS2_ACT_SILU) v = silu(v);
-    else if (p.act == NS2_ACT_GELU_TANH) v = gelu_tanh(v);
-    float* c = p.C + p.cOff + (long long)m * p.ldc + n;
-    if (!p.resid) *c = v;
-    else *c = *c + gt * v;
-  }
 }
 
 // W [N, K] row-major int8 -> Wt tiles [N/64][K/64][8 k-chunks of 8][64 rows][8 bytes] of biased
@@ -118,14 +75,8 @@ __global__ __launch_bounds__(256) void tile_w16_kernel(const uint16_t* __restric
 }  // namespace
 
 int ns2tiled::launch_splitk_reduce(const TGemmArgs& p, int splits) {
-  hipStream_t s = ns2::stream();
   const long long mn = (long long)p.M * p.N;
-  if (p.lr) {
-    const long long tiles32 = (long long)((p.M + 31) / 32) * (p.N / 32);
-    tiled_splitk_reduce_lora_kernel<<<(unsigned)((tiles32 + 3) / 4), 256, 0, s>>>(p, splits);
-  } else {
-    tiled_splitk_reduce_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, s>>>(p, splits);
-  }
+  tiled_splitk_reduce_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, ns2::stream()>>>(p, splits);
   NS2_LAUNCHED("gemm_tiled_splitk_reduce");
   return NS2_OK;
 }
@@ -134,10 +85,15 @@ namespace {
 
 // Block tiles and their time model: a launch gives every CU `per` = ceil(tiles / 256) tiles, run as
 // rounds of up to `occ` co-resident blocks; a round of n blocks per CU takes e[n-1] + c[n-1] us per
-// 64-wide k-tile, and a launch L us more. The constants are least-squares fits to 139 measured
-// launches per tile (23 row counts from 64 to 3952, N x K of 4608/6144/8192/27648 x 1536 and 1536 x
-// 1536/4096/6144, weights cycled through 8 copies); choosing by the model costs 1.1 % on average
-// against the best tile of each of those launches.
+// 64-wide k-tile, and a launch L us more. These are weights for ranking the tiles against each other, not
+// times: int8 rows were fitted to launches of 64-3952 rows x 1536-27648 x 1536-6144 with weights cycled through 8
+// copies (three stages: through 600 MB), fp16 rows to the tiles near the best of 396 launches of 33-8192 rows x
+// 64-16384 x 64-4096 (16 copies); two per CU of int8 128x192, fp16 128x192 and three per CU of fp16 64x64 were
+// raised by hand where they were picked too early. They know only the busiest CU and no clock, which
+// falls from 2.3 to 1.5 GHz as CUs fill up: one large tile per CU is put up to 26 % too low (3952 x 4608 x 1536:
+// 42.6 for 57.5 us; 3328: 39.9 for 49.6), fewer or smaller tiles within about 10 %. What counts is the pick: over 1254
+// measured launches of every tile (33-8192 rows, 19 shapes N x K; plain, C += and with a LoRA) it is 0.9 % off the
+// best on average and 60 % at most (8192 x 1024 x 256).
 //   64x64, 4 waves (2 k groups)   few tiles: each block's k chain halved, three 128-wide stages
 //   64x128, 8 waves (2 k groups)  two tiles per CU (1900 x 1536 x 1536 +=: 17.9 us)
 //   the same, three stages        one tile per CU: with the block alone on its CU, one k-tile ahead does not
@@ -152,22 +108,37 @@ namespace {
 //   192x384, 8 waves              one tile per CU (3952 x 4608 x 1536: 70.3 -> 57.5 us)
 //   256x256, 8 waves              one tile per CU (3328 x 4608 x 1536: 51.9 -> 49.6 us)
 struct TileCfg {
+  const char* name;
   int bm, bn, occ;
   float L, e[4], c[4];
 };
 constexpr TileCfg kCfgs[kTiles] = {
-    {64, 64, 2, 1.8f, {1.86f, 2.65f}, {0.210f, 0.322f}},
-    {64, 128, 2, 1.5f, {2.56f, 4.34f}, {0.398f, 0.474f}},
-    {64, 128, 1, 1.5f, {3.20f}, {0.263f}},
-    {64, 128, 4, 3.8f, {0.f, 1.49f, 3.17f, 0.f}, {0.413f, 0.510f, 0.731f, 1.147f}},
-    {128, 128, 3, 2.9f, {2.49f, 5.20f, 0.f}, {0.513f, 0.790f, 1.550f}},
-    {128, 192, 2, 0.9f, {5.77f, 0.f}, {0.696f, 1.497f}},
-    {128, 192, 1, 0.f, {8.83f}, {0.520f}},
-    {192, 384, 1, 0.f, {13.86f}, {1.199f}},
-    {256, 256, 1, 0.f, {12.80f}, {1.130f}},
+    {"64x64", 64, 64, 2, 1.8f, {1.86f, 2.65f}, {0.210f, 0.322f}},
+    {"64x128K2", 64, 128, 2, 1.5f, {2.56f, 4.34f}, {0.398f, 0.474f}},
+    {"64x128K2S3", 64, 128, 1, 1.5f, {3.20f}, {0.263f}},
+    {"64x128", 64, 128, 4, 3.8f, {0.f, 1.49f, 3.17f, 0.f}, {0.413f, 0.510f, 0.731f, 1.147f}},
+    {"128x128", 128, 128, 3, 2.9f, {2.49f, 5.20f, 0.f}, {0.513f, 0.790f, 1.550f}},
+    {"128x192", 128, 192, 2, 0.9f, {5.77f, 5.00f}, {0.696f, 1.289f}},
+    {"128x192K2", 128, 192, 1, 0.f, {8.83f}, {0.520f}},
+    {"192x384", 192, 384, 1, 0.f, {13.86f}, {1.199f}},
+    {"256x256", 256, 256, 1, 0.f, {12.80f}, {1.130f}},
+};
+constexpr TileCfg kCfgsF16[kTiles] = {
+    {"64x64", 64, 64, 3, 2.88f, {0.61f, 1.42f, 2.88f}, {0.245f, 0.384f, 0.520f}},
+    {},
+    {"64x128K2S3", 64, 128, 1, 2.63f, {1.68f}, {0.314f}},
+    {"64x128", 64, 128, 3, 3.33f, {0.55f, 1.94f, 3.85f}, {0.504f, 0.653f, 0.894f}},
+    {"128x128", 128, 128, 2, 1.05f, {4.13f, 6.69f}, {0.644f, 0.949f}},
+    {"128x192", 128, 192, 2, 1.44f, {5.86f, 10.11f}, {0.920f, 1.205f}},
+    {},
+    {},
+    {"256x256", 256, 256, 1, 0.f, {12.05f}, {1.605f}},
 };
 constexpr int kCUs = 256;
-constexpr float kReduceUs = 4.0f;  // the reduce launch of a split-K linear (2.4 us of it the launch)
+
+// The reduce launch of a split-K linear and its traffic (33 x 64 x 1536 in 3: 2.0 us, 33 x 1536 x 1536 in 3: 2.9, 120 x 1536 x 6144
+// in 3: 3.8, 256 x 1536 x 4096 in 2: 4.5).
+float reduce_time(int M, int N, int splits) { return 2.0f + 3e-6f * (float)M * (float)N * (float)splits; }
 
 // Modelled time of `tiles` block tiles of configuration t over kt k-tiles each.
 float tile_time(const TileCfg& t, long long tiles, int kt) {
@@ -183,18 +154,20 @@ long long tile_count(const TileCfg& t, int M, int N) {
 }
 
 // The tile of the least modelled time, and for 64x64 tiles how many ways K is split (over
-// blockIdx.y, reduced in a second launch; at least 8 k-tiles per split). `allowed`: bit t for tile t.
-Tile pick_tile(int M, int N, int K, unsigned allowed, bool can_split, int* splits) {
+// blockIdx.y, reduced in a second launch; at least 8 k-tiles per split). `allowed`: bit t for tile t. Only a
+// grid of up to kSplitTiles is split, over at least 16 k-tiles: the launches that take the scratch for it.
+constexpr long long kSplitTiles = 213;
+Tile pick_tile(const TileCfg* cfgs, int M, int N, int K, unsigned allowed, bool can_split, int* splits) {
   const int kt = K / 64;
   Tile best = T64x64;
   float best_us = 0;
   *splits = 0;
   for (int i = 0; i < kTiles; ++i) {
     if (!(allowed >> i & 1)) continue;
-    const long long tiles = tile_count(kCfgs[i], M, N);
-    const int most = i == T64x64 && can_split && tiles < kCUs ? (kt / 8 < 8 ? kt / 8 : 8) : 1;
+    const long long tiles = tile_count(cfgs[i], M, N);
+    const int most = i == T64x64 && can_split && tiles <= kSplitTiles ? (kt / 8 < 8 ? kt / 8 : 8) : 1;
     for (int s = 1; s <= (most > 1 ? most : 1); ++s) {
-      const float us = tile_time(kCfgs[i], tiles * s, (kt + s - 1) / s) + (s > 1 ? kReduceUs : 0.f);
+      const float us = tile_time(cfgs[i], tiles * s, (kt + s - 1) / s) + (s > 1 ? reduce_time(M, N, s) : 0.f);
       if (!*splits || us < best_us) {
         best = (Tile)i;
         best_us = us;
@@ -203,6 +176,22 @@ Tile pick_tile(int M, int N, int K, unsigned allowed, bool can_split, int* split
     }
   }
   return best;
+}
+
+// The block tile of a linear, and its K splits: whole 128-wide stages of int8 tiles; none with a LoRA,
+// whose term the reduce would have to add (256 x 1536 x 4096, rank 32: 51.5 us split, 39.6 unsplit), none where the
+// values are packed, none for row-major operands, which use no scratch.
+Tile plan_tile(Ops ops, int M, int N, int K, int act, int resid, int lora_r, bool packed, int* splits, int* ksplit) {
+  const unsigned allowed = ops == kF16 ? allowed_tiles<kF16>(act, resid, lora_r) : allowed_tiles<kI8>(act, resid, lora_r);
+  const Tile t = pick_tile(ops == kF16 ? kCfgsF16 : kCfgs, M, N, K, allowed, ops != kI8Rows && !packed && !lora_r, splits);
+  *ksplit = 0;
+  if (*splits > 1) {
+    const int kt = K / 64;
+    *ksplit = (kt + *splits - 1) / *splits;
+    if (ops != kF16) *ksplit += *ksplit & 1;
+    *splits = (kt + *ksplit - 1) / *ksplit;
+  }
+  return t;
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -236,22 +225,8 @@ int linear_tiled(const char* fn, Ops ops, const uint16_t* At, int lda, const voi
     p.lr = lora_r;
   }
   ns2::ProfScope prof_(ops == kF16 ? "gemm_f16_tiled" : ops == kI8 ? "gemm_i8_tiled" : "linear_i8");
-  // The tiles a launch may take: activations (none of the models' tiled linears has one) are built
-  // for the two small tiles; fp16 weights for three tiles of one 64-wide k-tile per stage; the two
-  // largest tiles have no registers left for old outputs or the LoRA term, 128x128 (three blocks
-  // per CU) none for old outputs.
-  unsigned allowed = (1u << kTiles) - 1;
-  if (act != NS2_ACT_NONE) allowed = 1u << T64x64 | 1u << T64x128;
-  else if (ops == kF16) allowed = 1u << T64x64 | 1u << T64x128 | 1u << T128x192K2;
-  else if (resid || lora_r) allowed &= ~(1u << T192x384 | 1u << T256x256 | (resid ? 1u << T128x128 : 0u));
   int splits;
-  const Tile tile = pick_tile(M, N, K, allowed, ops != kI8Rows && !vpk, &splits);
-  if (splits > 1) {
-    const int kt = K / 64;
-    p.ksplit = (kt + splits - 1) / splits;
-    if (ops != kF16) p.ksplit += p.ksplit & 1;  // whole 128-wide stages
-    splits = (kt + p.ksplit - 1) / p.ksplit;
-  }
+  const Tile tile = plan_tile(ops, M, N, K, act, resid, lora_r, vpk != nullptr, &splits, &p.ksplit);
   if (splits > 1) {
     p.part = static_cast<float*>(ns2::workspace(5, (size_t)splits * M * N * sizeof(float)));
     if (!p.part) return ns2::set_error(NS2_ERR_OOM, "%s: split-K workspace allocation failed", fn);
@@ -290,10 +265,18 @@ int ns2::linear_f16w_tiled_raw(const char* fn, const uint16_t* At, const uint16_
   *part = p.part;
   *splits = s;
   ns2::ProfScope prof_("gemm_f16_tiled");
-  return launch_tiled<64, 64, 2, 2, 1, 1, 3, 1, 2, 0, kF16, false, false>(p, s, false);
+  return launch_tiled<64, 64, 2, 2, 1, 1, 3, 1, 2, kF16, kPlain>(p, s, false);
 }
 
 extern "C" {
+
+// For tests, not part of the C ABI: the block tile and the K splits that a linear would be launched with
+// (ops: 0 int8 tiles, 1 fp16 tiles, 2 row-major operands). Host only.
+const char* ns2_internal_tile(int ops, int M, int N, int K, int act, int resid, int lora_r, int packed, int* splits) {
+  int ksplit;
+  const Tile t = plan_tile((Ops)ops, M, N, K, act, resid, lora_r, packed, splits, &ksplit);
+  return kCfgs[t].name;
+}
 
 int ns2_tile_i8_weight(const int8_t* W, int8_t* Wt, int N, int K) {
   NS2_READY();
@@ -349,10 +332,13 @@ int ns2_linear_i8_glu_rot_tiled_lora(const uint16_t* At, const int8_t* Wt, const
   // busiest CU gets an even number of 64-row tiles, that many halves as 128-row tiles are faster
   // (x 8192 x 1536, us 64 -> 128: 1100 rows 44.1 -> 38.7, 2048 53.0 -> 49.8, 3328 94.3 -> 88.9, 3952 101.6 ->
   // 96.8, 5200 143.3 -> 134.8); where it gets an odd number, a last pair's half would be padding
-  // (1024 29.0 -> 39.1, 2304 70.5 -> 83.5, 6200 166.9 -> 175.6).
+  // (1024 29.0 -> 39.1, 2304 70.5 -> 83.5, 6200 166.9 -> 175.6). A 64-row tile alone on its CU takes a third
+  // stage for a long K, whose weights come from memory too late otherwise (x 16384 x 4096, 33-512 rows: 77 -> 62
+  // us; x 8192 x 1536: 23.4 -> 24.1).
   const long long per = ((long long)p.mblocks * (N / 512) + kCUs - 1) / kCUs;
-  if (per % 2 == 0) return launch_tiled<128, 512, 1, 8, 1, 1, 2, 2, 2, 1>(p);
-  return launch_tiled<64, 512, 1, 8, 1, 1, 2, 1, 4, 1>(p);
+  if (per == 1 && K > 2048) return launch_tiled<64, 512, 1, 8, 1, 1, 3, 1, 2, kI8, kLora, 1>(p);
+  if (per % 2 == 0) return launch_tiled<128, 512, 1, 8, 1, 1, 2, 2, 2, kI8, kLora, 1>(p);
+  return launch_tiled<64, 512, 1, 8, 1, 1, 2, 1, 4, kI8, kLora, 1>(p);
 }
 
 int ns2_linear_i8_tiled(const uint16_t* At, const int8_t* Wt, const float* scale, const float* bias,

@@ -1,12 +1,13 @@
 """The block tiles of the tiled int8 / fp16 linears at their edges: ragged last rows and columns, the
-shortest K, split K, old outputs, the LoRA term and the packed values, each at a size whose launch
-takes the named tile (the time model of ns2_gemm_tiled.hip).
+shortest K, split K, old outputs, the LoRA term, the activations and the packed values, each at a size whose
+launch takes the named tile (asked of the library, which chooses it by a time model).
 
 The operands are given (fp16 activations, int8 weights), so the reference is the same product in
 float64 and the only error is that of fp32 sums: the K products of an output are added in fp32, a
 random walk of at most sqrt(K) 2^-24 of the result's size (4.7e-6 at K = 6144).
 """
 
+import ctypes
 import math
 
 import pytest
@@ -24,40 +25,58 @@ def tiled(x):
     return p.reshape(-1, 64, K // 64, 8, 8).permute(0, 2, 3, 1, 4).contiguous()
 
 
+def tile_of(lib, ops, M, N, K, act="none", resid=False, rank=0, packed=False):
+    """The block tile and K splits of a linear; ops: 0 int8 tiles, 1 fp16 tiles, 2 row-major operands."""
+    fn, splits = lib.dll.ns2_internal_tile, ctypes.c_int()
+    fn.restype = ctypes.c_char_p
+    name = fn(ops, M, N, K, {"none": 0, "silu": 1, "gelu_tanh": 2}[act], int(resid), rank, int(packed), ctypes.byref(splits))
+    return name.decode(), splits.value
+
+
 def close(got, ref, K, what):
     rel = ((got.double() - ref).norm() / ref.norm()).item()
     print(f"[parity] {what}: rel-L2 {rel:.2e}", flush=True)
     assert torch.isfinite(got).all() and rel <= math.sqrt(K) * 2.0**-24, what
 
 
+def assert_tile(lib, tile, ops, M, N, K, **form):
+    name, splits = tile_of(lib, ops, M, N, K, **form)
+    assert name == tile.split()[0] and (splits > 1) == ("split" in tile), (name, splits)
+
+
 CASES = [
-    # tile, M, N, K, resid, LoRA rank
+    # tile, M, N, K, resid, LoRA rank; K2: two k groups, S3: three stages
     ("64x64", 33, 1536, 256, False, 0),
     ("64x64 split K", 65, 1536, 4096, True, 0),
-    ("64x64 split K", 120, 1536, 6144, False, 32),
+    ("64x64", 120, 1536, 6144, False, 32),
+    ("64x64 split K", 120, 1536, 6144, False, 0),
     ("64x64", 64, 64, 1536, True, 32),
-    ("64x128, two k groups", 1501, 1536, 1536, True, 0),
-    ("64x128, two k groups", 1460, 1536, 1536, False, 32),
-    ("64x128, two k groups, three stages", 1025, 1536, 1536, True, 0),
-    ("64x128, two k groups, three stages", 999, 1536, 1536, False, 32),
-    ("64x128, two k groups, three stages", 1000, 1472, 1536, False, 0),
-    ("64x128", 511, 4672, 1536, False, 0),
-    ("64x128", 513, 4672, 1536, True, 32),
+    ("64x128K2", 1501, 1536, 1536, True, 0),
+    ("64x128K2", 1460, 1536, 1536, False, 32),
+    ("64x128K2S3", 1025, 1536, 1536, True, 0),
+    ("64x128K2S3", 999, 1536, 1536, False, 32),
+    ("64x128K2S3", 1000, 1472, 1536, False, 0),
+    ("64x128K2", 511, 4672, 1536, False, 0),
+    ("64x128K2", 513, 4672, 1536, True, 32),
+    ("64x128", 257, 4608, 256, False, 0),
+    ("64x128", 257, 4608, 256, True, 32),
     ("128x128", 1537, 4672, 1536, False, 0),
     ("128x128", 1800, 4608, 256, False, 32),
     ("128x192", 2305, 4672, 1536, False, 0),
     ("128x192", 2433, 4608, 1536, True, 32),
-    ("128x192, two k groups", 3951, 1536, 4096, True, 0),
-    ("128x192, two k groups", 2867, 1600, 6144, False, 32),
-    ("192x384", 3951, 4672, 1536, False, 0),
-    ("192x384", 3800, 4608, 256, False, 0),
-    ("256x256", 3329, 4672, 1536, False, 0),
+    ("128x192K2", 3951, 1536, 4096, True, 0),
+    ("128x192K2", 2867, 1600, 6144, False, 32),
+    ("128x128", 3951, 4672, 1536, False, 0),
+    ("64x128", 3800, 4608, 256, False, 0),
+    ("192x384", 3329, 4672, 1536, False, 0),
+    ("256x256", 1501, 8256, 512, False, 0),
 ]
 
 
 @pytest.mark.parametrize("tile,M,N,K,resid,rank", CASES)
 def test_i8_tiles(ns2lib, tile, M, N, K, resid, rank):
     print(f"[case] {tile} {M}x{N}x{K} resid {resid} rank {rank}", flush=True)
+    assert_tile(ns2lib, tile, 0, M, N, K, resid=resid, rank=rank)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     x = torch.randn(M, K, generator=g, device=DEV).half()
     q = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
@@ -112,9 +131,10 @@ def test_rows_far_apart(ns2lib, M, N, K):
 
 
 @pytest.mark.parametrize("tile,M,N,K,resid", [("64x64", 70, 64, 64, False), ("64x64 split K", 65, 1536, 1600, True),
-                                              ("64x128", 1000, 1536, 64, False), ("128x192", 3951, 1600, 1536, True)])
+                                              ("64x128", 1000, 1536, 64, False), ("128x128", 3951, 1600, 1536, True)])
 def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
     print(f"[case] {tile} {M}x{N}x{K} resid {resid}", flush=True)
+    assert_tile(ns2lib, tile, 1, M, N, K, resid=resid)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     x = torch.randn(M, K, generator=g, device=DEV).half()
     w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
@@ -129,12 +149,12 @@ def test_f16w_tiles(ns2lib, tile, M, N, K, resid):
     close(buf[:M], before[:M].double() + ref if resid else ref, max(K, 1024), f"{tile} {M}x{N}x{K}")
 
 
-# both sides of the rule that takes file-layout operands to the block tiles: rows, work, 64-row weight blocks
-# ("tiled" 3953x64x4096 has too few tiles and 8193x64x4096 enough)
+# both sides of the rule that takes file-layout operands to the block tiles: rows, work, 64-row weight blocks,
+# the number of tiles
 @pytest.mark.parametrize("route,M,N,K,resid,rank,act", [
     ("tiled", 400, 2560, 1024, True, 0, "none"), ("rows", 399, 2560, 1024, True, 0, "none"),
     ("tiled", 1001, 1600, 768, False, 32, "none"), ("rows", 1001, 1616, 768, False, 32, "none"),
-    ("tiled", 3953, 64, 4096, True, 0, "silu"), ("rows", 3953, 64, 3840, True, 0, "silu"),
+    ("rows", 3953, 64, 4096, True, 0, "silu"), ("rows", 3953, 64, 3840, True, 0, "silu"),
     ("tiled", 8193, 64, 4096, True, 0, "silu"), ("tiled", 2500, 4608, 1536, False, 0, "none"),
     ("tiled", 3953, 1536, 1536, False, 0, "none"), ("tiled", 1025, 1536, 1536, True, 0, "none"),
 ])
@@ -248,9 +268,82 @@ def test_i8_activation(ns2lib, M, act):
     close(y, ref, 1024, act)
 
 
+# a size per operand kind at which every form a tile is built for takes it
+SIZES = {
+    0: {"64x64": (65, 192, 768), "64x128K2": (777, 2624, 1536), "64x128K2S3": (65, 8256, 512), "64x128": (257, 4608, 256),
+        "128x128": (1801, 4608, 256), "128x192": (2867, 1536, 256), "128x192K2": (1537, 2624, 1536), "192x384": (3329, 4672, 1536),
+        "256x256": (1501, 8256, 512)},
+    1: {"64x64": (65, 192, 768), "64x128K2S3": (65, 8256, 512), "64x128": (999, 4160, 256), "128x128": (1460, 1536, 256),
+        "128x192": (2305, 4608, 256), "256x256": (2867, 4608, 256)},
+    2: {"64x64": (511, 1536, 1536), "64x128K2": (777, 2560, 1024), "64x128K2S3": (401, 2560, 1024), "64x128": (511, 4672, 512),
+        "128x128": (999, 8256, 512), "128x192": (511, 8256, 512), "128x192K2": (1801, 2560, 1024), "192x384": (3329, 4672, 1536),
+        "256x256": (1501, 8256, 512)},
+}
+FORMS = [("none", False, 0), ("none", True, 0), ("none", False, 64), ("none", True, 32), ("silu", False, 0), ("gelu_tanh", True, 0),
+         ("gelu_tanh", False, 32), ("silu", True, 32)]
+
+
+@pytest.mark.parametrize("ops,tile", [(o, t) for o in SIZES for t in SIZES[o]])
+@pytest.mark.parametrize("act,resid,rank", FORMS)
+def test_tile_forms(ns2lib, ops, tile, act, resid, rank):
+    """Every kernel of every block tile: old outputs, the LoRA term, the activations and what combines them,
+    a column window of a wider output, with fp16-exact operands. Beside the fp32 sums the activation is off
+    by a few ulp (__expf and the quotient: 2^-21 of a value), and t of the LoRA may round to the other fp16
+    neighbour in few places (2^-12 of the result)."""
+    M, N, K = SIZES[ops][tile]
+    if tile == "192x384" and (act, resid, rank) != ("none", False, 0) or tile == "128x128" and resid and rank:
+        assert tile_of(ns2lib, ops, M, N, K, act, resid, rank)[0] != tile
+        return
+    print(f"[case] ops {ops} {tile} {M}x{N}x{K} {act} resid {resid} rank {rank}", flush=True)
+    assert_tile(ns2lib, tile, ops, M, N, K, act=act, resid=resid, rank=rank)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K + rank)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    bias, gate = torch.randn(N, generator=g, device=DEV), torch.randn(N, generator=g, device=DEV)
+    if ops == 1:
+        w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+        ref = x.double() @ w.half().double().T
+    else:
+        w = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+        s = (torch.rand(N, generator=g, device=DEV) + 0.5) / (73 * math.sqrt(K))
+        ref = (x.double() @ w.double().T) * s.double()
+    ref = ref + bias.double()
+    lora = None
+    if rank:
+        a = (torch.randn(rank, K, generator=g, device=DEV) / math.sqrt(K)).half()
+        b = (torch.randn(N, rank, generator=g, device=DEV) / math.sqrt(rank)).half()
+        lora = (a, b, rank)
+        ref = ref + (x.double() @ a.double().T).half().double() @ b.double().T
+    if act != "none":
+        ref = torch.nn.functional.silu(ref) if act == "silu" else torch.nn.functional.gelu(ref, approximate="tanh")
+    ldc = N + 32
+    buf = torch.randn(M + 300, ldc, generator=g, device=DEV)
+    before = buf.clone()
+    if resid:
+        ref = before[:M, 32:].double() + gate.double() * ref
+    kw = dict(bias=bias, act=act, resid=resid, gate=gate if resid else None, lora=lora, ldc=ldc, cOff=32)
+    if ops == 2:
+        ns2lib.linear_i8(x, 1, K, w, s, buf, M, N, K, **kw)
+    else:
+        wt = torch.empty_like(w)
+        if ops == 1:
+            ns2lib.tile_bf16_weight(w, wt, N, K)
+            ns2lib.linear_f16w_tiled(tiled(x), wt, buf, M, N, K, **kw)
+        else:
+            ns2lib.tile_i8_weight(w, wt, N, K)
+            ns2lib.linear_i8_tiled(tiled(x), wt, s, buf, M, N, K, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(buf[M:], before[M:]) and torch.equal(buf[:, :32], before[:, :32]), "values outside the window were written"
+    got = buf[:M, 32:]
+    rel = ((got.double() - ref).norm() / ref.norm()).item()
+    tol = math.sqrt(max(K, 1024)) * 2.0**-24 + (2.0**-21 if act != "none" else 0) + (2.0**-12 if rank else 0)
+    print(f"[parity] ops {ops} {tile}: rel-L2 {rel:.2e} (tol {tol:.1e})", flush=True)
+    assert torch.isfinite(got).all() and rel <= tol
+
+
 # 1030: 17 row blocks of 64, so the last 128-row tile holds one real block; 1090: a ragged second one
 @pytest.mark.parametrize("tile,M,N,K,rank", [("128x512", 1030, 8192, 256, 0), ("128x512", 1090, 8192, 1536, 32),
-                                             ("64x512", 1024, 8192, 256, 0), ("64x512", 2100, 8192, 256, 32)])
+                                             ("64x512", 1024, 8192, 256, 0), ("64x512", 2100, 8192, 256, 32),
+                                             ("64x512S3", 70, 1024, 2304, 0), ("64x512S3", 401, 2048, 4096, 32)])
 def test_glu_tiles(ns2lib, tile, M, N, K, rank):
     """The GLU + rotation epilogue's block tiles: one fp16 rounding of the result (2^-11 of a value at
     most), with a LoRA the rounding of its down-projection too; rows past the last row block stay."""
@@ -336,7 +429,6 @@ def test_vpack_tiles(ns2lib, M, N, K, H, HD):
     assert torch.equal(y[:, :vcol0], plain[:, :vcol0])
     # [head][tile][chunk][dim][8]: chunk 2g + hi holds keys 16g + 4hi + {0..3}, 16g + 8 + 4hi + {0..3}
     v = vpk.reshape(H, tiles, 4, 2, HD, 2, 4).permute(1, 2, 5, 3, 6, 0, 4).reshape(tiles * 64, H * HD)
-    # no K split with packed values, so where the plain launch splits K the sums differ in association
-    if torch.equal(v[:M], plain[:, vcol0:].half()):
-        return
-    close(v[:M].float(), plain[:, vcol0:].double(), 2.0**26, "packed values")  # fp16: 2^-11
+    # both launches take the same tile, and neither splits K
+    assert tile_of(ns2lib, 0, M, N, K) == tile_of(ns2lib, 0, M, N, K, packed=True)
+    assert torch.equal(v[:M], plain[:, vcol0:].half())
