@@ -95,8 +95,9 @@ __device__ __forceinline__ float act_t(float x) {
 
 // The GLU epilogue's gate activation. SiLU's quotient as the reciprocal's, corrected once by its residual
 // (5 instructions; the division's scaling steps for quotients out of range make it 10, which were a
-// third of the epilogue's vector instructions; 3952 x 8192 x 1536: 102.6 -> 101.0 us, the uncorrected product 100.2). Compared with the division for
-// all 2^32 inputs: the same bits for every result above 1e-35, at most 1e-36 off below.
+// third of the epilogue's vector instructions; 3952 x 8192 x 1536: 102.6 -> 101.0 us, the uncorrected
+// product 100.2). Compared with the division for all 2^32 inputs: the same bits for every result above
+// 1e-35, at most 1e-36 off below.
 template <int ACT>
 __device__ __forceinline__ float glu_act(float x) {
   if (ACT == NS2_ACT_SILU) {

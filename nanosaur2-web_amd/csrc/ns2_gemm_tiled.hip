@@ -179,7 +179,7 @@ Tile pick_tile(const TileCfg* cfgs, int M, int N, int K, unsigned allowed, bool 
 }
 
 // The block tile of a linear, and its K splits: whole 128-wide stages of int8 tiles; none with a LoRA,
-// whose term the reduce would have to add (256 x 1536 x 4096, rank 32: 51.5 us split, 39.6 unsplit), none where the
+// whose term the reduce would have to add (256 x 1536 x 4096, rank 32: 51.5 us split, 27.6 unsplit), none where the
 // values are packed, none for row-major operands, which use no scratch.
 Tile plan_tile(Ops ops, int M, int N, int K, int act, int resid, int lora_r, bool packed, int* splits, int* ksplit) {
   const unsigned allowed = ops == kF16 ? allowed_tiles<kF16>(act, resid, lora_r) : allowed_tiles<kI8>(act, resid, lora_r);
@@ -333,8 +333,8 @@ int ns2_linear_i8_glu_rot_tiled_lora(const uint16_t* At, const int8_t* Wt, const
   // (x 8192 x 1536, us 64 -> 128: 1100 rows 44.1 -> 38.7, 2048 53.0 -> 49.8, 3328 94.3 -> 88.9, 3952 101.6 ->
   // 96.8, 5200 143.3 -> 134.8); where it gets an odd number, a last pair's half would be padding
   // (1024 29.0 -> 39.1, 2304 70.5 -> 83.5, 6200 166.9 -> 175.6). A 64-row tile alone on its CU takes a third
-  // stage for a long K, whose weights come from memory too late otherwise (x 16384 x 4096, 33-512 rows: 77 -> 62
-  // us; x 8192 x 1536: 23.4 -> 24.1).
+  // stage for a long K, whose weights come from memory too late otherwise (x 16384 x 4096, 33-512 rows: 77 ->
+  // 58-60 us; x 8192 x 1536: 23.4 -> 24.1).
   const long long per = ((long long)p.mblocks * (N / 512) + kCUs - 1) / kCUs;
   if (per == 1 && K > 2048) return launch_tiled<64, 512, 1, 8, 1, 1, 3, 1, 2, kI8, kLora, 1>(p);
   if (per % 2 == 0) return launch_tiled<128, 512, 1, 8, 1, 1, 2, 2, 2, kI8, kLora, 1>(p);

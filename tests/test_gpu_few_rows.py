@@ -1,6 +1,7 @@
 """The one-launch linears of a short sequence (q|k|v with head norms, gate/up with GLU and down shares) at
-their edges: row tiles with and without rows, two row tiles per block, chunks of one and five k-tiles,
-the largest K their LDS holds and the calls beyond, which keep the two-launch path.
+their edges: row tiles with and without rows, two row tiles per block, chunks of one and five k-tiles, both
+sides of the rules that choose between one launch and two (which of them ran is read back), the largest weight
+slice of one launch, outputs that overlap the rows or the weights.
 
 The operands are fp16 and given, the reference is float64: fp32 sums of K products are off by at most
 sqrt(K) 2^-24 of the result's size (a random walk), values rounded to fp16 by 2^-11 of theirs.
