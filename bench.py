@@ -66,10 +66,10 @@ CFG1_SHAPES = (("qkv", 4608, 1536), ("proj", 1536, 1536), ("up", 6144, 1536), ("
 # the algorithmic bytes of the same launches: the mean over one pass's 73 tiled-GEMM launches on the
 # 3952 image rows (18 each of qkv and w12+GLU, 36 of proj and w3, the stacked kv_y), and one flash
 # launch at 3952x4208 batch 2. The source files hold the per-kernel tables and the commands.
-GEMM_TRAFFIC_BYTES_PER_LAUNCH = 123.2e6
+GEMM_TRAFFIC_BYTES_PER_LAUNCH = 123.1e6
 GEMM_ALGORITHMIC_BYTES_PER_LAUNCH = 71.9e6   # N*K int8 W + 2*M*K fp16 A + output (+ old output for +=)
 GEMM_TRAFFIC_SOURCE = "profiles/dit_pass_832x1216_int8.md"
-ATTN_TRAFFIC_BYTES_PER_LAUNCH = 170.0e6
+ATTN_TRAFFIC_BYTES_PER_LAUNCH = 169.7e6
 ATTN_ALGORITHMIC_BYTES_PER_LAUNCH = 149.1e6  # fp32 Q (read in the kernel's prologue), fp16 K, V^T, fp32 O
 ATTN_TRAFFIC_SOURCE = "profiles/attn_flash_joint_3952x4208_b2.md"
 

@@ -338,16 +338,19 @@ __device__ __forceinline__ void finish(const TGemmArgs& p, const float16_t (&acc
 // which puts two waves on every SIMD where the grid leaves one tile per CU. STAGES LDS stages.
 //
 // What bounds it: the matrix cores, at the clock the chip's power allows (1.5-1.75 GHz with all CUs
-// multiplying). The k loop of the 192x384 tile keeps them 78 % busy (2940 clocks per k-tile of 2304),
-// that of the 64x128 tile 68 %; the rest of a launch is its prologue (2 us) and its stores. Three
-// things hold the loop there:
+// multiplying), and what a wave issues beside its products. Of a whole launch's active cycles they are
+// busy 43 % with the 192x384 tile (3952 x 4608 x 1536), 48 % with the GLU's 128x512 (3952 x 8192 x 1536),
+// 41 % with 256x256 (2432 x 6144 x 1536), 35 and 32 % with 128x192 in one and two k groups and 30 % with
+// 64x128 (SQ_VALU_MFMA_BUSY_CYCLES against GRBM_GUI_ACTIVE); the prologue (2 us) and the stores, when they
+// idle, are in those cycles. Three things keep the k loop's products together:
 //  * fragments are read one k16 step ahead, across the k-tile's barrier too: the barrier comes
 //    before the last step of a tile (whose fragments are in registers by then), so no wave waits
 //    for LDS behind it;
 //  * the weight fragment of the next column is decoded behind the current column's products;
 //  * the copies of a k-tile go out in SPREAD steps between products, since a wave that issues them
 //    all at once issues no products meanwhile (64 bytes per clock and CU).
-// Three stages or a raised wave priority around the products measured no faster.
+// A raised wave priority around the products measured no faster; a third stage pays where a tile has
+// its CU to itself.
 // EPI 0: C = act(A W^T * alpha * scale + bias) (RM 0) or C += (gate *) that (RM 1), the order of
 // gemm.js:159-164. EPI 1 (GLU): W's rows are interleaved in 32-row blocks
 // (ns2_tile_i8_weight_glu), so 64 columns of a wave hold 32 columns of each GLU half; the
